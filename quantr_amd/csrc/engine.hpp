@@ -114,6 +114,12 @@ void pauli_tables(const std::vector<PauliMasks>& terms, std::vector<PauliGroup>&
 // groups too wide for a tile form a last, direct pass. Writes each group's X mask in its
 // pass's tile coordinates to lxm[] and returns the number of passes (at most G + 1).
 int pauli_passes(uint32_t n, int prec, PauliGroup* groups, int G, PauliPass* passes, uint32_t* lxm);
+// The device records of those passes, in the order of their use: 16 bytes per group and 24 per
+// term, each with one more behind them (which the kernel fetches ahead and does not use), one
+// entry per pass, and how many terms of X mask 0 have each of the 16 patterns. Allocates nothing.
+void pauli_tile_tables(int prec, const PauliGroup* groups, const uint32_t* lxm, const PauliPass* passes, int np,
+                       const PauliZTerm* flat, void* group_records, void* term_records, PauliTilePass* out,
+                       uint32_t* diag_count);
 
 // Validates and lowers a program. Throws Error.
 void validate_program(uint32_t n, const qr_program* p);

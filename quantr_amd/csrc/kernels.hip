@@ -701,139 +701,310 @@ __global__ __launch_bounds__(256) void k_pauli_expect(const typename CT<R>::T* _
   if (threadIdx.x == 0) part[blockIdx.x] = accumulate ? part[blockIdx.x] + red[0] : red[0];
 }
 
-// f[r] += (-1)^{popcount(r & hz)} a for the positions r of a chunk: one case per pattern hz,
-// so the signs are compile-time constants (adds and subtracts, no selects).
-template <int CH, int HZ>
-__device__ __forceinline__ void add_signed_fixed(double (&f)[CH], double a) {
+// The pairs (r, r ^ M) of a thread's 16 amplitudes, r running over the 8 registers whose bit B
+// (the top bit of M) is 0: conj(a_r) a_{r^M}, real and imaginary parts.
+template <int B>
+__device__ __forceinline__ constexpr int pair_rep(int i) {
+  return ((i >> B) << (B + 1)) | (i & ((1 << B) - 1));
+}
+// The values as the compiler must take them here: nothing computed from them moves above.
+template <typename T, int N>
+__device__ __forceinline__ void pin(T (&a)[N]) {
 #pragma unroll
-  for (int r = 0; r < CH; ++r) {
-    if (__builtin_popcount((unsigned)(r & HZ)) & 1) f[r] -= a;
-    else f[r] += a;
+  for (int r = 0; r < N; ++r) asm volatile("" : "+v"(a[r].x), "+v"(a[r].y));
+}
+// Re (or Im) of conj(x) y in binary64.
+template <typename T>
+__device__ __forceinline__ double pair_part(const T& x, const T& y, bool im) {
+  return im ? fma((double)x.x, (double)y.y, -(double)x.y * (double)y.x)
+            : fma((double)x.x, (double)y.x, (double)x.y * (double)y.y);
+}
+// sum over the pairs (r, r ^ M) of Re conj(a_r) a_{r^M}
+template <typename T, int M>
+__device__ __forceinline__ double pairs_sum(const T (&a)[16]) {
+  constexpr int B = M >= 8 ? 3 : (M >= 4 ? 2 : (M >= 2 ? 1 : 0));
+  double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const T x = a[pair_rep<B>(i)], y = a[pair_rep<B>(i) ^ M];
+    s0 = fma((double)x.x, (double)y.x, s0);
+    s1 = fma((double)x.y, (double)y.y, s1);
+  }
+  return s0 + s1;
+}
+template <typename T, int M>
+__device__ __forceinline__ void reg_pairs(const T (&a)[16], bool re, bool im, double (&qr)[8], double (&qi)[8]) {
+  constexpr int B = M >= 8 ? 3 : (M >= 4 ? 2 : (M >= 2 ? 1 : 0));
+  if (re) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qr[i] = pair_part(a[pair_rep<B>(i)], a[pair_rep<B>(i) ^ M], false);
+  }
+  if (im) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qi[i] = pair_part(a[pair_rep<B>(i)], a[pair_rep<B>(i) ^ M], true);
+  }
+}
+// The same with the partners y (read from LDS) in the order of the representatives.
+template <typename T, int B>
+__device__ __forceinline__ void lds_pairs(const T (&a)[16], const T (&y)[8], bool re, bool im, double (&qr)[8],
+                                          double (&qi)[8]) {
+  if (re) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qr[i] = pair_part(a[pair_rep<B>(i)], y[i], false);
+  }
+  if (im) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qi[i] = pair_part(a[pair_rep<B>(i)], y[i], true);
   }
 }
 
-template <int CH>
-__device__ __forceinline__ void add_signed(double (&f)[CH], double a, uint32_t hz) {
-  static_assert(CH == 16, "chunks of 16 positions");
-  switch (hz) {
-    case 0: add_signed_fixed<CH, 0>(f, a); break;
-    case 1: add_signed_fixed<CH, 1>(f, a); break;
-    case 2: add_signed_fixed<CH, 2>(f, a); break;
-    case 3: add_signed_fixed<CH, 3>(f, a); break;
-    case 4: add_signed_fixed<CH, 4>(f, a); break;
-    case 5: add_signed_fixed<CH, 5>(f, a); break;
-    case 6: add_signed_fixed<CH, 6>(f, a); break;
-    case 7: add_signed_fixed<CH, 7>(f, a); break;
-    case 8: add_signed_fixed<CH, 8>(f, a); break;
-    case 9: add_signed_fixed<CH, 9>(f, a); break;
-    case 10: add_signed_fixed<CH, 10>(f, a); break;
-    case 11: add_signed_fixed<CH, 11>(f, a); break;
-    case 12: add_signed_fixed<CH, 12>(f, a); break;
-    case 13: add_signed_fixed<CH, 13>(f, a); break;
-    case 14: add_signed_fixed<CH, 14>(f, a); break;
-    default: add_signed_fixed<CH, 15>(f, a); break;
-  }
-}
-
-// The same partial sums for groups whose X masks all lie in one tile: tile bits = the set
-// bits of tmask (K of them, the lowest first). Each workgroup walks tiles blockIdx.x,
-// +gridDim.x, ...: it loads the tile into LDS once and takes every partner amplitude
-// psi[o ^ xm] from there (lxm[g] = xm of group g in tile coordinates), so the whole pass reads
-// the state once however many groups it holds.
-template <typename R, int K>
-__global__ __launch_bounds__(256) void k_pauli_expect_tiles(const typename CT<R>::T* __restrict__ psi,
-                                                            uint64_t ntiles, uint64_t tmask, uint64_t nontile,
-                                                            const PauliGroup* __restrict__ groups,
-                                                            const uint32_t* __restrict__ lxm, int ngroups,
-                                                            const PauliZTerm* __restrict__ terms,
-                                                            double* __restrict__ part, int accumulate) {
-  using T = typename CT<R>::T;
-  constexpr int NPT = (1 << K) / 256;  // amplitudes per thread
-  __shared__ T lds[1 << K];
-  __shared__ double red[256];
-  const uint32_t tid = threadIdx.x;
-  // global offset of tile position p = tid + 256 r: the thread's part (tile bits 0..7) and the
-  // register part (tile bits 8..K-1)
-  uint64_t toff = 0, hib[K - 8];
-  {
-    uint64_t m = tmask;
-    for (int b = 0; b < K; ++b) {
-      const uint64_t low = m & (0ull - m);
-      m ^= low;
-      if (b < 8) {
-        if ((tid >> b) & 1u) toff |= low;
-      } else {
-        hib[b - 8] = low;
+// In-place Walsh-Hadamard transform: w[p] becomes sum_i (-1)^{popcount(i & p)} w[i], the sum of
+// the values under every sign pattern p at once.
+template <int N>
+__device__ __forceinline__ void walsh(double (&w)[N]) {
+#pragma unroll
+  for (int h = 1; h < N; h *= 2)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (!(i & h)) {
+        const double x = w[i], y = w[i | h];
+        w[i] = x + y;
+        w[i | h] = x - y;
       }
-    }
+}
+__device__ __forceinline__ double at_pattern(const double (&w)[8], uint32_t p) {
+  double v;
+  switch (p) {
+    case 0: v = w[0]; break;
+    case 1: v = w[1]; break;
+    case 2: v = w[2]; break;
+    case 3: v = w[3]; break;
+    case 4: v = w[4]; break;
+    case 5: v = w[5]; break;
+    case 6: v = w[6]; break;
+    default: v = w[7]; break;
   }
+  return v;
+}
+
+// A term's coefficient with its sign (-1)^{parity}: the parity of the tile's bits is uniform, the
+// thread's comes from its tile position pt.
+__device__ __forceinline__ double signed_coeff(const PauliTileTerm& t, uint64_t base, uint32_t pt) {
+  uint32_t hi = (uint32_t)__double2hiint(t.c);
+  hi ^= (uint32_t)__popcll(base & t.zout) << 31;
+  hi ^= (uint32_t)__popc(pt & t.lz) << 31;
+  return __hiloint2double((int)hi, __double2loint(t.c));
+}
+
+// sum of c (-1)^{parity} w[pattern] over `count` terms, of which t is the first and tp points at
+// the one behind it; on return both have moved past them (each term is fetched while the one
+// before is added).
+__device__ __forceinline__ double signed_terms(const double (&w)[8], const PauliTileTerm* __restrict__& tp,
+                                               uint32_t count, PauliTileTerm& t, uint64_t base, uint32_t pt) {
   double acc = 0.0;
-  for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const uint64_t base = deposit_bits(t, nontile) | toff;
-#pragma unroll
-    for (int r = 0; r < NPT; ++r) {
-      uint64_t off = 0;
-#pragma unroll
-      for (int q = 0; q < K - 8; ++q)
-        if ((r >> q) & 1) off |= hib[q];
-      const T* src = &psi[base | off];
-      T v;
-      v.x = src->x;
-      v.y = src->y;
-      lds[tid + 256 * r] = v;
-    }
-    __syncthreads();
-    // per group: the coefficient of every position (terms outer, the thread's positions inner),
-    // then the partner amplitudes from LDS. The sign (-1)^{popcount(j & zm)}, j = o ^ xm, splits
-    // into the thread's part (base ^ xm) and the register part of o: r's bits on the tile bits
-    // 8.. that zm holds (hz), a constant per position.
-    constexpr int CH = 16;  // positions per chunk (register budget)
-#pragma unroll 1
-    for (int c0 = 0; c0 < NPT; c0 += CH) {
-      double yr[CH], yi[CH];
-#pragma unroll
-      for (int r = 0; r < CH; ++r) yr[r] = yi[r] = 0.0;
-      for (int g = 0; g < ngroups; ++g) {
-        const uint64_t bx = base ^ groups[g].xm;
-        const uint32_t lx = lxm[g];
-        const uint32_t t0 = groups[g].first, t1 = t0 + groups[g].count;
-        double fr[CH], fi[CH];
-#pragma unroll
-        for (int r = 0; r < CH; ++r) fr[r] = fi[r] = 0.0;
-        for (uint32_t q = t0; q < t1; ++q) {
-          const uint64_t zm = terms[q].zm;
-          const double cr = terms[q].cr, ci = terms[q].ci;
-          uint32_t hz = 0;
-#pragma unroll
-          for (int b = 0; b < K - 8; ++b)
-            if (zm & hib[b]) hz |= 1u << b;
-          // the thread's signed coefficient (its part of the sign, and the chunk's), then each
-          // position adds or subtracts it by the parity of its register bits in hz
-          const uint32_t bt = ((uint32_t)__popcll(bx & zm) ^ (uint32_t)__popc((uint32_t)c0 & hz)) & 1u;
-          const double ar = bt ? -cr : cr;
-          add_signed<CH>(fr, ar, hz & (CH - 1));
-          if (ci != 0.0) add_signed<CH>(fi, bt ? -ci : ci, hz & (CH - 1));
-        }
-#pragma unroll
-        for (int r = 0; r < CH; ++r) {
-          const T w = lds[(tid + 256u * (uint32_t)(c0 + r)) ^ lx];
-          const double pr = (double)w.x, pi = (double)w.y;
-          yr[r] += fr[r] * pr - fi[r] * pi;
-          yi[r] += fr[r] * pi + fi[r] * pr;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < CH; ++r) {
-        const T v = lds[tid + 256u * (uint32_t)(c0 + r)];
-        acc += (double)v.x * yr[r] + (double)v.y * yi[r];
-      }
-    }
-    __syncthreads();  // the next tile overwrites lds
+  for (; count; --count) {
+    const PauliTileTerm next = *tp++;
+    acc = fma(signed_coeff(t, base, pt), at_pattern(w, t.pat), acc);
+    t = next;
   }
+  return acc;
+}
+
+// The groups of an arrangement that are one real term without a sign on the register bits, their
+// X masks the patterns set in `plain`: straight-line code (a dispatch on the pattern for each
+// group spent more scalar instructions than the group's own arithmetic).
+template <typename T, int M>
+__device__ __forceinline__ void plain_groups(const T (&a)[16], uint32_t plain, const PauliTileTerm* __restrict__& tp,
+                                             PauliTileTerm& t, uint64_t base, uint32_t pt, double& acc) {
+  if ((plain >> M) & 1u) {
+    const PauliTileTerm next = *tp++;
+    acc = fma(signed_coeff(t, base, pt), pairs_sum<T, M>(a), acc);
+    t = next;
+  }
+  if constexpr (M < 15) plain_groups<T, M + 1>(a, plain, tp, t, base, pt, acc);
+}
+
+// Partial sums of Re <psi|O|psi> for groups whose X masks lie in tiles of 2^K amplitudes (tile
+// bits = the set bits of a pass's tmask, the lowest first), all passes in one launch. Workgroups
+// of 2^(K-4) threads walk the tiles; a thread holds 16 amplitudes, which differ in 4 tile bits.
+// What bounds it: HBM when a pass holds few groups, else vector issue, then LDS (a 16-byte read
+// per amplitude costs a quarter of the CU's 128 B/clk for 8 clocks). So:
+//  * the tile is held in up to three arrangements, each with another 4 of the tile bits in
+//    registers: a group whose X mask lies in one of them pairs registers, with no LDS access;
+//    only masks that cross them read partners from LDS;
+//  * a hermitian term gives the same for (o, o ^ xm) and (o ^ xm, o): one product for each pair;
+//  * signs: a Walsh-Hadamard transform of the 8 pair products (16 probabilities for X mask 0)
+//    holds the sum under every pattern of register bits, so a term takes one multiply-add for
+//    all of a thread's amplitudes instead of one add for each.
+// What it measured against one LDS read and a signed add per amplitude, group and term: the Ising
+// observable of 29 qubits, complex128 (57 terms, 29 X masks, 3 passes), 13.5 -> 5.6 ms, 1.9 ms a
+// pass = 4.6 TB/s; complex64, 28 qubits, 6.5 -> 1.7 ms; 120 strings of up to 4 factors on 22
+// qubits 506 -> 367 us. Fetching the next tile ahead took longer (5.9 ms: its registers spill).
+// Element p of the tile sits at LDS slot p ^ (bits above the lowest arrangement's nibble, at its
+// place): consecutive lanes hit distinct slots in all three arrangements.
+template <typename R, int K, bool NT, bool GENERAL>
+__global__ __launch_bounds__(1 << (K - 4), K == 12 ? 2 : 4) void k_pauli_expect_tiles(
+    const typename CT<R>::T* __restrict__ psi, uint64_t dim, PauliTilePasses P,
+    const PauliTileGroup* __restrict__ groups, const PauliTileTerm* __restrict__ terms, double* __restrict__ part,
+    int accumulate) {
+  using T = typename CT<R>::T;
+  constexpr int TB = K - 4, LN = K - 12;  // thread bits; the lowest arrangement's first bit
+  __shared__ T lds[1 << K];
+  const uint32_t tid = threadIdx.x;
+  const uint32_t ntiles = (uint32_t)(dim >> K);  // 2^28 at most
+  auto slot = [](uint32_t p) { return p ^ (((p >> (LN + 4)) & 15u) << LN); };
+  double acc = 0.0;
+  uint32_t t = blockIdx.x;  // this workgroup's next (pass, tile), counted through all passes
+  for (uint32_t ip = 0; ip < P.count; ++ip) {
+    const PauliTilePass& ps = P.p[ip];
+    const uint64_t tmask = ps.tmask, nontile = (dim - 1) & ~tmask;
+    uint64_t toff = 0, hib[4];
+    {
+      uint64_t m = tmask;
+#pragma unroll
+      for (int b = 0; b < K; ++b) {
+        const uint64_t low = m & (0ull - m);
+        m ^= low;
+        if (b < TB) {
+          if ((tid >> b) & 1u) toff |= low;
+        } else {
+          hib[b - TB] = low;
+        }
+      }
+    }
+    // tile t's base has t's bits on the bits outside the tile; a step adds the deposited stride
+    // with the tile's bits set, so that carries run through them
+    const uint64_t step = deposit_bits(gridDim.x, nontile);
+    uint64_t base = deposit_bits(t, nontile);
+    for (; t < ntiles; t += gridDim.x, base = ((base | tmask) + step) & nontile) {
+      uint32_t lane = tid;  // opaque: LDS addresses are recomputed for each tile, not kept
+      asm volatile("" : "+v"(lane));
+      T a[16];
+      {
+        const T* src = psi + (base | toff);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          uint64_t off = 0;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if ((r >> q) & 1) off |= hib[q];
+          if (NT) {
+            load_nt(a[r], src + off);
+          } else {
+            a[r].x = src[off].x;
+            a[r].y = src[off].y;
+          }
+        }
+      }
+      // records and terms in the order of their use, each fetched one ahead
+      const PauliTileGroup* __restrict__ gp = groups + ps.first;
+      const PauliTileTerm* __restrict__ tp = terms + ps.term0;
+      PauliTileGroup gr = *gp++;
+      PauliTileTerm tm = *tp++;
+      if (ps.lds) {
+        __syncthreads();  // the previous tile's reads are over
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          T& d = lds[slot(lane | ((uint32_t)r << TB))];
+          d.x = a[r].x;
+          d.y = a[r].y;
+        }
+        __syncthreads();
+      }
+#pragma unroll 1
+      for (int arr = 0; arr < kPauliArrangements; ++arr) {
+        if (!((ps.arrs >> arr) & 1u)) continue;
+        const uint32_t nb = (uint32_t)pauli_arrangement_bit(K, arr);  // the register bits' place in the tile
+        const uint32_t pt = (lane & ((1u << nb) - 1u)) | ((lane >> nb) << (nb + 4));
+        if (arr > 0) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const T& d = lds[slot(pt | ((uint32_t)r << nb))];
+            a[r].x = d.x;
+            a[r].y = d.y;
+          }
+        }
+        if (arr == 0 && ps.diag) {  // X mask 0: terms sorted by pattern
+          double w[16];
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            w[r] = fma((double)a[r].x, (double)a[r].x, (double)a[r].y * (double)a[r].y);
+          walsh<16>(w);
+#pragma unroll
+          for (int p = 0; p < 16; ++p) {
+            uint32_t count = P.diag_count[p];
+            if (count == 0) continue;
+            double f = 0.0;
+            for (; count; --count) {
+              const PauliTileTerm tn = *tp++;
+              f += signed_coeff(tm, base, pt);
+              tm = tn;
+            }
+            acc = fma(f, w[p], acc);
+          }
+        }
+        if (ps.plain[arr]) plain_groups<T, 1>(a, ps.plain[arr], tp, tm, base, pt, acc);
+#pragma unroll 1
+        for (uint32_t left = GENERAL ? ps.cnt[arr] : 0; left; --left) {
+          const PauliTileGroup next = *gp++;
+          const uint32_t op = gr.op, nre = gr.nre, nim = gr.nim, lx = gr.lx;
+          gr = next;
+          // products of the loop-invariant amplitudes must not move out of the group loop: the
+          // compiler would keep every mask's pairs in registers at once, and spill them
+          pin(a);
+          const bool re = nre != 0, im = nim != 0;
+          double qr[8] = {}, qi[8] = {};
+          T y[8];
+          if (op >= PAULI_LDS) {
+            const uint32_t b = op & 3u;  // the register bit that tells a pair's two ends apart
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+              const uint32_t r = ((i >> b) << (b + 1)) | (i & ((1u << b) - 1u));
+              const T& d = lds[slot((pt | (r << nb)) ^ lx)];
+              y[i].x = d.x;
+              y[i].y = d.y;
+            }
+          }
+          switch (op) {
+            case 1: reg_pairs<T, 1>(a, re, im, qr, qi); break;
+            case 2: reg_pairs<T, 2>(a, re, im, qr, qi); break;
+            case 3: reg_pairs<T, 3>(a, re, im, qr, qi); break;
+            case 4: reg_pairs<T, 4>(a, re, im, qr, qi); break;
+            case 5: reg_pairs<T, 5>(a, re, im, qr, qi); break;
+            case 6: reg_pairs<T, 6>(a, re, im, qr, qi); break;
+            case 7: reg_pairs<T, 7>(a, re, im, qr, qi); break;
+            case 8: reg_pairs<T, 8>(a, re, im, qr, qi); break;
+            case 9: reg_pairs<T, 9>(a, re, im, qr, qi); break;
+            case 10: reg_pairs<T, 10>(a, re, im, qr, qi); break;
+            case 11: reg_pairs<T, 11>(a, re, im, qr, qi); break;
+            case 12: reg_pairs<T, 12>(a, re, im, qr, qi); break;
+            case 13: reg_pairs<T, 13>(a, re, im, qr, qi); break;
+            case 14: reg_pairs<T, 14>(a, re, im, qr, qi); break;
+            case 15: reg_pairs<T, 15>(a, re, im, qr, qi); break;
+            case PAULI_LDS + 0: lds_pairs<T, 0>(a, y, re, im, qr, qi); break;
+            case PAULI_LDS + 1: lds_pairs<T, 1>(a, y, re, im, qr, qi); break;
+            case PAULI_LDS + 2: lds_pairs<T, 2>(a, y, re, im, qr, qi); break;
+            default: lds_pairs<T, 3>(a, y, re, im, qr, qi); break;
+          }
+          if (re) {
+            walsh<8>(qr);
+            acc += signed_terms(qr, tp, nre, tm, base, pt);
+          }
+          if (im) {
+            walsh<8>(qi);
+            acc += signed_terms(qi, tp, nim, tm, base, pt);
+          }
+        }
+      }
+    }
+    t -= ntiles;
+  }
+  __syncthreads();
+  double* red = reinterpret_cast<double*>(lds);
   red[tid] = acc;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)tid < w) red[tid] += red[tid + w];
+  for (uint32_t w = 1u << (TB - 1); w > 0; w >>= 1) {
+    if (tid < w) red[tid] += red[tid + w];
     __syncthreads();
   }
   if (tid == 0) part[blockIdx.x] = accumulate ? part[blockIdx.x] + red[0] : red[0];
@@ -1141,31 +1312,50 @@ hipError_t launch_sample_fold_instances(int prec, const void* psi, uint64_t dim,
 
 int pauli_expect_partials(uint64_t dim) { return (int)std::min<uint64_t>(1024, std::max<uint64_t>(1, dim / 256)); }
 
-hipError_t launch_pauli_expect_passes(int prec, const void* psi, uint64_t dim, const PauliGroup* groups,
-                                      const uint32_t* lxm, const PauliZTerm* terms, const PauliPass* passes,
-                                      int npasses, double* part, hipStream_t s) {
-  const int nb = pauli_expect_partials(dim);
-  for (int i = 0; i < npasses; ++i) {
-    const PauliPass& ps = passes[i];
-    const int acc = i > 0 ? 1 : 0;
-    if (ps.tmask == 0) {
-      const hipError_t e = launch_pauli_expect(prec, psi, dim, groups + ps.first, (int)ps.count, terms, part, nb, s, acc);
+hipError_t launch_pauli_expect_passes(int prec, const void* psi, uint64_t dim, const void* groups, const void* terms,
+                                      const PauliTilePass* passes, int npasses, const uint32_t* diag_count,
+                                      double* part, hipStream_t s) {
+  const int nb = pauli_expect_partials(dim), K = pauli_tile_bits(prec), nt = streamed(prec, dim);
+  int acc = 0;
+  for (int i = 0; i < npasses;) {
+    if (passes[i].tmask == 0) {
+      const PauliTilePass& ps = passes[i++];
+      const hipError_t e = launch_pauli_expect(prec, psi, dim, (const PauliGroup*)groups + ps.first, (int)ps.cnt[0],
+                                               (const PauliZTerm*)terms, part, nb, s, acc);
       if (e != hipSuccess) return e;
+      acc = 1;
       continue;
     }
-    const int K = __builtin_popcountll(ps.tmask);
-    if (K != pauli_tile_bits(prec) || (dim >> K) == 0) return hipErrorInvalidValue;
-    const uint64_t ntiles = dim >> K, nontile = (dim - 1) & ~ps.tmask;
-    if (prec == 0)
-      dev::k_pauli_expect_tiles<double, 12><<<nb, 256, 0, s>>>((const double2*)psi, ntiles, ps.tmask, nontile,
-                                                              groups + ps.first, lxm + ps.first, (int)ps.count,
-                                                              terms, part, acc);
-    else
-      dev::k_pauli_expect_tiles<float, 13><<<nb, 256, 0, s>>>((const float2*)psi, ntiles, ps.tmask, nontile,
-                                                             groups + ps.first, lxm + ps.first, (int)ps.count,
-                                                             terms, part, acc);
+    PauliTilePasses P{};
+    for (int p = 0; p < 16; ++p) P.diag_count[p] = diag_count[p];
+    for (; i < npasses && passes[i].tmask != 0 && P.count < kPauliPassesPerLaunch; ++i) {
+      if (__builtin_popcountll(passes[i].tmask) != K || (dim >> K) == 0) return hipErrorInvalidValue;
+      P.p[P.count++] = passes[i];
+    }
+    const PauliTileGroup* tg = (const PauliTileGroup*)groups;
+    const PauliTileTerm* tt = (const PauliTileTerm*)terms;
+    // observables without general groups (Ising and the like) run a variant without their code,
+    // whose registers cost the others their occupancy
+    bool general = false;
+    for (uint32_t p = 0; p < P.count; ++p)
+      for (int a = 0; a < kPauliArrangements; ++a) general = general || P.p[p].cnt[a] != 0;
+    auto run = [&](auto kernel, auto* amp, unsigned threads) { kernel<<<nb, threads, 0, s>>>(amp, dim, P, tg, tt, part, acc); };
+    if (prec == 0) {
+      const double2* amp = (const double2*)psi;
+      if (nt) general ? run(dev::k_pauli_expect_tiles<double, 12, true, true>, amp, 256)
+                      : run(dev::k_pauli_expect_tiles<double, 12, true, false>, amp, 256);
+      else general ? run(dev::k_pauli_expect_tiles<double, 12, false, true>, amp, 256)
+                   : run(dev::k_pauli_expect_tiles<double, 12, false, false>, amp, 256);
+    } else {
+      const float2* amp = (const float2*)psi;
+      if (nt) general ? run(dev::k_pauli_expect_tiles<float, 13, true, true>, amp, 512)
+                      : run(dev::k_pauli_expect_tiles<float, 13, true, false>, amp, 512);
+      else general ? run(dev::k_pauli_expect_tiles<float, 13, false, true>, amp, 512)
+                   : run(dev::k_pauli_expect_tiles<float, 13, false, false>, amp, 512);
+    }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    acc = 1;
   }
   return hipSuccess;
 }

@@ -147,16 +147,53 @@ struct PauliPass {
   uint32_t first, count;
 };
 // Tile width of the grouped expectation passes: 2^12 complex128 / 2^13 complex64 amplitudes
-// (64 KB of LDS), of which the lowest 3 / 4 bits (128-byte segments) are always tile bits.
+// (64 KB of LDS, two workgroups per CU), of which the lowest 3 / 4 bits (128-byte segments) are always tile bits.
 inline int pauli_tile_bits(int prec) { return prec == 0 ? 12 : 13; }
 inline int pauli_low_bits(int prec) { return prec == 0 ? 3 : 4; }
+// Device records of the tiled passes (pauli_tile_tables). A pass holds each tile in up to four
+// arrangements; arrangement a keeps the tile bits pauli_arrangement_bit(K, a) + 0..3 in a thread's
+// 16 registers (the last one only serves the lowest bits of 2^13 tiles).
+constexpr int kPauliArrangements = 4;
+__host__ __device__ constexpr int pauli_arrangement_bit(int K, int a) { return K - 4 - 4 * a > 0 ? K - 4 - 4 * a : 0; }
+// Group ops. 1..15: the X mask is this pattern of the register bits; PAULI_LDS + b: partners read
+// from LDS, b = the highest of its register bits.
+enum PauliOp : uint32_t { PAULI_DIAG = 0, PAULI_LDS = 16 };
+// nre terms with an even number of Y factors, then nim with an odd one; lx = X mask in the tile
+// (whole words: the record is read with scalar loads).
+struct PauliTileGroup {
+  uint32_t op, lx, nre, nim;
+};
+// One term: its Z mask outside the tile, on the thread's tile bits (lz), and on the register bits
+// as a sign pattern (pat); c = its real coefficient, doubled where each pair is taken once.
+struct PauliTileTerm {
+  uint64_t zout;
+  double c;
+  uint32_t lz, pat;
+};
+static_assert(sizeof(PauliTileGroup) == sizeof(PauliGroup) && sizeof(PauliTileTerm) == sizeof(PauliZTerm),
+              "tiled and direct passes share one table");
+// One pass over the state, its groups by arrangement: with `diag`, X mask 0 (in arrangement 0);
+// the register patterns plain[a] whose group is one real term of pattern 0; then cnt[a] other
+// groups, whose records lie from `first` on. Terms lie in this order from `term0` on. arrs: the
+// arrangements in use; lds: the tile goes through LDS. A direct pass has tmask 0 and cnt[0] groups.
+struct PauliTilePass {
+  uint64_t tmask;
+  uint32_t first, term0, lds, diag, arrs;
+  uint32_t cnt[kPauliArrangements], plain[kPauliArrangements];
+};
+constexpr uint32_t kPauliPassesPerLaunch = 16;  // passes travel as a kernel argument
+struct PauliTilePasses {
+  uint32_t count;
+  uint32_t diag_count[16];  // X mask 0: its terms are sorted by pattern; how many each has
+  PauliTilePass p[kPauliPassesPerLaunch];
+};
 // Partial sums (workgroups) of every expectation pass over a state of dim amplitudes.
 int pauli_expect_partials(uint64_t dim);
-// part[0 .. pauli_expect_partials(dim)) = partial sums of Re <psi|O|psi>, pass after pass;
-// lxm[g] = group g's X mask in the tile coordinates of its pass.
-hipError_t launch_pauli_expect_passes(int prec, const void* psi, uint64_t dim, const PauliGroup* groups,
-                                      const uint32_t* lxm, const PauliZTerm* terms, const PauliPass* passes,
-                                      int npasses, double* part, hipStream_t s);
+// part[0 .. pauli_expect_partials(dim)) = partial sums of Re <psi|O|psi>, pass after pass, from
+// the records of pauli_tile_tables.
+hipError_t launch_pauli_expect_passes(int prec, const void* psi, uint64_t dim, const void* groups, const void* terms,
+                                      const PauliTilePass* passes, int npasses, const uint32_t* diag_count,
+                                      double* part, hipStream_t s);
 // part[b] = partial sums of Re sum_j conj(a_j) b_j over nblocks blocks.
 hipError_t launch_dot_re_partial(int prec, const void* a, const void* b, uint64_t dim, double* part, int nblocks,
                                  hipStream_t s);

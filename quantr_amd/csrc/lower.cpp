@@ -529,6 +529,121 @@ int pauli_passes(uint32_t n, int prec, PauliGroup* groups, int G, PauliPass* pas
   return np;
 }
 
+namespace {
+
+// The tile coordinates of a mask: its bits on the set bits of tmask, lowest first.
+uint32_t tile_mask(uint64_t m, uint64_t tmask) {
+  uint32_t out = 0;
+  for (int b = 0; tmask; ++b) {
+    const uint64_t low = tmask & (0ull - tmask);
+    tmask ^= low;
+    if (m & low) out |= 1u << b;
+  }
+  return out;
+}
+
+// Where a group of X mask lx (tile coordinates) is evaluated: with its mask inside one
+// arrangement's register bits if it fits, else from LDS in the first arrangement that holds one
+// of its bits. Returns the arrangement; `op` as in PauliOp.
+int pauli_place(int K, uint32_t lx, uint32_t& op) {
+  op = PAULI_DIAG;
+  if (lx == 0) return 0;
+  for (int a = 0; a < kPauliArrangements; ++a) {
+    const int nb = pauli_arrangement_bit(K, a);
+    if ((lx & ~(15u << nb)) == 0) {
+      op = lx >> nb;
+      return a;
+    }
+  }
+  int a = 0;
+  while (((lx >> pauli_arrangement_bit(K, a)) & 15u) == 0) ++a;
+  op = PAULI_LDS + (31 - __builtin_clz((lx >> pauli_arrangement_bit(K, a)) & 15u));
+  return a;
+}
+
+}  // namespace
+
+void pauli_tile_tables(int prec, const PauliGroup* groups, const uint32_t* lxm, const PauliPass* passes, int np,
+                       const PauliZTerm* flat, void* group_records, void* term_records, PauliTilePass* out,
+                       uint32_t* diag_count) {
+  const int K = pauli_tile_bits(prec);
+  PauliTileGroup* tg = (PauliTileGroup*)group_records;
+  PauliTileTerm* tt = (PauliTileTerm*)term_records;
+  uint32_t nt = 0, ng = 0;  // terms and groups written
+  for (int p = 0; p < 16; ++p) diag_count[p] = 0;
+  for (int p = 0; p < np; ++p) {
+    const PauliPass& ps = passes[p];
+    PauliTilePass& o = out[p];
+    o = PauliTilePass{ps.tmask, ng, nt, 0, 0, 0, {0, 0, 0, 0}, {0, 0, 0, 0}};
+    const uint32_t end = ps.first + ps.count;
+    if (ps.tmask == 0) {  // read directly: the plain records
+      o.cnt[0] = ps.count;
+      for (uint32_t i = ps.first; i < end; ++i) {
+        const PauliGroup g{groups[i].xm, nt, groups[i].count};
+        std::memcpy(tg + ng++, &g, sizeof g);
+        std::memcpy(tt + nt, flat + groups[i].first, g.count * sizeof(PauliZTerm));
+        nt += g.count;
+      }
+      continue;
+    }
+    // writes group i's terms (real coefficients first) and returns its record
+    auto put = [&](uint32_t i, int a, uint32_t op) {
+      const PauliGroup& g = groups[i];
+      const int nb = pauli_arrangement_bit(K, a);
+      // the register bit that tells a pair's ends apart
+      const int top = op >= PAULI_LDS ? (int)(op - PAULI_LDS) : (op ? 31 - __builtin_clz(op) : 0);
+      PauliTileGroup r{op, lxm[i], 0, 0};
+      for (int odd = 0; odd < 2; ++odd)  // by the number of Y factors
+        for (uint32_t t = g.first; t < g.first + g.count; ++t) {
+          const PauliZTerm& z = flat[t];
+          if ((__builtin_popcountll(g.xm & z.zm) & 1) != odd) continue;
+          // Re(conj(psi_o) c s(o') psi_o') with o' = o ^ xm and s(o') = (-1)^{ny} s(o):
+          // cr s(o) Re(conj(psi_o) psi_o') for even ny, ci s(o) Im(...) for odd
+          double c = odd ? z.ci : z.cr;
+          if (op != PAULI_DIAG) c *= 2.0;
+          const uint32_t zt = tile_mask(z.zm, ps.tmask), nib = (zt >> nb) & 15u;
+          const uint32_t pat = op == PAULI_DIAG ? nib : (nib & ((1u << top) - 1u)) | ((nib >> (top + 1)) << top);
+          tt[nt++] = PauliTileTerm{z.zm & ~ps.tmask, c, zt & ~(15u << nb), pat};
+          ++(odd ? r.nim : r.nre);
+        }
+      return r;
+    };
+    for (int a = 0; a < kPauliArrangements; ++a) {
+      // X mask 0 and the plain groups, by pattern
+      for (uint32_t want = 0; want < PAULI_LDS; ++want)
+        for (uint32_t i = ps.first; i < end; ++i) {
+          uint32_t op;
+          if (pauli_place(K, lxm[i], op) != a || op != want) continue;
+          const uint32_t t0 = nt;
+          const PauliTileGroup r = put(i, a, op);
+          if (op == PAULI_DIAG) {
+            std::sort(tt + t0, tt + nt, [](const PauliTileTerm& x, const PauliTileTerm& y) {
+              return x.pat != y.pat ? x.pat < y.pat : (x.zout != y.zout ? x.zout < y.zout : x.lz < y.lz);
+            });
+            for (uint32_t t = t0; t < nt; ++t) diag_count[tt[t].pat]++;
+            o.diag = 1;
+          } else if (r.nre == 1 && r.nim == 0 && tt[t0].pat == 0) {
+            o.plain[a] |= 1u << op;
+          } else {
+            nt = t0;  // not plain: below
+          }
+        }
+      for (uint32_t i = ps.first; i < end; ++i) {
+        uint32_t op;
+        if (pauli_place(K, lxm[i], op) != a || op == PAULI_DIAG) continue;
+        if (op < PAULI_LDS && ((o.plain[a] >> op) & 1u)) continue;  // an X mask occurs once
+        tg[ng++] = put(i, a, op);
+        o.cnt[a]++;
+        if (op >= PAULI_LDS) o.lds = 1;
+      }
+      if (o.cnt[a] || o.plain[a] || (a == 0 && o.diag)) o.arrs |= 1u << a;
+    }
+    if (o.arrs > 1) o.lds = 1;
+  }
+  tg[ng] = PauliTileGroup{0, 0, 0, 0};
+  tt[nt] = PauliTileTerm{0, 0.0, 0, 0};
+}
+
 void pauli_tables(const std::vector<PauliMasks>& terms, std::vector<PauliGroup>& groups,
                   std::vector<PauliZTerm>& flat) {
   // terms grouped by X mask; Z masks and i^ny folded into per-term complex coefficients

@@ -2,8 +2,8 @@
 //
 // Callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
 // that forbid hipMalloc) get the expectation value through the same passes and kernels as
-// qr_expectation, with its device working set (the observable's X-mask groups, their tile
-// masks, its Z-mask terms and the per-workgroup partial sums) in a fixed device array instead
+// qr_expectation, with its device working set (the records of the observable's X-mask groups
+// and terms and the per-workgroup partial sums) in a fixed device array instead
 // of workspaces that grow by hipMalloc. Host staging lives in fixed static arrays as well.
 // Results are bitwise equal to qr_expectation's: same tables in the same order, same passes,
 // same kernels, same partial count and the same host summation.
@@ -32,10 +32,9 @@ constexpr uint64_t kMaxTerms = 16384;         // observable terms at most
 constexpr int kMaxParts = 1024;               // partial sums (one per workgroup)
 constexpr int kMaxDevices = 64;
 
-// groups (16 B), their tile masks (4 B) and terms (24 B) of at most kMaxTerms terms, then the
-// partials
-static_assert(kMaxTerms * (sizeof(PauliGroup) + sizeof(uint32_t) + sizeof(PauliZTerm)) + 8 +
-                      kMaxParts * sizeof(double) + 256 <=
+// group records (16 B) and term records (24 B) of at most kMaxTerms terms and one more of each,
+// then the partials
+static_assert((kMaxTerms + 1) * (sizeof(PauliGroup) + sizeof(PauliZTerm)) + kMaxParts * sizeof(double) + 256 <=
                   kScratchBytes,
               "scratch layout");
 
@@ -58,7 +57,10 @@ struct KeyIdx {
 };
 KeyIdx g_keys[kMaxTerms];
 PauliZTerm g_terms_in[kMaxTerms];
+PauliGroup g_groups[kMaxTerms];
+PauliZTerm g_flat[kMaxTerms];
 PauliPass g_passes[kMaxTerms + 1];
+PauliTilePass g_tile_passes[kMaxTerms + 1];
 uint32_t g_lxm[kMaxTerms];
 double g_parts[kMaxParts];
 
@@ -101,7 +103,7 @@ double expectation_noalloc(qr_state* st, const qr_observable* o) {
   }
   std::sort(g_keys, g_keys + T,
             [](const KeyIdx& a, const KeyIdx& b) { return a.xm != b.xm ? a.xm < b.xm : a.idx < b.idx; });
-  PauliGroup* groups = (PauliGroup*)g_stage;
+  PauliGroup* groups = g_groups;
   uint64_t G = 0;
   for (uint64_t t = 0; t < T; ++t)
     if (t == 0 || g_keys[t].xm != g_keys[t - 1].xm) groups[G++] = PauliGroup{g_keys[t].xm, (uint32_t)t, 0u};
@@ -111,18 +113,16 @@ double expectation_noalloc(qr_state* st, const qr_observable* o) {
   }
   // the same passes as qr_expectation (groups reordered in place)
   const int np = pauli_passes(st->n, st->prec, groups, (int)G, g_passes, g_lxm);
-  const size_t gb = (size_t)G * sizeof(PauliGroup), lb = ((size_t)G * 4 + 7) & ~(size_t)7;
-  std::memcpy(g_stage + gb, g_lxm, (size_t)G * 4);
-  PauliZTerm* flat = (PauliZTerm*)(g_stage + gb + lb);
-  for (uint64_t t = 0; t < T; ++t) flat[t] = g_terms_in[g_keys[t].idx];
-  const size_t tb = (size_t)T * sizeof(PauliZTerm);
-  const size_t part_off = (gb + lb + tb + 255) & ~(size_t)255;
+  for (uint64_t t = 0; t < T; ++t) g_flat[t] = g_terms_in[g_keys[t].idx];
+  const size_t gb = (size_t)(G + 1) * sizeof(PauliGroup), tb = (size_t)(T + 1) * sizeof(PauliZTerm);
+  uint32_t diag_count[16];
+  pauli_tile_tables(st->prec, groups, g_lxm, g_passes, np, g_flat, g_stage, g_stage + gb, g_tile_passes, diag_count);
+  const size_t part_off = (gb + tb + 255) & ~(size_t)255;
   const int nb = pauli_expect_partials(st->dim);
   static_assert(kMaxParts >= 1024, "pauli_expect_partials returns at most 1024");
-  hip_check(hipMemcpyAsync(dev, g_stage, gb + lb + tb, hipMemcpyHostToDevice, st->stream), "hipMemcpyAsync H2D");
-  hip_check(launch_pauli_expect_passes(st->prec, st->amp, st->dim, (const PauliGroup*)dev,
-                                       (const uint32_t*)(dev + gb), (const PauliZTerm*)(dev + gb + lb), g_passes,
-                                       np, (double*)(dev + part_off), st->stream),
+  hip_check(hipMemcpyAsync(dev, g_stage, gb + tb, hipMemcpyHostToDevice, st->stream), "hipMemcpyAsync H2D");
+  hip_check(launch_pauli_expect_passes(st->prec, st->amp, st->dim, dev, dev + gb, g_tile_passes, np,
+                                       diag_count, (double*)(dev + part_off), st->stream),
             "expectation");
   hip_check(hipMemcpyAsync(g_parts, dev + part_off, nb * sizeof(double), hipMemcpyDeviceToHost, st->stream), "D2H");
   hip_check(hipStreamSynchronize(st->stream), "sync");

@@ -621,19 +621,18 @@ double expectation(qr_state* st, const std::vector<PauliMasks>& terms) {
   std::vector<PauliPass> passes(G + 1);
   std::vector<uint32_t> lxm(G);
   const int np = pauli_passes(st->n, st->prec, groups.data(), G, passes.data(), lxm.data());
-  // device tables: groups, their tile masks (padded to 8 bytes), terms
-  const size_t gb = (size_t)G * sizeof(PauliGroup), lb = ((size_t)G * 4 + 7) & ~(size_t)7;
-  const size_t tb = flat.size() * sizeof(PauliZTerm);
-  std::vector<uint8_t> blob(gb + lb + tb, 0);
-  std::memcpy(blob.data(), groups.data(), gb);
-  std::memcpy(blob.data() + gb, lxm.data(), (size_t)G * 4);
-  if (tb) std::memcpy(blob.data() + gb + lb, flat.data(), tb);
+  // device tables: group records, then term records
+  const size_t gb = (size_t)(G + 1) * sizeof(PauliGroup), tb = (flat.size() + 1) * sizeof(PauliZTerm);
+  std::vector<uint8_t> blob(gb + tb, 0);
+  std::vector<PauliTilePass> tp(np);
+  uint32_t diag_count[16];
+  pauli_tile_tables(st->prec, groups.data(), lxm.data(), passes.data(), np, flat.data(), blob.data(), blob.data() + gb,
+                    tp.data(), diag_count);
   uint8_t* d = upload(st, st->aux, blob);
   const int nb = pauli_expect_partials(st->dim);
   st->aux2.reserve(nb * sizeof(double));
-  hip_check(launch_pauli_expect_passes(st->prec, st->amp, st->dim, (const PauliGroup*)d, (const uint32_t*)(d + gb),
-                                       (const PauliZTerm*)(d + gb + lb), passes.data(), np, (double*)st->aux2.p,
-                                       st->stream),
+  hip_check(launch_pauli_expect_passes(st->prec, st->amp, st->dim, d, d + gb, tp.data(), np, diag_count,
+                                       (double*)st->aux2.p, st->stream),
             "expectation");
   std::vector<double> h(nb);
   hip_check(hipMemcpyAsync(h.data(), st->aux2.p, nb * sizeof(double), hipMemcpyDeviceToHost, st->stream), "D2H");

@@ -764,3 +764,36 @@ def test_batch_autotuned_widths_match():
             assert np.max(np.abs(x - y)) < 1e-11
         b.close()
     b0.close()
+
+
+def _arrangement_observable(n, rng):
+    """X masks in each group of tile bits the expectation kernel pairs in registers (the tile's
+    lowest and highest wires and every nibble between), masks that cross them, both parities of
+    Y, several terms on one X mask, and Z strings inside and outside the tile."""
+    terms = [(0.5, [(w, "X")]) for w in range(n)] + [(-0.3, [(w, "Y")]) for w in range(n)]
+    terms += [(1.0, [(w, "Z"), ((w + 1) % n, "Z")]) for w in range(n)]
+    terms += [(0.7, [(w, "X"), (w + 1, "Y")]) for w in range(n - 1)]
+    for w in range(n - 3):
+        terms.append((0.2, [(w, "X"), (w + 1, "X"), (w + 2, "Y"), (w + 3, "Y")]))
+    for _ in range(40):
+        wires = rng.permutation(n)[:int(rng.integers(1, 7))]
+        terms.append((float(rng.normal()), [(int(w), "XYZ"[int(rng.integers(3))]) for w in wires]))
+    return _capi.Observable(terms)
+
+
+@pytest.mark.parametrize("precision,n", [(_capi.QR_C128, 15), (_capi.QR_C128, 16), (_capi.QR_C128, 21),
+                                         (_capi.QR_C64, 16), (_capi.QR_C64, 17), (_capi.QR_C64, 20)])
+def test_expectation_arrangements(precision, n):
+    """Every arrangement and dispatch of the tiled expectation kernel, from the smallest tiled
+    state on, against the oracle on the amplitudes the state holds. The kernel and the oracle sum
+    the same products in binary64 in other orders: at most 2^n terms of total weight 1 per
+    string, so n * 2^-52 each, with a factor 16 for the oracle's and the kernel's own steps."""
+    rng = np.random.default_rng(4100 + n)
+    st = _capi.State(n, precision)
+    st.apply(W.to_program(W.brickwork(n, depth=7, seed=n + 1)))
+    psi = st.amplitudes()
+    for obs in (_arrangement_observable(n, rng), _capi.Observable(W.hea_observable(n))):
+        got = st.expectation(obs)
+        want = H.oracle_expectation(n, psi, obs)
+        assert abs(got - want) < 16 * n * 2.0 ** -52 * sum(abs(c) for c, _ in obs.terms)
+    st.close()
