@@ -224,11 +224,9 @@ qr_status qr_sample(qr_state* st, const double* uniforms, uint64_t shots, uint64
     if (!uniforms || !idx_out) throw Error{QR_ERR_ARG, "NULL argument"};
     for (uint64_t s = 0; s < shots; ++s)
       if (std::isnan(uniforms[s])) throw Error{QR_ERR_ARG, "uniform draws must not be NaN"};
-    std::vector<uint64_t> perm(shots);
-    std::iota(perm.begin(), perm.end(), 0);
-    std::stable_sort(perm.begin(), perm.end(), [&](uint64_t a, uint64_t b) { return uniforms[a] < uniforms[b]; });
-    std::vector<double> us(shots);
-    for (uint64_t s = 0; s < shots; ++s) us[s] = uniforms[perm[s]];
+    std::vector<uint64_t> perm;
+    std::vector<double> us;
+    sort_draws(uniforms, shots, us, perm);
     std::vector<uint64_t> res(shots, ~0ull);
     if (st->opt.exact_sample == 1) {
       // checker mode: one lane folds the whole state in index order

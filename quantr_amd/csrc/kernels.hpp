@@ -105,6 +105,10 @@ hipError_t launch_block_mass(int prec, const void* psi, uint64_t dim, int bb, do
 // Exact sums of rint(p_i * 2^(52-e)) per block for e = ebase[b] + 0..2, and halfway flags.
 hipError_t launch_block_exact_sums(int prec, const void* psi, uint64_t dim, int bb, const int32_t* ebase,
                                    double* sums, uint32_t* flags, hipStream_t s);
+// out[y * 2^bb + q] = re^2 + im^2 (no fused operations) of amplitude q of block list[y] (block y if
+// list is null), y < count; out and list may be pinned host memory.
+hipError_t launch_gather_probs(int prec, const void* psi, int bb, const uint64_t* list, uint32_t count, double* out,
+                               hipStream_t s);
 // Resolves each job's draws with its block's exact fold values (bb >= 12).
 hipError_t launch_sample_exact_blocks(int prec, const void* psi, uint64_t dim, int bb, const ExactJob* jobs,
                                       uint64_t njobs, const double* u, uint64_t* out, hipStream_t s);

@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <fstream>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -22,6 +23,76 @@
 
 namespace qr {
 
+
+// ---- pinned host memory -------------------------------------------------------------------
+namespace {
+constexpr size_t kPinnedKeep = 8, kPinnedBytes = 64ull << 20;
+struct PinnedBlock {
+  void* p;
+  size_t cap;
+};
+std::mutex g_pin_mu;
+std::vector<PinnedBlock> g_pinned;  // kept blocks, none in use
+uint64_t g_pin_states = 0;
+
+void pinned_give_back(void* p, size_t cap) {
+  void* drop = p;
+  {
+    std::lock_guard<std::mutex> lk(g_pin_mu);
+    size_t held = cap;
+    for (const PinnedBlock& b : g_pinned) held += b.cap;
+    if (g_pin_states > 0 && g_pinned.size() < kPinnedKeep && held <= kPinnedBytes) {
+      g_pinned.push_back({p, cap});
+      drop = nullptr;
+    }
+  }
+  if (drop) (void)hipHostFree(drop);
+}
+}  // namespace
+
+void pinned_state_created() {
+  std::lock_guard<std::mutex> lk(g_pin_mu);
+  ++g_pin_states;
+}
+
+void pinned_state_destroyed() {
+  std::vector<PinnedBlock> drop;
+  {
+    std::lock_guard<std::mutex> lk(g_pin_mu);
+    if (--g_pin_states == 0) drop.swap(g_pinned);
+  }
+  for (const PinnedBlock& b : drop) (void)hipHostFree(b.p);
+}
+
+void PinnedLease::reserve(size_t bytes) {
+  if (bytes <= cap_) return;
+  if (p_) pinned_give_back(p_, cap_);
+  p_ = nullptr;
+  cap_ = 0;
+  {
+    std::lock_guard<std::mutex> lk(g_pin_mu);
+    size_t best = g_pinned.size();
+    for (size_t i = 0; i < g_pinned.size(); ++i)
+      if (g_pinned[i].cap >= bytes && (best == g_pinned.size() || g_pinned[i].cap < g_pinned[best].cap)) best = i;
+    if (best < g_pinned.size()) {
+      p_ = g_pinned[best].p;
+      cap_ = g_pinned[best].cap;
+      g_pinned.erase(g_pinned.begin() + best);
+      return;
+    }
+  }
+  size_t want = 1 << 16;
+  while (want < bytes) want *= 2;
+  hip_check(hipHostMalloc(&p_, want, hipHostMallocPortable | hipHostMallocCoherent), "hipHostMalloc");
+  cap_ = want;
+}
+
+PinnedLease::~PinnedLease() {
+  if (!p_) return;
+  // a call that ends in an error may leave work in flight on the block: hipHostFree waits for it
+  if (std::uncaught_exceptions()) (void)hipHostFree(p_);
+  else pinned_give_back(p_, cap_);
+}
 
 // Default tile shape: 2^12 complex128 / 2^13 complex64 amplitudes (64 KB of LDS, two
 // workgroups per CU), 16 amplitudes per thread.
@@ -573,6 +644,8 @@ qr_state* new_state(uint32_t n, qr_precision p) {
                                 "-qubit state: " + hipGetErrorString(e)};
   }
   hip_check(launch_init_basis(st->prec, st->amp, st->dim, 0, st->stream), "init kernel");
+  pinned_state_created();
+  st->counted = true;
   return st.release();
 }
 

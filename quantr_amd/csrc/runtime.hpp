@@ -41,6 +41,26 @@ struct DevBuf {
   }
 };
 
+// A block of pinned host memory, which kernels and copies reach directly, held for one call.
+// Blocks are kept for later calls (pinning a new one takes longer than a small call): at most
+// 8 of them and 64 MB, none once no state is left.
+class PinnedLease {
+ public:
+  PinnedLease() = default;
+  explicit PinnedLease(size_t bytes) { reserve(bytes); }
+  ~PinnedLease();
+  PinnedLease(const PinnedLease&) = delete;
+  PinnedLease& operator=(const PinnedLease&) = delete;
+  void reserve(size_t bytes);  // at least this size; what it held is lost
+  uint8_t* data() const { return (uint8_t*)p_; }
+
+ private:
+  void* p_ = nullptr;
+  size_t cap_ = 0;
+};
+void pinned_state_created();    // one more state lives
+void pinned_state_destroyed();  // one less; the last one frees the kept blocks
+
 struct ProfRec {
   std::string name;
   hipEvent_t a, b;
@@ -64,8 +84,10 @@ struct qr_state {
   qr_plan_stats last{};
   bool profiling = false;
   std::vector<qr::ProfRec> prof;
+  bool counted = false;  // among the states that keep pinned blocks alive
   size_t bytes_per_amp() const { return prec == 0 ? 16 : 8; }
   ~qr_state() {
+    if (counted) qr::pinned_state_destroyed();
     for (auto& r : prof) {
       (void)hipEventDestroy(r.a);
       (void)hipEventDestroy(r.b);
@@ -185,6 +207,8 @@ void do_apply(qr_state* st, const qr_program* prog);
 double sum_partials_host(const std::vector<double>& v);
 // Compensated (Neumaier) sum of count partials, in index order.
 double sum_partials_host(const double* v, size_t count);
+// us = the draws in ascending order (none is NaN), perm[s] = where us[s] was (sampler.cpp).
+void sort_draws(const double* u, uint64_t shots, std::vector<double>& us, std::vector<uint64_t>& perm);
 // measure_all's sampling (sampler.cpp): draws `us` in ascending order; res[s] = the first index
 // whose left-fold cumulative probability exceeds us[s], or UINT64_MAX (None).
 void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vector<uint64_t>& res);

@@ -120,3 +120,28 @@ def test_sampler_28q_boundaries():
     st.set_options(exact_sample=1)
     assert np.array_equal(st.sample(u), ref)
     st.close()
+
+
+@pytest.mark.parametrize("precision", [_capi.QR_C128, _capi.QR_C64])
+@pytest.mark.parametrize("n", [1, 11, 15, 16, 17])
+def test_draw_sorting_and_small_states(precision, n):
+    """States on both sides of the size that is folded on the host as a whole, near a basis state
+    (most draws fall into one block, more than one job takes) and spread out, with draws that the
+    counting sort clamps or finds crowded into one bucket: every bin equals the one-lane fold's."""
+    rng = np.random.default_rng(50 + n)
+    near = np.full(1 << n, 1e-3 / np.sqrt(1 << n), dtype=np.complex128)
+    near[(5 << n) >> 3] = 1.0
+    near /= np.linalg.norm(near)
+    spread = rng.standard_normal(1 << n) + 1j * rng.standard_normal(1 << n)
+    spread /= np.linalg.norm(spread)
+    draws = np.concatenate([rng.random(6000), 0.25 + 1e-9 * rng.random(300)[::-1], np.full(70, 0.5),
+                            [-1.0, -0.0, 0.0, 1.0 - 2.0 ** -53, 1.0, 7.5, np.inf, -np.inf]])
+    rng.shuffle(draws)
+    st = _capi.State(n, precision)
+    for amps in (near, spread):
+        st.set_amplitudes(amps)
+        st.set_options(exact_sample=2)
+        got = st.sample(draws)
+        st.set_options(exact_sample=1)
+        assert np.array_equal(got, st.sample(draws))
+    st.close()
