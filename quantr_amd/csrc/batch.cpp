@@ -43,9 +43,7 @@ struct Inst {
   std::vector<PauliMasks> terms;
   PlanParams ppf, ppb;
   std::shared_ptr<CachedPlan> pf, pb;
-  std::vector<Loc> locf, locb;
   size_t blob_f = 0, blob_b = 0;  // offsets of the two plan blobs in the batch blob
-  size_t blob_f_size = 0, blob_b_size = 0;
   size_t obs_groups = 0, obs_terms = 0;  // byte offsets of the observable's tables in the blob
   int ngroups = 0;
   uint64_t nparams = 0, nslots = 0;
@@ -70,7 +68,8 @@ struct qr_batch {
   hipStream_t origin = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  std::vector<uint8_t> host_blob;
+  qr::PinnedLease host_blob;  // every instance's plan blobs and tables
+  size_t host_blob_size = 0;
   uint64_t total_params = 0;
   double clock_khz = 0.0;
   ~qr_batch() {
@@ -109,26 +108,11 @@ PlanParams dual_params(uint32_t n, int prec, int k = 0) {
   return pp;
 }
 
-void check_unitary_customs(const std::vector<ExactGate>& gates) {
-  for (const auto& e : gates)
-    if (e.custom) {
-      const int dim = 1 << e.K;
-      for (int r = 0; r < dim; ++r)
-        for (int c = 0; c < dim; ++c) {
-          cd s(0, 0);
-          for (int k = 0; k < dim; ++k) s += std::conj(e.M[k * dim + r]) * e.M[k * dim + c];
-          if (std::abs(s - cd(r == c ? 1.0 : 0.0, 0.0)) > 1e-10)
-            throw Error{QR_ERR_UNSUPPORTED, "adjoint differentiation needs unitary custom gates"};
-        }
-    }
-}
-
 // Lowers one instance's program (forward ops and the reverse-sweep ops).
 void lower_instance(Inst& I, const qr_program* prog) {
   validate_program(I.n, prog);
-  const std::vector<ExactGate> gates = lower_exact(I.n, prog);
-  check_unitary_customs(gates);
-  I.fwd = lower_fast(I.n, gates, true);
+  check_unitary_customs(I.n, prog);
+  I.fwd = lower_program(I.n, prog, true);
   I.rev = adjoint_sweep_ops(I.fwd);
 }
 
@@ -148,17 +132,23 @@ size_t densek_tmp_bytes(const FastOp& op, uint64_t dim, int prec) {
   return tg * dimk * (prec == 0 ? 16 : 8);
 }
 
-// Writes every instance's plan blobs and Pauli term tables at their offsets.
-void fill_blob(qr_batch* b) {
-  for (Inst& I : b->inst) {
-    std::vector<Loc> lf, lb;
-    const std::vector<uint8_t> f = pack_blob(I.fwd, I.pf->stages, lf);
-    const std::vector<uint8_t> r = pack_blob(I.rev, I.pb->stages, lb);
-    if (f.size() != I.blob_f_size || r.size() != I.blob_b_size)
-      throw Error{QR_ERR_ARG, "program structure differs from the batch's"};
-    std::memcpy(b->host_blob.data() + I.blob_f, f.data(), f.size());
-    std::memcpy(b->host_blob.data() + I.blob_b, r.data(), r.size());
-  }
+// Writes the values of instance I's programs into its plan blobs.
+void fill_blob(qr_batch* b, const Inst& I) {
+  write_values(I.fwd, I.pf->stages, I.pf->image.loc, b->host_blob.data() + I.blob_f);
+  write_values(I.rev, I.pb->stages, I.pb->image.loc, b->host_blob.data() + I.blob_b);
+}
+
+// Instances handled per host thread at least: below that, starting threads takes longer than the
+// lowering (0.1 ms for a 300-gate instance).
+constexpr size_t kInstancesPerThread = 4;
+
+// fn(i) for every instance, in groups over the host's cores.
+template <class F>
+void for_instances(size_t m, F fn) {
+  const size_t groups = (m + kInstancesPerThread - 1) / kInstancesPerThread;
+  parallel_for(groups, [&](uint64_t g) {
+    for (size_t i = g * kInstancesPerThread; i < std::min(m, (g + 1) * kInstancesPerThread); ++i) fn(i);
+  });
 }
 
 void launch_instance(qr_batch* b, const Inst& I, hipStream_t s, uint64_t* stamps, size_t idx) {
@@ -174,11 +164,11 @@ void launch_instance(qr_batch* b, const Inst& I, hipStream_t s, uint64_t* stamps
   for (size_t si = 0; si < I.pf->stages.size(); ++si) {
     const Stage& st = I.pf->stages[si];
     if (st.tile) {
-      const TileArgs a = tile_args_at(I.n, st, dblob + I.blob_f, I.locf[si]);
+      const TileArgs a = tile_args_at(I.n, st, dblob + I.blob_f, I.pf->image.loc[si]);
       hip_check(jit_launch(I.pf->fns[si], st.k, I.ppf.reg_bits, false, psi, a.coefs, a.ntiles, a.nontile_mask, s),
                 "compiled tile kernel");
     } else {
-      launch_standalone_raw(prec, I.dim, psi, b->tmp[I.stream], I.fwd[st.standalone], dblob + I.blob_f, I.locf[si], s);
+      launch_standalone_raw(prec, I.dim, psi, b->tmp[I.stream], I.fwd[st.standalone], dblob + I.blob_f, I.pf->image.loc[si], s);
     }
   }
   // lam = O psi (one pass), E = Re <psi|lam>
@@ -191,14 +181,14 @@ void launch_instance(qr_batch* b, const Inst& I, hipStream_t s, uint64_t* stamps
   for (size_t si = 0; si < I.pb->stages.size(); ++si) {
     const Stage& st = I.pb->stages[si];
     if (st.tile) {
-      const TileArgs a = tile_args_at(I.n, st, dblob + I.blob_b, I.locb[si]);
+      const TileArgs a = tile_args_at(I.n, st, dblob + I.blob_b, I.pb->image.loc[si]);
       hip_check(jit_launch_dual(I.pb->fns[si], st.k, I.ppb.reg_bits, psi, lam, a.coefs, a.ntiles, a.nontile_mask,
                                 work + I.part, I.nslots, s),
                 "compiled adjoint stage");
     } else {
       const FastOp& op = I.rev[st.standalone];
-      launch_standalone_raw(prec, I.dim, psi, b->tmp[I.stream], op, dblob + I.blob_b, I.locb[si], s);
-      launch_standalone_raw(prec, I.dim, lam, b->tmp[I.stream], op, dblob + I.blob_b, I.locb[si], s);
+      launch_standalone_raw(prec, I.dim, psi, b->tmp[I.stream], op, dblob + I.blob_b, I.pb->image.loc[si], s);
+      launch_standalone_raw(prec, I.dim, lam, b->tmp[I.stream], op, dblob + I.blob_b, I.pb->image.loc[si], s);
     }
   }
   const size_t m = b->inst.size();
@@ -297,13 +287,10 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
   // ---- layout ---------------------------------------------------------------------------------
   size_t blob_size = 0, state_bytes = 0, work_doubles = 0;
   for (Inst& I : b->inst) {
-    std::vector<Loc> tmp;
     I.blob_f = blob_size = align_up(blob_size, kAlign);
-    I.blob_f_size = pack_blob(I.fwd, I.pf->stages, I.locf).size();
-    blob_size += I.blob_f_size;
+    blob_size += I.pf->image.live;  // compiled stages read nothing else
     I.blob_b = blob_size = align_up(blob_size, kAlign);
-    I.blob_b_size = pack_blob(I.rev, I.pb->stages, I.locb).size();
-    blob_size += I.blob_b_size;
+    blob_size += I.pb->image.live;
     // the observable's tables: terms grouped by X mask
     {
       std::vector<PauliGroup> groups;
@@ -326,8 +313,11 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
     I.grad = b->total_params;
     b->total_params += I.nparams;
   }
-  b->host_blob.assign(blob_size, 0);
-  for (Inst& I : b->inst) {  // observable tables (fixed for the batch's lifetime)
+  b->host_blob.reserve(std::max<size_t>(blob_size, 1));
+  b->host_blob_size = blob_size;
+  for (Inst& I : b->inst) {  // standalone and observable tables (fixed for the batch's lifetime)
+    std::memcpy(b->host_blob.data() + I.blob_f, I.pf->image.bytes.data(), I.pf->image.live);
+    std::memcpy(b->host_blob.data() + I.blob_b, I.pb->image.bytes.data(), I.pb->image.live);
     std::vector<PauliGroup> groups;
     std::vector<PauliZTerm> flat;
     pauli_tables(I.terms, groups, flat);
@@ -335,7 +325,7 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
       std::memcpy(b->host_blob.data() + I.obs_groups, groups.data(), groups.size() * sizeof(PauliGroup));
     if (!flat.empty()) std::memcpy(b->host_blob.data() + I.obs_terms, flat.data(), flat.size() * sizeof(PauliZTerm));
   }
-  fill_blob(b.get());
+  for (const Inst& I : b->inst) fill_blob(b.get(), I);
   const size_t out_doubles = m + b->total_params;
   b->states.reserve(std::max<size_t>(state_bytes, 1));
   b->blob.reserve(std::max<size_t>(blob_size, 1));
@@ -405,27 +395,27 @@ void batch_run(qr_batch* b, const qr_program* programs, double* expvals, double*
   if (programs) {
     // lower everything first; the batch keeps its previous programs if any instance fails
     std::vector<Inst> fresh(m);
-    for (size_t i = 0; i < m; ++i) {
+    for_instances(m, [&](size_t i) {
       fresh[i].n = b->inst[i].n;
       lower_instance(fresh[i], &programs[i]);
       if (structure_key(fresh[i].fwd) != b->inst[i].key)
         throw Error{QR_ERR_ARG, "instance " + std::to_string(i) + ": program structure differs from the batch's"};
-    }
-    for (size_t i = 0; i < m; ++i) {
+    });
+    for_instances(m, [&](size_t i) {
       b->inst[i].fwd = std::move(fresh[i].fwd);
       b->inst[i].rev = std::move(fresh[i].rev);
-    }
-    fill_blob(b);
+      fill_blob(b, b->inst[i]);
+    });
   }
-  hip_check(hipMemcpyAsync(b->blob.p, b->host_blob.data(), b->host_blob.size(), hipMemcpyHostToDevice, b->origin),
+  hip_check(hipMemcpyAsync(b->blob.p, b->host_blob.data(), b->host_blob_size, hipMemcpyHostToDevice, b->origin),
             "plan upload");
   hip_check(hipGraphLaunch(b->exec, b->origin), "hipGraphLaunch");
-  const size_t out_doubles = m + b->total_params;
-  std::vector<double> h(out_doubles);
-  std::vector<uint64_t> st(m + 1);
-  hip_check(hipMemcpyAsync(h.data(), b->out.p, out_doubles * sizeof(double), hipMemcpyDeviceToHost, b->origin), "D2H");
-  hip_check(hipMemcpyAsync(st.data(), (uint8_t*)b->out.p + align_up(out_doubles * sizeof(double), kAlign),
-                           (m + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, b->origin),
+  // results and stamps lie in one buffer: one copy
+  const size_t stamp_off = align_up((m + b->total_params) * sizeof(double), kAlign);
+  PinnedLease pin(stamp_off + (m + 1) * sizeof(uint64_t));
+  const double* h = (const double*)pin.data();
+  const uint64_t* st = (const uint64_t*)(pin.data() + stamp_off);
+  hip_check(hipMemcpyAsync(pin.data(), b->out.p, stamp_off + (m + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, b->origin),
             "D2H");
   hip_check(hipStreamSynchronize(b->origin), "sync");
   for (size_t i = 0; i < m; ++i) {

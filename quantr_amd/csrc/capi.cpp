@@ -292,19 +292,8 @@ qr_status qr_grad_forward(qr_grad* g, const qr_program* program, const qr_observ
     if (!g) throw Error{QR_ERR_ARG, "grad is NULL"};
     qr_state* st = g->psi.get();
     validate_program(st->n, program);
-    auto gates = lower_exact(st->n, program);
-    for (const auto& e : gates)
-      if (e.custom) {  // the reverse sweep needs U^dagger = U^-1
-        const int dim = 1 << e.K;
-        for (int r = 0; r < dim; ++r)
-          for (int c = 0; c < dim; ++c) {
-            cd s(0, 0);
-            for (int k = 0; k < dim; ++k) s += std::conj(e.M[k * dim + r]) * e.M[k * dim + c];
-            if (std::abs(s - cd(r == c ? 1.0 : 0.0, 0.0)) > 1e-10)
-              throw Error{QR_ERR_UNSUPPORTED, "adjoint differentiation needs unitary custom gates"};
-          }
-      }
-    g->ops = lower_fast(st->n, gates, true);
+    check_unitary_customs(st->n, program);  // the reverse sweep needs U^dagger = U^-1
+    g->ops = lower_program(st->n, program, true);
     g->terms = parse_observable(st->n, observable);
     g->nparams = 0;
     for (const auto& op : g->ops)
@@ -348,7 +337,7 @@ qr_status qr_grad_backward(qr_grad* g, double grad_out, double* grads_out, uint6
     hip_check(hipStreamSynchronize(ls->stream), "sync");
     hipStream_t s = ps->stream;
     // lambda = O psi
-    apply_observable(ps->prec, ls->amp, ps->amp, ps->dim, g->terms, ls->aux, s);
+    apply_observable(ps->prec, ls->amp, ps->amp, ps->dim, g->terms, ls->aux, ps->up, s);
     if (ps->opt.fused && ps->opt.jit) {
       backward_fused(g, grad_out, grads_out);
       return;

@@ -125,6 +125,10 @@ void pauli_tile_tables(int prec, const PauliGroup* groups, const uint32_t* lxm, 
 void validate_program(uint32_t n, const qr_program* p);
 std::vector<ExactGate> lower_exact(uint32_t n, const qr_program* p);
 std::vector<FastOp> lower_fast(uint32_t n, const std::vector<ExactGate>& gates, bool want_params);
+// The same ops straight from a validated program: lower_fast(lower_exact(program)).
+std::vector<FastOp> lower_program(uint32_t n, const qr_program* p, bool want_params);
+// Throws if a custom gate of a validated program isn't unitary (the reverse sweep needs U^-1).
+void check_unitary_customs(uint32_t n, const qr_program* p);
 // Human-readable form of an op (Rust Debug style, e.g. "CNot(2)").
 std::string gate_debug(const qr_op& op, const uint32_t* controls);
 
@@ -232,5 +236,6 @@ void plan_key_append(const FastOp& op, std::vector<uint64_t>& key);
 // The 4 coefficients of every op of a tile stage (c[4i..4i+3]), taken from the program's own
 // ops with the stage's scalar folding applied.
 void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, std::vector<cd>& c);
+void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, cd* c);  // 4 * s.ops.size() entries
 
 }  // namespace qr

@@ -39,34 +39,45 @@ int wires_expected(uint32_t kind) {
   }
 }
 
-// Matrix of a standard gate, M[r*dim + j] (standard_gate_ops.rs:37-267).
-std::vector<cd> standard_matrix(uint32_t kind, double th, int kk) {
+// Matrix of a standard single-wire gate (standard_gate_ops.rs:37-267); false for other kinds.
+bool standard_2x2(uint32_t kind, double th, cd a[4]) {
   const cd z(0, 0), one(1, 0), I(0, 1);
+  auto set = [&](cd a0, cd a1, cd a2, cd a3) {
+    a[0] = a0; a[1] = a1; a[2] = a2; a[3] = a3;
+    return true;
+  };
   switch (kind) {
-    case QR_GATE_H: return {cd(kS, 0), cd(kS, 0), cd(kS, 0), cd(-kS, 0)};
-    case QR_GATE_X: return {z, one, one, z};
-    case QR_GATE_Y: return {z, cd(0, -1), I, z};
-    case QR_GATE_Z: return {one, z, z, cd(-1, 0)};
-    case QR_GATE_S: return {one, z, z, I};
-    case QR_GATE_SDAG: return {one, z, z, cd(0, -1)};
-    case QR_GATE_T: return {one, z, z, cd(kS, kS)};
-    case QR_GATE_TDAG: return {one, z, z, cd(kS, -kS)};
+    case QR_GATE_H: return set(cd(kS, 0), cd(kS, 0), cd(kS, 0), cd(-kS, 0));
+    case QR_GATE_X: return set(z, one, one, z);
+    case QR_GATE_Y: return set(z, cd(0, -1), I, z);
+    case QR_GATE_Z: return set(one, z, z, cd(-1, 0));
+    case QR_GATE_S: return set(one, z, z, I);
+    case QR_GATE_SDAG: return set(one, z, z, cd(0, -1));
+    case QR_GATE_T: return set(one, z, z, cd(kS, kS));
+    case QR_GATE_TDAG: return set(one, z, z, cd(kS, -kS));
     case QR_GATE_RX: {
       const double c = std::cos(0.5 * th), s = std::sin(0.5 * th);
-      return {cd(c, 0), cd(0, -s), cd(0, -s), cd(c, 0)};
+      return set(cd(c, 0), cd(0, -s), cd(0, -s), cd(c, 0));
     }
     case QR_GATE_RY: {
       const double c = std::cos(0.5 * th), s = std::sin(0.5 * th);
-      return {cd(c, 0), cd(-s, 0), cd(s, 0), cd(c, 0)};
+      return set(cd(c, 0), cd(-s, 0), cd(s, 0), cd(c, 0));
     }
-    case QR_GATE_RZ: return {expi(-th * 0.5), z, z, expi(th * 0.5)};
-    case QR_GATE_PHASE: return {expi(th * 0.5), z, z, expi(th * 0.5)};
-    case QR_GATE_X90: return {z, cd(0, -1), cd(0, -1), z};
-    case QR_GATE_Y90: return {z, one, cd(-1, 0), z};
-    case QR_GATE_MX90: return {z, I, I, z};
-    case QR_GATE_MY90: return {z, cd(-1, 0), one, z};
-    default: break;
+    case QR_GATE_RZ: return set(expi(-th * 0.5), z, z, expi(th * 0.5));
+    case QR_GATE_PHASE: return set(expi(th * 0.5), z, z, expi(th * 0.5));
+    case QR_GATE_X90: return set(z, cd(0, -1), cd(0, -1), z);
+    case QR_GATE_Y90: return set(z, one, cd(-1, 0), z);
+    case QR_GATE_MX90: return set(z, I, I, z);
+    case QR_GATE_MY90: return set(z, cd(-1, 0), one, z);
+    default: return false;
   }
+}
+
+// Matrix of a standard gate, M[r*dim + j] (standard_gate_ops.rs:37-267).
+std::vector<cd> standard_matrix(uint32_t kind, double th, int kk) {
+  const cd z(0, 0), one(1, 0), I(0, 1);
+  cd a[4];
+  if (standard_2x2(kind, th, a)) return std::vector<cd>(a, a + 4);
   std::vector<cd> m(16, z);
   auto set_perm = [&](const int* img) { for (int j = 0; j < 4; ++j) m[img[j] * 4 + j] = one; };
   switch (kind) {
@@ -190,16 +201,16 @@ void validate_program(uint32_t n, const qr_program* p) {
         throw arg_error("control list of gate " + std::to_string(g) + " is out of range");
     }
     const uint32_t* c = op.ncontrols ? p->controls + op.controls_offset : nullptr;
-    std::string dbg = gate_debug(op, p->controls);
+    auto dbg = [&] { return gate_debug(op, p->controls); };  // text for an error message only
     // repeated control wires (contains_repeating_values, circuit.rs:296-305)
     for (uint32_t i = 0; i < op.ncontrols; ++i)
       for (uint32_t j = i + 1; j < op.ncontrols; ++j)
         if (c[i] == c[j] && c[i] < n)
-          throw arg_error("The gate, " + dbg + ", has overlapping control nodes.");
+          throw arg_error("The gate, " + dbg() + ", has overlapping control nodes.");
     for (uint32_t i = 0; i < op.ncontrols; ++i)
       if (c[i] == op.position) {
         std::ostringstream os;
-        os << "The gate, " << dbg << ", has a control node that equals the gate's position "
+        os << "The gate, " << dbg() << ", has a control node that equals the gate's position "
            << op.position << ".";
         throw arg_error(os.str());
       }
@@ -222,45 +233,61 @@ void validate_program(uint32_t n, const qr_program* p) {
   }
 }
 
+static ExactGate exact_gate(uint32_t n, const qr_program* p, const qr_op& op) {
+  ExactGate e;
+  e.kind = op.kind;
+  e.arg = op.arg;
+  const uint32_t* c = op.ncontrols ? p->controls + op.controls_offset : nullptr;
+  for (uint32_t i = 0; i < op.ncontrols; ++i) e.bits.push_back((int)(n - 1 - c[i]));
+  e.bits.push_back((int)(n - 1 - op.position));
+  e.K = (int)e.bits.size();
+  const uint64_t dim = 1ull << e.K;
+  e.some.assign(dim, 1);
+  e.keep.assign(dim, 0);
+  if (op.kind == QR_GATE_CUSTOM) {
+    e.custom = true;
+    e.M.assign(dim * dim, cd(0, 0));
+    const double* img = p->images + op.image_offset;
+    for (uint64_t j = 0; j < dim; ++j) e.some[j] = p->some[op.some_offset + j] ? 1 : 0;
+    // Overwrite rule (simulation.rs:120-133): an input whose image is None keeps its
+    // amplitude and overwrites whatever the other inputs scattered into its slot.
+    for (uint64_t r = 0; r < dim; ++r) {
+      if (!e.some[r]) {
+        e.keep[r] = 1;
+        e.M[r * dim + r] = cd(1, 0);
+        continue;
+      }
+      for (uint64_t j = 0; j < dim; ++j)
+        if (e.some[j]) e.M[r * dim + j] = cd(img[(j * dim + r) * 2], img[(j * dim + r) * 2 + 1]);
+    }
+  } else {
+    e.M = standard_matrix(op.kind, op.arg, op.arg_int);
+  }
+  return e;
+}
+
 std::vector<ExactGate> lower_exact(uint32_t n, const qr_program* p) {
   validate_program(n, p);
   std::vector<ExactGate> out;
   out.reserve(p->nops);
-  for (uint64_t g = 0; g < p->nops; ++g) {
-    const qr_op& op = p->ops[g];
-    if (op.kind == QR_GATE_ID) continue;  // simulation.rs:38-41
-    ExactGate e;
-    e.kind = op.kind;
-    e.arg = op.arg;
-    const uint32_t* c = op.ncontrols ? p->controls + op.controls_offset : nullptr;
-    for (uint32_t i = 0; i < op.ncontrols; ++i) e.bits.push_back((int)(n - 1 - c[i]));
-    e.bits.push_back((int)(n - 1 - op.position));
-    e.K = (int)e.bits.size();
-    const uint64_t dim = 1ull << e.K;
-    e.some.assign(dim, 1);
-    e.keep.assign(dim, 0);
-    if (op.kind == QR_GATE_CUSTOM) {
-      e.custom = true;
-      e.M.assign(dim * dim, cd(0, 0));
-      const double* img = p->images + op.image_offset;
-      for (uint64_t j = 0; j < dim; ++j) e.some[j] = p->some[op.some_offset + j] ? 1 : 0;
-      // Overwrite rule (simulation.rs:120-133): an input whose image is None keeps its
-      // amplitude and overwrites whatever the other inputs scattered into its slot.
-      for (uint64_t r = 0; r < dim; ++r) {
-        if (!e.some[r]) {
-          e.keep[r] = 1;
-          e.M[r * dim + r] = cd(1, 0);
-          continue;
-        }
-        for (uint64_t j = 0; j < dim; ++j)
-          if (e.some[j]) e.M[r * dim + j] = cd(img[(j * dim + r) * 2], img[(j * dim + r) * 2 + 1]);
-      }
-    } else {
-      e.M = standard_matrix(op.kind, op.arg, op.arg_int);
-    }
-    out.push_back(std::move(e));
-  }
+  for (uint64_t g = 0; g < p->nops; ++g)
+    if (p->ops[g].kind != QR_GATE_ID) out.push_back(exact_gate(n, p, p->ops[g]));  // simulation.rs:38-41
   return out;
+}
+
+void check_unitary_customs(uint32_t n, const qr_program* p) {
+  for (uint64_t g = 0; g < p->nops; ++g) {
+    if (p->ops[g].kind != QR_GATE_CUSTOM) continue;
+    const ExactGate e = exact_gate(n, p, p->ops[g]);
+    const int dim = 1 << e.K;
+    for (int r = 0; r < dim; ++r)
+      for (int c = 0; c < dim; ++c) {
+        cd s(0, 0);
+        for (int k = 0; k < dim; ++k) s += std::conj(e.M[k * dim + r]) * e.M[k * dim + c];
+        if (std::abs(s - cd(r == c ? 1.0 : 0.0, 0.0)) > 1e-10)
+          throw Error{QR_ERR_UNSUPPORTED, "adjoint differentiation needs unitary custom gates"};
+      }
+  }
 }
 
 namespace {
@@ -310,67 +337,119 @@ bool is_diagonal(const std::vector<cd>& A, int K) {
 
 }  // namespace
 
+// The fast form of a gate from its matrix, whatever it is.
+static FastOp fast_op(const ExactGate& e) {
+  std::vector<cd> A = e.M;
+  std::vector<int> wires(e.bits);
+  int K = e.K;
+  uint64_t cmask = 0;
+  // Peel control wires (CNOT, CY, CZ, CR, CRk, Toffoli, controlled custom tables).
+  bool changed = true;
+  while (changed && K > 1) {
+    changed = false;
+    for (int q = 0; q < K; ++q) {
+      if (is_control_wire(A, K, q)) {
+        cmask |= 1ull << wires[q];
+        A = restrict_to_one(A, K, q);
+        wires.erase(wires.begin() + q);
+        --K;
+        changed = true;
+        break;
+      }
+    }
+  }
+  FastOp f;
+  f.cmask = cmask;
+  f.k = K;
+  for (int i = 0; i < K; ++i) f.bits[i] = wires[i];
+  const int dim = 1 << K;
+  const int nc = __builtin_popcountll(cmask);
+  if (is_diagonal(A, K)) {
+    f.kind = K == 1 ? FK_DIAG1 : FK_DIAGK;
+    f.m.resize(dim);
+    int nontrivial = 0;
+    for (int r = 0; r < dim; ++r) {
+      f.m[r] = A[r * dim + r];
+      if (!is_one(f.m[r])) ++nontrivial;
+    }
+    f.f_touch = (double)nontrivial / dim / (double)(1ull << nc);
+  } else {
+    f.kind = K == 1 ? FK_DENSE1 : FK_DENSEK;
+    f.m = A;
+    f.f_touch = 1.0 / (double)(1ull << nc);
+  }
+  classify(f);
+  return f;
+}
+
+// Numbers the op and, for a parameter gate, gives it its generator and parameter.
+static void finish_op(FastOp& f, int kind, int target, int index, bool want_params, int& pcount) {
+  f.gate_index = index;
+  if (!want_params) return;
+  switch (kind) {
+    case QR_GATE_RX: f.param = pcount++; f.gen = 1; break;
+    case QR_GATE_RY: f.param = pcount++; f.gen = 2; break;
+    case QR_GATE_RZ: f.param = pcount++; f.gen = 3; break;
+    case QR_GATE_PHASE: f.param = pcount++; f.gen = 4; break;
+    default: return;
+  }
+  f.k = 1;  // keep the parameter gate's bit even if the matrix is trivial
+  f.bits[0] = target;
+}
+
 std::vector<FastOp> lower_fast(uint32_t n, const std::vector<ExactGate>& gates, bool want_params) {
   std::vector<FastOp> out;
   out.reserve(gates.size());
   int pcount = 0;
   for (size_t gi = 0; gi < gates.size(); ++gi) {
-    const ExactGate& e = gates[gi];
-    std::vector<cd> A = e.M;
-    std::vector<int> wires(e.bits);
-    int K = e.K;
-    uint64_t cmask = 0;
-    // Peel control wires (CNOT, CY, CZ, CR, CRk, Toffoli, controlled custom tables).
-    bool changed = true;
-    while (changed && K > 1) {
-      changed = false;
-      for (int q = 0; q < K; ++q) {
-        if (is_control_wire(A, K, q)) {
-          cmask |= 1ull << wires[q];
-          A = restrict_to_one(A, K, q);
-          wires.erase(wires.begin() + q);
-          --K;
-          changed = true;
-          break;
-        }
-      }
-    }
-    FastOp f;
-    f.cmask = cmask;
-    f.gate_index = (int)gi;
-    f.k = K;
-    for (int i = 0; i < K; ++i) f.bits[i] = wires[i];
-    const int dim = 1 << K;
-    const int nc = __builtin_popcountll(cmask);
-    if (is_diagonal(A, K)) {
-      f.kind = K == 1 ? FK_DIAG1 : FK_DIAGK;
-      f.m.resize(dim);
-      int nontrivial = 0;
-      for (int r = 0; r < dim; ++r) {
-        f.m[r] = A[r * dim + r];
-        if (!is_one(f.m[r])) ++nontrivial;
-      }
-      f.f_touch = (double)nontrivial / dim / (double)(1ull << nc);
-    } else {
-      f.kind = K == 1 ? FK_DENSE1 : FK_DENSEK;
-      f.m = A;
-      f.f_touch = 1.0 / (double)(1ull << nc);
-    }
-    classify(f);
-    if (want_params) {
-      switch (e.kind) {
-        case QR_GATE_RX: f.param = pcount++; f.gen = 1; break;
-        case QR_GATE_RY: f.param = pcount++; f.gen = 2; break;
-        case QR_GATE_RZ: f.param = pcount++; f.gen = 3; break;
-        case QR_GATE_PHASE: f.param = pcount++; f.gen = 4; break;
-        default: break;
-      }
-      if (f.param >= 0) {  // keep the parameter gate's bit even if the matrix is trivial
-        f.k = 1;
-        f.bits[0] = e.bits.back();
-      }
-    }
-    out.push_back(std::move(f));
+    out.push_back(fast_op(gates[gi]));
+    finish_op(out.back(), gates[gi].kind, gates[gi].bits.back(), (int)gi, want_params, pcount);
+  }
+  return out;
+}
+
+// The fast form of a standard gate without going through its full matrix: its controls are known
+// to be controls, and the rest is the 2x2 they leave (a Swap keeps its 4x4).
+static FastOp standard_op(uint32_t n, const qr_program* p, const qr_op& op) {
+  static const cd z(0, 0), one(1, 0), I(0, 1);
+  cd a[4];
+  switch (op.kind) {
+    case QR_GATE_SWAP: return fast_op(exact_gate(n, p, op));
+    case QR_GATE_CNOT:
+    case QR_GATE_TOFFOLI: a[0] = z; a[1] = one; a[2] = one; a[3] = z; break;
+    case QR_GATE_CY: a[0] = z; a[1] = cd(0, -1); a[2] = I; a[3] = z; break;
+    case QR_GATE_CZ: a[0] = one; a[1] = z; a[2] = z; a[3] = cd(-1, 0); break;
+    case QR_GATE_CR: a[0] = one; a[1] = z; a[2] = z; a[3] = expi(op.arg); break;
+    case QR_GATE_CRK: a[0] = one; a[1] = z; a[2] = z; a[3] = expi((2.0 * M_PI) / std::ldexp(1.0, op.arg_int)); break;
+    default: standard_2x2(op.kind, op.arg, a); break;
+  }
+  FastOp f;
+  for (uint32_t i = 0; i < op.ncontrols; ++i) f.cmask |= 1ull << (n - 1 - p->controls[op.controls_offset + i]);
+  f.bits[0] = (int)(n - 1 - op.position);
+  const double part = 1.0 / (double)(1ull << op.ncontrols);
+  if (is_zero(a[1]) && is_zero(a[2])) {
+    f.kind = FK_DIAG1;
+    f.m = {a[0], a[3]};
+    f.f_touch = ((is_one(a[0]) ? 0 : 1) + (is_one(a[3]) ? 0 : 1)) / 2.0 * part;
+  } else {
+    f.kind = FK_DENSE1;
+    f.m.assign(a, a + 4);
+    f.f_touch = part;
+  }
+  classify(f);
+  return f;
+}
+
+std::vector<FastOp> lower_program(uint32_t n, const qr_program* p, bool want_params) {
+  std::vector<FastOp> out;
+  out.reserve(p->nops);
+  int pcount = 0;
+  for (uint64_t g = 0; g < p->nops; ++g) {
+    const qr_op& op = p->ops[g];
+    if (op.kind == QR_GATE_ID) continue;
+    const int index = (int)out.size();
+    out.push_back(op.kind == QR_GATE_CUSTOM ? fast_op(exact_gate(n, p, op)) : standard_op(n, p, op));
+    finish_op(out.back(), (int)op.kind, (int)(n - 1 - op.position), index, want_params, pcount);
   }
   return out;
 }

@@ -925,7 +925,12 @@ std::vector<Stage> plan_fused(uint32_t n, const std::vector<FastOp>& ops, const 
 }
 
 void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, std::vector<cd>& c) {
-  c.assign(4 * s.ops.size(), cd(0, 0));
+  c.resize(4 * s.ops.size());
+  stage_coefficients(s, ops, c.data());
+}
+
+void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, cd* c) {
+  std::fill(c, c + 4 * s.ops.size(), cd(0, 0));
   cd total(1, 0);
   int absorber = -1, scaler = -1;
   for (size_t i = 0; i < s.ops.size(); ++i) {

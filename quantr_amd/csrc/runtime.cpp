@@ -94,6 +94,26 @@ PinnedLease::~PinnedLease() {
   else pinned_give_back(p_, cap_);
 }
 
+Uploader::~Uploader() {
+  for (hipEvent_t e : ev_)
+    if (e) (void)hipEventDestroy(e);
+}
+
+uint8_t* Uploader::begin(size_t bytes) {
+  at_ ^= 1;
+  if (busy_[at_]) hip_check(hipEventSynchronize(ev_[at_]), "hipEventSynchronize");
+  busy_[at_] = false;
+  buf_[at_].reserve(std::max<size_t>(bytes, 1));
+  return buf_[at_].data();
+}
+
+void Uploader::send(void* dst, size_t bytes, hipStream_t s) {
+  if (!ev_[at_]) hip_check(hipEventCreateWithFlags(&ev_[at_], hipEventDisableTiming), "hipEventCreate");
+  hip_check(hipMemcpyAsync(dst, buf_[at_].data(), bytes, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
+  hip_check(hipEventRecord(ev_[at_], s), "hipEventRecord");
+  busy_[at_] = true;
+}
+
 // Default tile shape: 2^12 complex128 / 2^13 complex64 amplitudes (64 KB of LDS, two
 // workgroups per CU), 16 amplitudes per thread.
 int pick_tile_bits(const qr_state* st) {
@@ -140,76 +160,100 @@ PlanParams plan_params(uint32_t n, int prec, const qr_options& opt) {
   return pp;
 }
 
-// Device copy of a plan: every tile stage's ops, coefficients, slot maps and LDS patterns,
-// and the standalone ops' tables, in one upload.
-std::vector<uint8_t> pack_blob(const std::vector<FastOp>& ops, const std::vector<Stage>& stages, std::vector<Loc>& loc) {
-  std::vector<uint8_t> blob;
+PlanImage plan_image(const std::vector<FastOp>& ops, const std::vector<Stage>& stages) {
+  PlanImage im;
+  std::vector<uint8_t>& blob = im.bytes;
   auto align = [&](size_t a) {
     while (blob.size() % a) blob.push_back(0);
   };
   auto append = [&](const void* p, size_t bytes) {
     size_t off = blob.size();
     blob.resize(off + bytes);
-    if (bytes) std::memcpy(blob.data() + off, p, bytes);
+    if (bytes && p) std::memcpy(blob.data() + off, p, bytes);
     return off;
   };
-  loc.assign(stages.size(), Loc{});
+  im.loc.assign(stages.size(), Loc{});
+  // ---- coefficients and standalone tables
   for (size_t si = 0; si < stages.size(); ++si) {
     const Stage& s = stages[si];
+    Loc& loc = im.loc[si];
+    align(16);
     if (s.tile) {
-      align(64);
-      std::vector<TileOpDev> d(s.ops.size());
-      std::vector<double2> c(s.ops.size() * 4);
-      for (size_t i = 0; i < s.ops.size(); ++i) {
-        const TileOpHost& h = s.ops[i];
-        TileOpDev t{};
-        const bool maps_op = h.code == TC_REMAP || h.code == TC_SWAPSLOTS;
-        t.w0 = (h.code & 0xFF) | ((maps_op ? 0u : (h.a & 0xFF)) << 8) | ((h.b & 0xFF) << 16) | ((h.flags & 0xFF) << 24);
-        t.ns = h.ns;
-        t.lane_cmask = h.lane_cmask;
-        t.map = maps_op ? h.a : 0;
-        t.swz = h.swz;
-        d[i] = t;
-      }
-      // the current program's coefficients (plans are shared by structure), folded scalars
-      // applied; gradient taps carry their parameter row
-      std::vector<cd> cv;
-      stage_coefficients(s, ops, cv);
-      for (size_t i = 0; i < cv.size(); ++i) c[i] = make_double2(cv[i].real(), cv[i].imag());
-      loc[si].ops = append(d.data(), d.size() * sizeof(TileOpDev));
-      align(16);
-      loc[si].coefs = append(c.data(), c.size() * sizeof(double2));
-      align(4);
-      std::vector<uint32_t> m(s.maps.size());
-      for (size_t i = 0; i < m.size(); ++i)  // physical bit | tile position << 8
-        m[i] = (uint32_t)s.phys_bit((int)(i / s.k), s.maps[i]) | ((uint32_t)s.maps[i] << 8);
-      loc[si].maps = append(m.data(), m.size() * sizeof(uint32_t));
-      std::vector<uint32_t> z(s.swz.begin(), s.swz.end());
-      if (z.empty()) z.push_back(0);
-      loc[si].off = append(z.data(), z.size() * sizeof(uint32_t));
-    } else {
-      const FastOp& op = ops[s.standalone];
-      if (op.kind == FK_DENSEK || op.kind == FK_DIAGK) {
-        align(16);
-        std::vector<double2> c(op.m.size());
-        for (size_t i = 0; i < c.size(); ++i) c[i] = make_double2(op.m[i].real(), op.m[i].imag());
-        loc[si].coefs = append(c.data(), c.size() * sizeof(double2));
-        align(8);
-        const int dim = 1 << op.k;
-        std::vector<uint64_t> off(dim, 0);
-        for (int j = 0; j < dim; ++j)
-          for (int q = 0; q < op.k; ++q)
-            if ((j >> (op.k - 1 - q)) & 1) off[j] |= 1ull << op.bits[q];
-        loc[si].off = append(off.data(), off.size() * sizeof(uint64_t));
-      }
+      loc.coefs = append(nullptr, s.ops.size() * 4 * sizeof(double2));
+      continue;
+    }
+    const FastOp& op = ops[s.standalone];
+    if (op.kind == FK_DENSEK || op.kind == FK_DIAGK) {
+      loc.coefs = append(nullptr, op.m.size() * sizeof(double2));
+      align(8);
+      const int dim = 1 << op.k;
+      std::vector<uint64_t> off(dim, 0);
+      for (int j = 0; j < dim; ++j)
+        for (int q = 0; q < op.k; ++q)
+          if ((j >> (op.k - 1 - q)) & 1) off[j] |= 1ull << op.bits[q];
+      loc.off = append(off.data(), off.size() * sizeof(uint64_t));
     }
   }
-  return blob;
+  im.live = blob.size();
+  // ---- what interpreted stages read
+  for (size_t si = 0; si < stages.size(); ++si) {
+    const Stage& s = stages[si];
+    if (!s.tile) continue;
+    align(64);
+    std::vector<TileOpDev> d(s.ops.size());
+    for (size_t i = 0; i < s.ops.size(); ++i) {
+      const TileOpHost& h = s.ops[i];
+      TileOpDev t{};
+      const bool maps_op = h.code == TC_REMAP || h.code == TC_SWAPSLOTS;
+      t.w0 = (h.code & 0xFF) | ((maps_op ? 0u : (h.a & 0xFF)) << 8) | ((h.b & 0xFF) << 16) | ((h.flags & 0xFF) << 24);
+      t.ns = h.ns;
+      t.lane_cmask = h.lane_cmask;
+      t.map = maps_op ? h.a : 0;
+      t.swz = h.swz;
+      d[i] = t;
+    }
+    im.loc[si].ops = append(d.data(), d.size() * sizeof(TileOpDev));
+    align(4);
+    std::vector<uint32_t> m(s.maps.size());
+    for (size_t i = 0; i < m.size(); ++i)  // physical bit | tile position << 8
+      m[i] = (uint32_t)s.phys_bit((int)(i / s.k), s.maps[i]) | ((uint32_t)s.maps[i] << 8);
+    im.loc[si].maps = append(m.data(), m.size() * sizeof(uint32_t));
+    std::vector<uint32_t> z(s.swz.begin(), s.swz.end());
+    if (z.empty()) z.push_back(0);
+    im.loc[si].off = append(z.data(), z.size() * sizeof(uint32_t));
+  }
+  write_values(ops, stages, im.loc, blob.data());
+  return im;
 }
 
-void pack_plan(qr_state* st, const std::vector<FastOp>& ops, PackedPlan& P) {
-  const std::vector<uint8_t> blob = pack_blob(ops, P.stages, P.loc);
-  P.dblob = upload(st, st->aux, blob);
+void write_values(const std::vector<FastOp>& ops, const std::vector<Stage>& stages, const std::vector<Loc>& loc,
+                  uint8_t* blob) {
+  static_assert(sizeof(cd) == sizeof(double2), "coefficients are stored as pairs of doubles");
+  for (size_t si = 0; si < stages.size(); ++si) {
+    const Stage& s = stages[si];
+    cd* c = reinterpret_cast<cd*>(blob + loc[si].coefs);
+    if (s.tile) {
+      // the program's own coefficients (plans are shared by structure), folded scalars applied;
+      // gradient taps carry their parameter row
+      stage_coefficients(s, ops, c);
+      continue;
+    }
+    const FastOp& op = ops[s.standalone];
+    if (op.kind == FK_DENSEK || op.kind == FK_DIAGK) std::copy(op.m.begin(), op.m.end(), c);
+  }
+}
+
+void upload_plan(qr_state* st, const std::vector<FastOp>& ops, const CachedPlan& cp, bool live_only, PackedPlan& P) {
+  const PlanImage& im = cp.image;
+  const size_t bytes = live_only ? im.live : im.bytes.size();
+  uint8_t* h = st->up.begin(bytes);
+  std::memcpy(h, im.bytes.data(), bytes);
+  write_values(ops, cp.stages, im.loc, h);
+  st->aux.reserve(im.bytes.size() + 256);
+  if (bytes) st->up.send(st->aux.p, bytes, st->stream);
+  P.stages = &cp.stages;
+  P.loc = &im.loc;
+  P.dblob = (const uint8_t*)st->aux.p;
 }
 
 TileArgs tile_args_at(uint32_t n, const Stage& s, const uint8_t* dblob, const Loc& l) {
@@ -227,7 +271,7 @@ TileArgs tile_args_at(uint32_t n, const Stage& s, const uint8_t* dblob, const Lo
 }
 
 TileArgs tile_args(const qr_state* st, const PackedPlan& P, size_t si) {
-  return tile_args_at(st->n, P.stages[si], P.dblob, P.loc[si]);
+  return tile_args_at(st->n, (*P.stages)[si], P.dblob, (*P.loc)[si]);
 }
 
 void launch_standalone_raw(int prec, uint64_t dim, void* amp, DevBuf& tmp, const FastOp& op, const uint8_t* dblob,
@@ -284,8 +328,8 @@ void launch_standalone_raw(int prec, uint64_t dim, void* amp, DevBuf& tmp, const
 // One standalone (unfused) op on `amp`, a state of st's size, on st's stream.
 void launch_standalone(qr_state* st, void* amp, const FastOp& op, const PackedPlan& P, size_t si) {
   static const char* names[] = {"dense1", "diag1", "densek", "diagk"};
-  ProfScope ps_(st, op.kind >= 0 && op.kind < 4 ? names[op.kind] : "standalone", P.stages[si].bytes);
-  launch_standalone_raw(st->prec, st->dim, amp, st->tmp, op, P.dblob, P.loc[si], st->stream);
+  ProfScope ps_(st, op.kind >= 0 && op.kind < 4 ? names[op.kind] : "standalone", (*P.stages)[si].bytes);
+  launch_standalone_raw(st->prec, st->dim, amp, st->tmp, op, P.dblob, (*P.loc)[si], st->stream);
 }
 
 // ---- plan cache ---------------------------------------------------------------------------
@@ -364,6 +408,7 @@ std::shared_ptr<CachedPlan> get_plan_for(uint32_t n, int prec, const std::vector
       cp->stages.push_back(std::move(s));
     }
   }
+  cp->image = plan_image(ops, cp->stages);
   std::lock_guard<std::mutex> lk(g_plan_mu);
   cp->stamp = ++g_plan_clock;
   g_plans[key] = cp;
@@ -421,6 +466,7 @@ std::shared_ptr<TuneState> tune_state(qr_state* st, const std::shared_ptr<Cached
   for (size_t i = 1; i < alt.size(); ++i) {
     auto c = std::make_shared<CachedPlan>();
     c->stages = std::move(alt[i]);
+    c->image = plan_image(ops, c->stages);
     ts->cands.push_back(std::move(c));
   }
   ts->cand_ms.assign(ts->cands.size(), 0.0);
@@ -455,10 +501,7 @@ void run_fast(qr_state* st, const std::vector<FastOp>& ops, bool fused, qr_plan_
       tune_lock.unlock();
     }
   }
-  PackedPlan P;
-  P.stages = use->stages;
-  std::vector<Stage>& stages = P.stages;
-  pack_plan(st, ops, P);
+  const std::vector<Stage>& stages = use->stages;
   // ---- runtime-specialised stages: always with jit = 1, from 28 qubits or from the second
   // application of a structure with jit = 2, and for every measured plan
   bool use_jit = false;
@@ -467,6 +510,8 @@ void run_fast(qr_state* st, const std::vector<FastOp>& ops, bool fused, qr_plan_
     if (use_jit) prepare_compiled(*use, st->prec, pp.reg_bits, persistent, false);
   }
   cp->runs++;
+  PackedPlan P;
+  upload_plan(st, ops, *use, use_jit, P);
   std::unique_ptr<StageTimer> timer;
   if (step >= 0) timer = std::make_unique<StageTimer>(stages.size());
   // tiles dealt to the XCDs in contiguous eighths by default (faster on most sweeps of the
@@ -651,13 +696,11 @@ qr_state* new_state(uint32_t n, qr_precision p) {
 
 void do_apply(qr_state* st, const qr_program* prog) {
   validate_program(st->n, prog);
-  std::vector<ExactGate> gates = lower_exact(st->n, prog);
   if (!st->opt.fused) {
-    run_exact(st, gates, &st->last);
+    run_exact(st, lower_exact(st->n, prog), &st->last);
     return;
   }
-  std::vector<FastOp> ops = lower_fast(st->n, gates, false);
-  run_fast(st, ops, true, &st->last);
+  run_fast(st, lower_program(st->n, prog, false), true, &st->last);
 }
 
 double sum_partials_host(const double* v, size_t count) {
@@ -696,41 +739,40 @@ double expectation(qr_state* st, const std::vector<PauliMasks>& terms) {
   const int np = pauli_passes(st->n, st->prec, groups.data(), G, passes.data(), lxm.data());
   // device tables: group records, then term records
   const size_t gb = (size_t)(G + 1) * sizeof(PauliGroup), tb = (flat.size() + 1) * sizeof(PauliZTerm);
-  std::vector<uint8_t> blob(gb + tb, 0);
   std::vector<PauliTilePass> tp(np);
   uint32_t diag_count[16];
-  pauli_tile_tables(st->prec, groups.data(), lxm.data(), passes.data(), np, flat.data(), blob.data(), blob.data() + gb,
-                    tp.data(), diag_count);
-  uint8_t* d = upload(st, st->aux, blob);
+  uint8_t* blob = st->up.begin(gb + tb);
+  pauli_tile_tables(st->prec, groups.data(), lxm.data(), passes.data(), np, flat.data(), blob, blob + gb, tp.data(),
+                    diag_count);
+  st->aux.reserve(gb + tb);
+  st->up.send(st->aux.p, gb + tb, st->stream);
+  const uint8_t* d = (const uint8_t*)st->aux.p;
   const int nb = pauli_expect_partials(st->dim);
-  st->aux2.reserve(nb * sizeof(double));
+  PinnedLease pin(nb * sizeof(double));  // the kernels write the partial sums there
   hip_check(launch_pauli_expect_passes(st->prec, st->amp, st->dim, d, d + gb, tp.data(), np, diag_count,
-                                       (double*)st->aux2.p, st->stream),
+                                       (double*)pin.data(), st->stream),
             "expectation");
-  std::vector<double> h(nb);
-  hip_check(hipMemcpyAsync(h.data(), st->aux2.p, nb * sizeof(double), hipMemcpyDeviceToHost, st->stream), "D2H");
   hip_check(hipStreamSynchronize(st->stream), "sync");
-  return sum_partials_host(h);
+  return sum_partials_host((const double*)pin.data(), nb);
 }
 
 
 void apply_observable(int prec, void* lam, const void* psi, uint64_t dim, const std::vector<PauliMasks>& terms,
-                      DevBuf& scratch, hipStream_t s) {
+                      DevBuf& scratch, Uploader& up, hipStream_t s) {
   std::vector<PauliGroup> groups;
   std::vector<PauliZTerm> flat;
   pauli_tables(terms, groups, flat);
   const size_t gb = groups.size() * sizeof(PauliGroup), tb = flat.size() * sizeof(PauliZTerm);
   scratch.reserve(gb + tb + 16);
-  std::vector<uint8_t> blob(gb + tb);
-  if (gb) std::memcpy(blob.data(), groups.data(), gb);
-  if (tb) std::memcpy(blob.data() + gb, flat.data(), tb);
-  if (!blob.empty())
-    hip_check(hipMemcpyAsync(scratch.p, blob.data(), blob.size(), hipMemcpyHostToDevice, s), "H2D");
+  if (gb + tb) {
+    uint8_t* blob = up.begin(gb + tb);
+    std::memcpy(blob, groups.data(), gb);
+    std::memcpy(blob + gb, flat.data(), tb);
+    up.send(scratch.p, gb + tb, s);
+  }
   hip_check(launch_pauli_sum(prec, lam, psi, dim, (const PauliGroup*)scratch.p, (int)groups.size(),
                              (const PauliZTerm*)((uint8_t*)scratch.p + gb), s),
             "pauli sum");
-  // the tables must outlive the launch that reads them
-  hip_check(hipStreamSynchronize(s), "sync");
 }
 
 // Tile shape of the adjoint sweep: psi and lam share a workgroup, so tiles are half the
@@ -758,15 +800,15 @@ void backward_fused(qr_grad* g, double grad_out, double* grads_out) {
   std::shared_ptr<CachedPlan> cp = get_plan(ps, rev, pp, true, true, false);
   prepare_compiled(*cp, ps->prec, pp.reg_bits, false, true);
   PackedPlan P;
-  P.stages = cp->stages;
-  pack_plan(ps, rev, P);
+  upload_plan(ps, rev, *cp, true, P);
   const uint64_t nslots = jit_dual_slots((int)ps->n, pp.tile_bits, pp.reg_bits);
   const uint64_t np = g->nparams;
-  ls->aux2.reserve((std::max<uint64_t>(np, 1) * nslots + np + 1) * sizeof(double));
+  ls->aux2.reserve(std::max<uint64_t>(np, 1) * nslots * sizeof(double));
   double* part = (double*)ls->aux2.p;
-  double* sums = part + std::max<uint64_t>(np, 1) * nslots;
-  for (size_t si = 0; si < P.stages.size(); ++si) {
-    const Stage& st = P.stages[si];
+  PinnedLease pin((np + 1) * sizeof(double));
+  double* h = (double*)pin.data();  // the row sums, written there by their kernel
+  for (size_t si = 0; si < cp->stages.size(); ++si) {
+    const Stage& st = cp->stages[si];
     if (st.tile) {
       const TileArgs a = tile_args(ps, P, si);
       ProfScope ps_(ps, "adjoint_sweep", 2.0 * st.bytes);
@@ -780,9 +822,7 @@ void backward_fused(qr_grad* g, double grad_out, double* grads_out) {
       launch_standalone(ps, ls->amp, op, P, si);
     }
   }
-  hip_check(launch_sum_rows(part, nslots, (uint32_t)np, sums, s), "gradient sums");
-  std::vector<double> h(np);
-  if (np) hip_check(hipMemcpyAsync(h.data(), sums, np * sizeof(double), hipMemcpyDeviceToHost, s), "D2H");
+  hip_check(launch_sum_rows(part, nslots, (uint32_t)np, h, s), "gradient sums");
   hip_check(hipStreamSynchronize(s), "sync");
   g->have_forward = false;
   for (const auto& op : g->ops) {

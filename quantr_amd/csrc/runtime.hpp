@@ -4,11 +4,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "engine.hpp"
@@ -61,6 +64,22 @@ class PinnedLease {
 void pinned_state_created();    // one more state lives
 void pinned_state_destroyed();  // one less; the last one frees the kept blocks
 
+// Uploads of small host data onto a stream without waiting for it: two pinned blocks in turn, each
+// reused once its last copy is done. The owner's stream is idle before it is destroyed.
+class Uploader {
+ public:
+  ~Uploader();
+  // A block of `bytes` to fill, then send() it to dst on stream s.
+  uint8_t* begin(size_t bytes);
+  void send(void* dst, size_t bytes, hipStream_t s);
+
+ private:
+  PinnedLease buf_[2];
+  hipEvent_t ev_[2] = {nullptr, nullptr};
+  bool busy_[2] = {false, false};
+  int at_ = 0;
+};
+
 struct ProfRec {
   std::string name;
   hipEvent_t a, b;
@@ -84,9 +103,11 @@ struct qr_state {
   qr_plan_stats last{};
   bool profiling = false;
   std::vector<qr::ProfRec> prof;
+  qr::Uploader up;
   bool counted = false;  // among the states that keep pinned blocks alive
   size_t bytes_per_amp() const { return prec == 0 ? 16 : 8; }
   ~qr_state() {
+    if (stream) (void)hipStreamSynchronize(stream);
     if (counted) qr::pinned_state_destroyed();
     for (auto& r : prof) {
       (void)hipEventDestroy(r.a);
@@ -149,17 +170,27 @@ struct Loc {
   size_t ops = 0, maps = 0, coefs = 0, off = 0;
 };
 
+// Host image of a plan's blob, made once per plan: what a program's values fill (coefficients) and
+// the standalone tables first, [0, live), then what only interpreted stages read (ops, maps, LDS
+// patterns).
+struct PlanImage {
+  std::vector<uint8_t> bytes;
+  std::vector<Loc> loc;
+  size_t live = 0;
+};
+
 // A plan's stages plus the device copy of its blob.
 struct PackedPlan {
-  std::vector<Stage> stages;
-  std::vector<Loc> loc;
-  uint8_t* dblob = nullptr;
+  const std::vector<Stage>* stages = nullptr;
+  const std::vector<Loc>* loc = nullptr;
+  const uint8_t* dblob = nullptr;
 };
 
 struct TuneState;
 
 // A plan shared by every program of one structure, with its compiled stages.
 struct CachedPlan {
+  PlanImage image;
   std::vector<Stage> stages;
   std::mutex compile_mu;           // held while this plan's stages compile (not the cache lock)
   std::vector<std::string> src;    // compiled-stage sources (filled on first compiled use)
@@ -190,10 +221,13 @@ std::shared_ptr<CachedPlan> get_plan(const qr_state* st, const std::vector<FastO
 std::shared_ptr<CachedPlan> get_plan_for(uint32_t n, int prec, const std::vector<FastOp>& ops, const PlanParams& pp,
                                          bool fused, bool dual, bool persistent);
 void prepare_compiled(CachedPlan& cp, int prec, int RB, bool persistent, bool dual);
-// Host image of a plan's blob (stage ops, coefficients from `ops`, maps, LDS patterns and the
-// standalone tables); loc receives each stage's offsets.
-std::vector<uint8_t> pack_blob(const std::vector<FastOp>& ops, const std::vector<Stage>& stages, std::vector<Loc>& loc);
-void pack_plan(qr_state* st, const std::vector<FastOp>& ops, PackedPlan& P);
+// The image of a plan (its values those of `ops`, a program of the plan's structure).
+PlanImage plan_image(const std::vector<FastOp>& ops, const std::vector<Stage>& stages);
+// Writes the values of `ops` into a copy of the image's first `live` bytes.
+void write_values(const std::vector<FastOp>& ops, const std::vector<Stage>& stages, const std::vector<Loc>& loc,
+                  uint8_t* blob);
+// Uploads the plan's blob with the values of `ops` (all of it, or only its live part) to st->aux.
+void upload_plan(qr_state* st, const std::vector<FastOp>& ops, const CachedPlan& cp, bool live_only, PackedPlan& P);
 TileArgs tile_args_at(uint32_t n, const Stage& s, const uint8_t* dblob, const Loc& loc);
 // One standalone op on a state of 2^n amplitudes (tmp: staging for wide dense gates).
 void launch_standalone_raw(int prec, uint64_t dim, void* amp, DevBuf& tmp, const FastOp& op, const uint8_t* dblob,
@@ -218,11 +252,34 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
                      const double* u, uint64_t* out);
 double norm_sqr(qr_state* st);
 double expectation(qr_state* st, const std::vector<PauliMasks>& terms);
+// fn(i) for i in [0, count) on up to 16 of the host's cores; the error of the lowest failing i is
+// rethrown.
+template <class F>
+void parallel_for(uint64_t count, F fn) {
+  const unsigned nt = (unsigned)std::min<uint64_t>(count, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
+  std::vector<std::exception_ptr> err(count);
+  std::atomic<uint64_t> next{0};
+  auto work = [&] {
+    for (uint64_t i = next++; i < count; i = next++) {
+      try {
+        fn(i);
+      } catch (...) {
+        err[i] = std::current_exception();
+      }
+    }
+  };
+  std::vector<std::thread> th;
+  for (unsigned t = 1; t < nt; ++t) th.emplace_back(work);
+  work();
+  for (auto& t : th) t.join();
+  for (auto& e : err)
+    if (e) std::rethrow_exception(e);
+}
 // The same value through fixed device and host arrays: no allocation (noalloc.cpp).
 double expectation_noalloc(qr_state* st, const qr_observable* o);
 // lam = O psi for an observable, on stream s (one pass over the state).
 void apply_observable(int prec, void* lam, const void* psi, uint64_t dim, const std::vector<PauliMasks>& terms,
-                      DevBuf& scratch, hipStream_t s);
+                      DevBuf& scratch, Uploader& up, hipStream_t s);
 void backward_fused(qr_grad* g, double grad_out, double* grads_out);
 
 // ---- batches (batch.cpp) ------------------------------------------------------------------------

@@ -37,29 +37,6 @@ struct Prepared {
   std::vector<uint64_t> key;
 };
 
-// fn(i) for i in [0, count) on the host's cores; the error of the lowest failing i is rethrown.
-template <class F>
-void parallel_for(uint64_t count, F fn) {
-  const unsigned nt = (unsigned)std::min<uint64_t>(count, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
-  std::vector<std::exception_ptr> err(count);
-  std::atomic<uint64_t> next{0};
-  auto work = [&] {
-    for (uint64_t i = next++; i < count; i = next++) {
-      try {
-        fn(i);
-      } catch (...) {
-        err[i] = std::current_exception();
-      }
-    }
-  };
-  std::vector<std::thread> th;
-  for (unsigned t = 1; t < nt; ++t) th.emplace_back(work);
-  work();
-  for (auto& t : th) t.join();
-  for (auto& e : err)
-    if (e) std::rethrow_exception(e);
-}
-
 }  // namespace
 
 void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t count, const uint64_t* draws,
@@ -85,7 +62,7 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
   std::vector<std::vector<uint64_t>> order;
   parallel_for(count, [&](uint64_t j) {
     validate_program(n, &programs[j]);
-    pr[j].ops = lower_fast(n, lower_exact(n, &programs[j]), false);
+    pr[j].ops = lower_program(n, &programs[j], false);
     for (const FastOp& op : pr[j].ops) plan_key_append(op, pr[j].key);
   });
   for (uint64_t j = 0; j < count; ++j) {
@@ -116,8 +93,8 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
     std::shared_ptr<CachedPlan> cp = get_plan_for(n, prec, pr[members[0]].ops, pp, true, false, false);
     prepare_compiled(*cp, prec, pp.reg_bits, false, false);
     const std::vector<Stage>& stages = cp->stages;
-    std::vector<Loc> loc;
-    const size_t blob_size = pack_blob(pr[members[0]].ops, stages, loc).size();
+    const std::vector<Loc>& loc = cp->image.loc;
+    const size_t blob_size = cp->image.live;  // compiled stages read nothing else
     const size_t blob_stride = (blob_size + 255) & ~(size_t)255;
     const uint64_t per_chunk =
         std::max<uint64_t>(1, std::min<uint64_t>(kMaxGridY, kChunkBytes / (dim * B)));
@@ -126,10 +103,8 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
       // coefficient blobs of the chunk's programs, back to back (same layout: same plan)
       std::vector<uint8_t> host(cnt * blob_stride, 0);
       parallel_for(cnt, [&](uint64_t y) {
-        std::vector<Loc> ly;
-        std::vector<uint8_t> b = pack_blob(pr[members[c0 + y]].ops, stages, ly);
-        if (b.size() != blob_size) throw Error{QR_ERR_UNSUPPORTED, "internal error: blob layouts differ"};
-        std::memcpy(host.data() + y * blob_stride, b.data(), b.size());
+        std::memcpy(host.data() + y * blob_stride, cp->image.bytes.data(), blob_size);
+        write_values(pr[members[c0 + y]].ops, stages, loc, host.data() + y * blob_stride);
       });
       blobs.reserve(host.size());
       hip_check(hipMemcpyAsync(blobs.p, host.data(), host.size(), hipMemcpyHostToDevice, s), "H2D");
