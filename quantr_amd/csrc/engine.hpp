@@ -162,9 +162,13 @@ struct TileOpHost {
 // factors is multiplied into one general-form op (FOLD_ABSORB) or applied by TC_SCALE.
 // FOLD_RROT / FOLD_XROT divide out the magnitude and a sign, leaving a rotation by at most
 // pi/2 that the kernel applies as three shears.
+// FOLD_DROP_*: the same for the parameter gates of an adjoint sweep, whose factors are dropped:
+// they have modulus 1 and both states take them, so the taps <lam| G |psi> do not see them. The
+// op keeps its plain form and values in the plan; compiled stages and launch coefficients take
+// the folded ones.
 enum FoldMode : int {
   FOLD_NONE = 0, FOLD_M00 = 1, FOLD_M10 = 2, FOLD_D0 = 3, FOLD_ABSORB = 4, FOLD_SCALE = 5, FOLD_RROT = 6,
-  FOLD_XROT = 7
+  FOLD_XROT = 7, FOLD_DROP_D0 = 8, FOLD_DROP_RROT = 9, FOLD_DROP_XROT = 10
 };
 
 struct Stage {

@@ -50,6 +50,8 @@ struct JitKernel {
   hipFunction_t fn = nullptr;
 };
 
+constexpr size_t kTapRows = 14;  // qr::dev::kTapRows of tile_ops.hpp
+
 std::mutex g_mu;
 std::map<std::string, JitKernel> g_cache;
 
@@ -150,6 +152,27 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
   if (!dual) o << "  psi += (uint64_t)blockIdx.y * inst_stride;\n  cf += (uint64_t)blockIdx.y * cf_stride;\n";
   o << "  using R = " << R << ";\n";
   o << "  __shared__ " << C << " lds[" << (split ? (1 << (K - 1)) : (lds2 ? 2 : 1) * (1 << K)) << "];\n";
+  // gradient taps go through LDS rows of their wavefront, summed together (tile_ops.hpp)
+  std::vector<size_t> taps;  // ops whose rows are waiting
+  bool rows = false;
+  if (dual && TPB >= 64)
+    for (const TileOpHost& op : s.ops) rows = rows || op.code == TC_GRAD;
+  if (rows)
+    o << "  __shared__ __align__(16) double taprows[" << TPB / 64 << " * qr::dev::kTapRows * qr::dev::kTapStride];\n"
+      << "  double* const myrows = taprows + (threadIdx.x >> 6) * (qr::dev::kTapRows * qr::dev::kTapStride);\n";
+  auto flush_taps = [&]() {
+    if (taps.empty()) return;
+    // the parameter's row comes from the op's coefficient slot, so that stages differing only in
+    // parameter numbering share one kernel
+    o << "  __syncthreads();\n  { const uint32_t lane = tid & 63u, q = lane >> 2;\n    uint32_t at = " << 4 * taps[0] << "u;\n";
+    for (size_t j = 1; j < taps.size(); ++j) o << "    if (q == " << j << "u) at = " << 4 * taps[j] << "u;\n";
+    o << "    const double prow = cf[at].x;\n"
+      << "    const double sum = qr::dev::tap_sum(myrows, " << taps.size() << ", lane);\n"
+      << "    if ((lane & 3u) == 0u && q < " << taps.size() << "u)\n"
+      << "      part[(uint64_t)prow * nslots + tile * " << TPB / 64 << "u + (tid >> 6)] = sum; }\n"
+      << "  __syncthreads();\n";
+    taps.clear();
+  };
   o << "  const uint32_t tid = threadIdx.x;\n";
   o << "  uint64_t tile = blockIdx.x;\n";
   o << "  if (tile >= ntiles) return;\n";
@@ -190,12 +213,13 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
     switch (op.code) {
       case TC_U1: {
         const uint64_t outside = op.lane_cmask & ~tile_mask, inside = op.lane_cmask & tile_mask;
+        const uint32_t form = op.fold == FOLD_DROP_RROT ? (uint32_t)TF_RROT : op.fold == FOLD_DROP_XROT ? (uint32_t)TF_XROT : op.b;
         if (inside == 0) {
           // controls outside the tile are the same for the whole workgroup: a scalar branch
           if (outside) o << "  if ((base & " << hex64(outside) << ") == " << hex64(outside) << ")";
           o << "  { const qr::dev::Coef4 u = " << coef(i) << ";";
           for (const auto& v : sets)
-            o << " qr::dev::u1_slot<R, " << RB << ", " << op.a << ", " << op.b << ", " << has_ns << ">(" << v
+            o << " qr::dev::u1_slot<R, " << RB << ", " << op.a << ", " << form << ", " << has_ns << ">(" << v
               << ", u, " << ns << ");";
           o << " }\n";
         } else if (op.b == TF_X) {  // controlled X: a per-lane exchange, no arithmetic
@@ -216,7 +240,7 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
         break;
       }
       case TC_D1: {
-        const bool only1 = op.flags & 1;
+        const bool only1 = (op.flags & 1) || op.fold == FOLD_DROP_D0;
         const int form = (int)(op.flags >> 4);
         const uint64_t outside = op.lane_cmask & ~tile_mask, inside = op.lane_cmask & tile_mask;
         if (op.b != 0xFFu && inside == 0) {
@@ -235,6 +259,7 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
               << has_ns << ">(" << v << ", d, " << ns << ");\n";
           o << "  }\n";
         } else {
+          // (per-lane factors: dropping d0 saves nothing here, its lanes multiply by 1)
           o << "  { const bool bit = (g0 >> " << op.a << ") & 1;\n"
             << "    double2 f = bit ? cf[" << 4 * i + 1 << "] : cf[" << 4 * i << "];\n";
           if (op.lane_cmask)
@@ -261,8 +286,12 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
         } else {
           o << "    acc = qr::dev::tap_diag<R, " << RB << ", -1>(l, r);\n";
         }
-        // the parameter's row comes from the op's coefficient slot, so that stages differing
-        // only in parameter numbering share one kernel
+        if (rows) {
+          o << "    qr::dev::tap_put(myrows, " << taps.size() << ", tid & 63u, acc); }\n";
+          taps.push_back(i);
+          if (taps.size() == kTapRows) flush_taps();
+          break;
+        }
         o << "    qr::dev::tap_store<" << TPB << ">(acc, part + (uint64_t)cf[" << 4 * i << "].x * nslots, tile, tid); }\n";
         break;
       }
@@ -390,6 +419,7 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
         break;
     }
   }
+  flush_taps();
   for (size_t v = 0; v < sets.size(); ++v)
     for (int m = 0; m < NR; ++m)
       o << "  " << store_amp(sets[v] + ".v[" + std::to_string(m) + "]", arrays[v], "g0", reg_off(mi, m)) << "\n";

@@ -795,6 +795,11 @@ std::vector<Stage> plan_fused(uint32_t n, const std::vector<FastOp>& ops, const 
             form = TF_NEGSWAP;
             t.fold = FOLD_M10;
           }
+          // gen 1 and 2: Rx and Ry (unitary, uncontrolled) in the adjoint sweep
+          if (dual && rot && t.ns == 0 && t.lane_cmask == 0 && (op.gen == 1 || op.gen == 2)) {
+            if (op.sub == SUB_RROT) t.fold = FOLD_DROP_RROT;
+            if (op.sub == SUB_XROT) t.fold = FOLD_DROP_XROT;
+          }
           t.b = (uint32_t)form;
           t.src = i;
           s.ops.push_back(t);
@@ -815,6 +820,8 @@ std::vector<Stage> plan_fused(uint32_t n, const std::vector<FastOp>& ops, const 
           } else if (!dual && t.ns == 0 && t.lane_cmask == 0 && op.sub == SUB_D0) {
             t.flags = 1;  // d0 factored out: diag(1, d1/d0)
             t.fold = FOLD_D0;
+          } else if (dual && t.ns == 0 && t.lane_cmask == 0 && op.sub == SUB_D0 && op.gen == 3) {
+            t.fold = FOLD_DROP_D0;  // Rz in the adjoint sweep
           }
           s.ops.push_back(t);
         } else if (op.kind == FK_GRAD) {
@@ -852,7 +859,7 @@ std::vector<Stage> plan_fused(uint32_t n, const std::vector<FastOp>& ops, const 
     // ---- folded scalars: one general-form uncontrolled op absorbs their product, else a
     // final scale applies it
     bool folded = false;
-    for (const auto& t : s.ops) folded = folded || (t.fold != FOLD_NONE);
+    for (const auto& t : s.ops) folded = folded || (t.fold != FOLD_NONE && t.fold < FOLD_DROP_D0);
     if (folded) {
       bool absorbed = false;
       for (auto& t : s.ops)
@@ -908,7 +915,11 @@ std::vector<Stage> plan_fused(uint32_t n, const std::vector<FastOp>& ops, const 
       std::vector<cd> c;
       stage_coefficients(s, ops, c);
       for (size_t i = 0; i < s.ops.size(); ++i)
-        for (int q = 0; q < 4; ++q) s.ops[i].coef[q] = c[4 * i + q];
+        for (int q = 0; q < 4; ++q) {
+          const TileOpHost& t = s.ops[i];
+          const bool plain = t.fold >= FOLD_DROP_D0;  // its factor is not part of the plan
+          s.ops[i].coef[q] = plain ? (q < (int)ops[t.src].m.size() ? ops[t.src].m[q] : cd(0, 0)) : c[4 * i + q];
+        }
     }
     stages.push_back(std::move(s));
     remaining = left;
@@ -963,11 +974,15 @@ void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, cd* c) {
       o[1] = m[1] / f;
       o[0] = cd(1, 0);
       total *= f;
-    } else if (t.fold == FOLD_RROT || t.fold == FOLD_XROT) {
+    } else if (t.fold == FOLD_DROP_D0) {
+      o[1] = m[1] / m[0];
+      o[0] = cd(1, 0);
+    } else if (t.fold == FOLD_RROT || t.fold == FOLD_XROT || t.fold == FOLD_DROP_RROT || t.fold == FOLD_DROP_XROT) {
       // [[a,-b],[b,a]] (RROT), or [[a,-ib],[-ib,a]] (XROT: the same rotation of (x, i y)),
       // = r * rotation(phi). phi is reduced to [-pi/2, pi/2] (a >= 0, the sign folded out),
       // then al = -tan(phi/2) = -b / (r + a) and be = sin(phi) = b / r, both in [-1, 1].
-      double a = m[0].real(), b = t.fold == FOLD_RROT ? m[2].real() : -m[1].imag();
+      const bool real = t.fold == FOLD_RROT || t.fold == FOLD_DROP_RROT;
+      double a = m[0].real(), b = real ? m[2].real() : -m[1].imag();
       double sgn = 1.0;
       if (a < 0) {
         a = -a;

@@ -259,28 +259,34 @@ __device__ __forceinline__ double rec(const C& l, const C& p) {
 // register slot J: (X p)_j = p_{j^J}; (Y p)_j = -i (-1)^{bit J of j} p_{j^J}.
 template <typename R, int RB, int J, int GEN>
 __device__ __forceinline__ double tap_pair(const Regs<R, RB>& l, const Regs<R, RB>& p) {
-  double acc = 0.0;
+  double acc[2] = {0.0, 0.0};  // two chains: one would wait for each multiply-add's result
 #pragma unroll
   for (int m0 = 0; m0 < (1 << RB); ++m0) {
     if (m0 & (1 << J)) continue;
     const int m1 = m0 | (1 << J);
-    if (GEN == 1) acc += imc(l.v[m0], p.v[m1]) + imc(l.v[m1], p.v[m0]);
-    else acc += rec(l.v[m1], p.v[m0]) - rec(l.v[m0], p.v[m1]);
+    if (GEN == 1) {
+      acc[0] += imc(l.v[m0], p.v[m1]);
+      acc[1] += imc(l.v[m1], p.v[m0]);
+    } else {
+      acc[0] += rec(l.v[m1], p.v[m0]);
+      acc[1] -= rec(l.v[m0], p.v[m1]);
+    }
   }
-  return acc;
+  return acc[0] + acc[1];
 }
 
 // sum_j s_j Im(conj(l_j) p_j) with s_j = (-1)^{bit J of j} (J >= 0) or 1 (J < 0).
 template <typename R, int RB, int J>
 __device__ __forceinline__ double tap_diag(const Regs<R, RB>& l, const Regs<R, RB>& p) {
-  double acc = 0.0;
+  double acc[2] = {0.0, 0.0};
 #pragma unroll
   for (int m = 0; m < (1 << RB); ++m) {
     const double v = imc(l.v[m], p.v[m]);
-    if (J >= 0 && (m & (1 << J))) acc -= v;
-    else acc += v;
+    const int c = (m >> 1) & 1;
+    if (J >= 0 && (m & (1 << J))) acc[c] -= v;
+    else acc[c] += v;
   }
-  return acc;
+  return acc[0] + acc[1];
 }
 
 // Sums `acc` over each group of min(TPB, 64) threads (one wavefront, or the whole workgroup
@@ -291,6 +297,43 @@ __device__ __forceinline__ void tap_store(double acc, double* row, unsigned long
 #pragma unroll
   for (int off = W / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, W);
   if ((tid & (W - 1)) == 0) row[tile * (unsigned long long)(TPB / W) + tid / W] = acc;
+}
+
+// Taps of workgroups of whole wavefronts: each lane's value is put into the wavefront's LDS rows
+// (a store nothing waits for) and kTapRows rows are summed together, four lanes to a row of 64:
+// 16 values from LDS in a fixed order, then across the four. One by one, a tap's six exchanges
+// between lanes take longer than its products where a wavefront has its SIMD to itself (20 qubits,
+// complex128, 400 parameters: 32 -> 21 us per sweep together with the folded rotations).
+// A row is 4 x 18 doubles: the lanes of an access then hit distinct banks. 14 rows: with the 32 KB
+// of both states' exchange, four workgroups still share a CU's LDS.
+constexpr int kTapRows = 14, kTapStride = 72;
+__device__ __forceinline__ void tap_put(double* rows, int row, unsigned int lane, double acc) {
+  rows[row * kTapStride + lane + 2 * (lane >> 4)] = acc;
+}
+// x + (x of lane ^ MASK), MASK 1 or 2 (inside groups of four lanes)
+template <int MASK>
+__device__ __forceinline__ double add_quad(double x) {
+  constexpr int perm = MASK == 1 ? 0xB1 : 0x4E;  // [1,0,3,2] or [2,3,0,1]
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), perm, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), perm, 0xF, 0xF, true);
+  return x + __hiloint2double(hi, lo);
+}
+// The sums of the wavefront's first `count` rows; lanes 4 q .. 4 q + 3 return row q's.
+__device__ __forceinline__ double tap_sum(const double* rows, int count, unsigned int lane) {
+  const unsigned int q = lane >> 2;
+  double s = 0.0;
+  if ((int)q < count) {
+    const double2* src = reinterpret_cast<const double2*>(rows + q * kTapStride + 18 * (lane & 3));
+    double a = 0.0, b = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const double2 v = src[i];
+      a += v.x;
+      b += v.y;
+    }
+    s = a + b;
+  }
+  return add_quad<2>(add_quad<1>(s));
 }
 
 // Amplitude loads and stores marked non-temporal (streamed once per sweep, not kept in cache),

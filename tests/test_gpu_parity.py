@@ -797,3 +797,23 @@ def test_expectation_arrangements(precision, n):
         want = H.oracle_expectation(n, psi, obs)
         assert abs(got - want) < 16 * n * 2.0 ** -52 * sum(abs(c) for c, _ in obs.terms)
     st.close()
+
+
+@pytest.mark.parametrize("precision,tol", [(_capi.QR_C128, 1e-11), (_capi.QR_C64, 2e-5)])
+@pytest.mark.parametrize("tile_bits", [6, 10, 11, 12, 13])
+def test_adjoint_tap_rows(tile_bits, precision, tol):
+    """Gradient taps summed through LDS rows (workgroups of one to eight wavefronts, stages with
+    more taps than rows) and singly (smaller workgroups), with angles beyond the shears' range and
+    Phase gates between, against the per-op reverse sweep."""
+    n = 13
+    gates, _ = W.hea(n, 4, seed=31, angle_lo=-9.0, angle_hi=9.0)
+    gates = gates[:40] + [("Phase", 3, (), 0.8, 0), ("Rx", 5, (), -2.9, 0), ("H", 2, (), 0.0, 0)] + gates[40:]
+    p, obs = W.to_program(gates), _capi.Observable(W.hea_observable(n))
+    got = []
+    for fused in (1, 0):
+        g = _capi.Grad(n, precision)
+        g.set_options(fused=fused, tile_bits=tile_bits)
+        g.forward(p, obs)
+        got.append(g.backward())
+        g.close()
+    assert np.max(np.abs(got[0] - got[1])) < tol * n
