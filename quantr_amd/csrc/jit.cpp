@@ -152,11 +152,16 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
   if (!dual) o << "  psi += (uint64_t)blockIdx.y * inst_stride;\n  cf += (uint64_t)blockIdx.y * cf_stride;\n";
   o << "  using R = " << R << ";\n";
   o << "  __shared__ " << C << " lds[" << (split ? (1 << (K - 1)) : (lds2 ? 2 : 1) * (1 << K)) << "];\n";
-  // gradient taps go through LDS rows of their wavefront, summed together (tile_ops.hpp)
+  // gradient taps go through LDS rows of their wavefront, summed together (tile_ops.hpp), unless
+  // the rows (8 KB a wavefront) would leave a CU with one workgroup in place of two
   std::vector<size_t> taps;  // ops whose rows are waiting
   bool rows = false;
-  if (dual && TPB >= 64)
-    for (const TileOpHost& op : s.ops) rows = rows || op.code == TC_GRAD;
+  if (dual && TPB >= 64) {
+    const size_t exchange = (size_t)(lds2 ? 2 : 1) * (1ull << K) * amp_bytes, cu = 160 * 1024;
+    const size_t with_rows = exchange + (size_t)(TPB / 64) * kTapRows * 72 * sizeof(double);
+    if (cu / with_rows >= std::min<size_t>(2, cu / exchange))
+      for (const TileOpHost& op : s.ops) rows = rows || op.code == TC_GRAD;
+  }
   if (rows)
     o << "  __shared__ __align__(16) double taprows[" << TPB / 64 << " * qr::dev::kTapRows * qr::dev::kTapStride];\n"
       << "  double* const myrows = taprows + (threadIdx.x >> 6) * (qr::dev::kTapRows * qr::dev::kTapStride);\n";
