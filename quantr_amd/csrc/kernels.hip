@@ -237,12 +237,17 @@ __global__ void k_densek(typename CT<R>::T* __restrict__ psi, typename CT<R>::T*
 
 // Dense 2^K x 2^K on K <= 4 target bits (+ controls) with the group in registers: one thread
 // per group of 2^K amplitudes, which it reads once, transforms and writes back in place.
-// off[j] is the offset of local basis state j (MSB-first local index).
+// off[j] is the offset of local basis state j (MSB-first local index). Instance blockIdx.y has its
+// state and its table at fixed strides: 500 states of 2^12 amplitudes with a table each take one
+// launch (1.2 ms of launches before).
 template <typename R, int K>
 __global__ __launch_bounds__(256) void k_densek_reg(typename CT<R>::T* __restrict__ psi, uint64_t ngroups, DenseKArgs a,
-                                                    const double2* __restrict__ M, const uint64_t* __restrict__ off) {
+                                                    const double2* __restrict__ M, const uint64_t* __restrict__ off,
+                                                    Instances in) {
   using C = typename CT<R>::T;
   constexpr int D = 1 << K;
+  psi += (uint64_t)blockIdx.y * in.state_stride;
+  M += (uint64_t)blockIdx.y * in.table_stride;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < ngroups; g += stride) {
     const uint64_t base = insert_zero_bits(g, a.sorted_bits, K);
@@ -269,8 +274,10 @@ __global__ __launch_bounds__(256) void k_densek_reg(typename CT<R>::T* __restric
 // 2^k diagonal phases over k bits (+ controls).
 template <typename R>
 __global__ void k_diagk(typename CT<R>::T* __restrict__ psi, uint64_t dim, DiagKArgs a,
-                        const double2* __restrict__ D) {
+                        const double2* __restrict__ D, Instances in) {
   using C = typename CT<R>::T;
+  psi += (uint64_t)blockIdx.y * in.state_stride;
+  D += (uint64_t)blockIdx.y * in.table_stride;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += stride) {
     if ((i & a.cmask) != a.cmask) continue;
@@ -644,6 +651,10 @@ __global__ __launch_bounds__(256) void k_init_instances(typename CT<R>::T* __res
 // One workgroup per state (states back to back, `stride` amplitudes apart): its draws
 // u[off[y] .. off[y+1]) (ascending) placed by the left fold of its probabilities in index
 // order, as k_sample_fold does for one state: probabilities in parallel, the fold in one lane.
+// The fold is a chain of additions: sixteen values at a time come from LDS while the sixteen
+// before are added, and draws are looked at once for each sixteen (the fold does not decrease, so
+// a draw below its end, or an unordered one, is found inside): 500 states of 2^12 amplitudes
+// took 690 us with an LDS read and a comparison in every step of the chain.
 template <typename R>
 __global__ __launch_bounds__(256) void k_sample_fold_instances(const typename CT<R>::T* __restrict__ psi,
                                                                uint64_t dim, uint64_t stride,
@@ -651,14 +662,15 @@ __global__ __launch_bounds__(256) void k_sample_fold_instances(const typename CT
                                                                const uint64_t* __restrict__ off,
                                                                uint64_t* __restrict__ out) {
 #pragma clang fp contract(off)
-  constexpr int CH = 2048;
-  __shared__ double p[CH];
+  constexpr int CH = 2048, ST = 16;
+  __shared__ double p[CH + ST];  // zeros behind the chunk: the last values fetched ahead
   __shared__ int done;
   const typename CT<R>::T* ps = psi + (uint64_t)blockIdx.x * stride;
   const uint64_t d1 = off[blockIdx.x + 1];
   uint64_t d = off[blockIdx.x];
-  double cum = 0.0;
+  double cum = 0.0, ud = d < d1 ? u[d] : 0.0;
   if (threadIdx.x == 0) done = (d >= d1);
+  if (threadIdx.x < ST) p[CH + threadIdx.x] = 0.0;
   __syncthreads();
   for (uint64_t base = 0; base < dim && !done; base += CH) {
     for (int q = threadIdx.x; q < CH; q += blockDim.x) {
@@ -672,10 +684,30 @@ __global__ __launch_bounds__(256) void k_sample_fold_instances(const typename CT
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      const uint64_t cnt = (dim - base < (uint64_t)CH) ? (dim - base) : (uint64_t)CH;
-      for (uint64_t q = 0; q < cnt; ++q) {
-        cum = cum + p[q];
-        while (d < d1 && u[d] < cum) out[d++] = base + q;
+      const int cnt = (int)((dim - base < (uint64_t)CH) ? (dim - base) : (uint64_t)CH);
+      double next[ST];
+#pragma unroll
+      for (int j = 0; j < ST; ++j) next[j] = p[j];
+      for (int q = 0; q < cnt && d < d1; q += ST) {
+        double s[ST];
+#pragma unroll
+        for (int j = 0; j < ST; ++j) s[j] = next[j];
+#pragma unroll
+        for (int j = 0; j < ST; ++j) next[j] = p[q + ST + j];
+        // values at and beyond dim are +0 and leave the fold where it is
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+          cum = cum + s[j];
+          s[j] = cum;
+        }
+        if (!(ud >= cum)) {
+#pragma unroll
+          for (int j = 0; j < ST; ++j)
+            while (d < d1 && ud < s[j]) {
+              out[d++] = base + q + j;
+              ud = d < d1 ? u[d] : 0.0;
+            }
+        }
       }
       done = (d >= d1);
     }
@@ -1185,14 +1217,15 @@ hipError_t launch_diag1(int prec, void* psi, uint64_t dim, int t, uint64_t cmask
 }
 
 hipError_t launch_densek_reg(int prec, void* psi, uint64_t ngroups, const DenseKArgs& a, const double2* M,
-                             const uint64_t* off, hipStream_t s) {
-  const unsigned g = grid_for(ngroups, 256, 1u << 18);
+                             const uint64_t* off, hipStream_t s, const Instances& in) {
+  if (in.count == 0 || in.count > 65535u) return hipErrorInvalidValue;
+  const dim3 g(grid_for(ngroups, 256, 1u << 18), in.count);
 #define QR_DENSEK_CASE(KK)                                                                     \
   case KK:                                                                                     \
     if (prec == 0)                                                                             \
-      dev::k_densek_reg<double, KK><<<g, 256, 0, s>>>((double2*)psi, ngroups, a, M, off);      \
+      dev::k_densek_reg<double, KK><<<g, 256, 0, s>>>((double2*)psi, ngroups, a, M, off, in);  \
     else                                                                                       \
-      dev::k_densek_reg<float, KK><<<g, 256, 0, s>>>((float2*)psi, ngroups, a, M, off);        \
+      dev::k_densek_reg<float, KK><<<g, 256, 0, s>>>((float2*)psi, ngroups, a, M, off, in);    \
     break;
   switch (a.k) {
     QR_DENSEK_CASE(2)
@@ -1217,12 +1250,13 @@ hipError_t launch_densek(int prec, void* psi, void* tmp, uint64_t tmp_groups, ui
 }
 
 hipError_t launch_diagk(int prec, void* psi, uint64_t dim, const DiagKArgs& a, const double2* D,
-                        hipStream_t s) {
-  const unsigned g = grid_for(dim, 256, 1u << 18);
+                        hipStream_t s, const Instances& in) {
+  if (in.count == 0 || in.count > 65535u) return hipErrorInvalidValue;
+  const dim3 g(grid_for(dim, 256, 1u << 18), in.count);
   if (prec == 0)
-    dev::k_diagk<double><<<g, 256, 0, s>>>((double2*)psi, dim, a, D);
+    dev::k_diagk<double><<<g, 256, 0, s>>>((double2*)psi, dim, a, D, in);
   else
-    dev::k_diagk<float><<<g, 256, 0, s>>>((float2*)psi, dim, a, D);
+    dev::k_diagk<float><<<g, 256, 0, s>>>((float2*)psi, dim, a, D, in);
   return hipGetLastError();
 }
 

@@ -28,6 +28,13 @@ struct DenseKArgs {
   uint64_t cmask;
 };
 
+// Several states of one shape in a launch: instance y's state is y * state_stride amplitudes and its
+// table y * table_stride double2 behind the first one's (at most 65535).
+struct Instances {
+  uint32_t count = 1;
+  uint64_t state_stride = 0, table_stride = 0;
+};
+
 struct DiagKArgs {
   int k;
   uint8_t bits[20];  // local MSB first
@@ -95,9 +102,9 @@ hipError_t launch_densek(int prec, void* psi, void* tmp, uint64_t tmp_groups, ui
                          const DenseKArgs& a, const double2* M, const uint64_t* off, hipStream_t s);
 // Dense 2^k x 2^k, 2 <= k <= 4, each group of amplitudes in registers (no staging).
 hipError_t launch_densek_reg(int prec, void* psi, uint64_t ngroups, const DenseKArgs& a, const double2* M,
-                             const uint64_t* off, hipStream_t s);
+                             const uint64_t* off, hipStream_t s, const Instances& in = Instances());
 hipError_t launch_diagk(int prec, void* psi, uint64_t dim, const DiagKArgs& a, const double2* D,
-                        hipStream_t s);
+                        hipStream_t s, const Instances& in = Instances());
 hipError_t launch_tile(int prec, int K, int RB, bool prefetch, void* psi, const TileArgs& a, hipStream_t s);
 hipError_t launch_sample_fold(int prec, const void* psi, uint64_t dim, const double* u, uint64_t shots,
                               uint64_t* out, hipStream_t s);

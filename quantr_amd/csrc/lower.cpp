@@ -484,7 +484,7 @@ void classify(FastOp& f) {
     return;
   }
   if (f.kind != FK_DENSE1) return;
-  const std::vector<cd>& A = f.m;
+  const OpCoefs& A = f.m;
   if (is_zero(A[0]) && is_zero(A[3])) {
     f.form = U1_PERM;
     if (A[1] == A[2]) f.sub = SUB_XLIKE;

@@ -953,7 +953,7 @@ void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, cd* c) {
       if (t.fold == FOLD_SCALE) scaler = (int)i;
       continue;
     }
-    const std::vector<cd>& m = ops[t.src].m;
+    const OpCoefs& m = ops[t.src].m;
     for (size_t q = 0; q < 4 && q < m.size(); ++q) o[q] = m[q];
     cd f(1, 0);
     switch (t.fold) {

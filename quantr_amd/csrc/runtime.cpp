@@ -41,7 +41,7 @@ void pinned_give_back(void* p, size_t cap) {
     std::lock_guard<std::mutex> lk(g_pin_mu);
     size_t held = cap;
     for (const PinnedBlock& b : g_pinned) held += b.cap;
-    if (g_pin_states > 0 && g_pinned.size() < kPinnedKeep && held <= kPinnedBytes) {
+    if (g_pinned.size() < kPinnedKeep && held <= kPinnedBytes) {
       g_pinned.push_back({p, cap});
       drop = nullptr;
     }
@@ -93,6 +93,77 @@ PinnedLease::~PinnedLease() {
   if (std::uncaught_exceptions()) (void)hipHostFree(p_);
   else pinned_give_back(p_, cap_);
 }
+
+// ---- device memory kept between calls -----------------------------------------------------
+namespace {
+constexpr size_t kDeviceKeep = 8, kDeviceBytes = 256ull << 20;
+struct DeviceBlock {
+  void* p;
+  size_t cap;
+  int device;
+};
+std::mutex g_dev_mu;
+std::vector<DeviceBlock> g_device_blocks;  // kept blocks, none in use
+}  // namespace
+
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory && e != hipErrorMemoryAllocation) return e;
+  std::vector<DeviceBlock> drop;
+  {
+    std::lock_guard<std::mutex> lk(g_dev_mu);
+    drop.swap(g_device_blocks);
+  }
+  if (drop.empty()) return e;
+  (void)hipGetLastError();
+  for (const DeviceBlock& b : drop) (void)hipFree(b.p);
+  return hipMalloc(p, bytes);
+}
+
+void DeviceLease::reserve(size_t bytes) {
+  if (bytes <= cap_) return;
+  release();
+  hip_check(hipGetDevice(&device_), "hipGetDevice");
+  {
+    std::lock_guard<std::mutex> lk(g_dev_mu);
+    size_t best = g_device_blocks.size();
+    for (size_t i = 0; i < g_device_blocks.size(); ++i) {
+      const DeviceBlock& b = g_device_blocks[i];
+      if (b.device == device_ && b.cap >= bytes && (best == g_device_blocks.size() || b.cap < g_device_blocks[best].cap))
+        best = i;
+    }
+    if (best < g_device_blocks.size()) {
+      p = g_device_blocks[best].p;
+      cap_ = g_device_blocks[best].cap;
+      g_device_blocks.erase(g_device_blocks.begin() + best);
+      return;
+    }
+  }
+  size_t want = 1 << 16;
+  while (want < bytes && want < kDeviceBytes) want *= 2;
+  want = std::max(want, bytes);
+  hip_check(device_malloc(&p, want), "hipMalloc (workspace)");
+  cap_ = want;
+}
+
+void DeviceLease::release() {
+  if (!p) return;
+  void* drop = p;
+  if (!std::uncaught_exceptions()) {  // after an error, hipFree waits for what may still run
+    std::lock_guard<std::mutex> lk(g_dev_mu);
+    size_t held = cap_;
+    for (const DeviceBlock& b : g_device_blocks) held += b.cap;
+    if (g_device_blocks.size() < kDeviceKeep && held <= kDeviceBytes) {
+      g_device_blocks.push_back({p, cap_, device_});
+      drop = nullptr;
+    }
+  }
+  if (drop) (void)hipFree(drop);
+  p = nullptr;
+  cap_ = 0;
+}
+
+DeviceLease::~DeviceLease() { release(); }
 
 Uploader::~Uploader() {
   for (hipEvent_t e : ev_)
@@ -274,6 +345,33 @@ TileArgs tile_args(const qr_state* st, const PackedPlan& P, size_t si) {
   return tile_args_at(st->n, (*P.stages)[si], P.dblob, (*P.loc)[si]);
 }
 
+static DenseKArgs densek_args(const FastOp& op) {
+  DenseKArgs a{};
+  a.k = op.k;
+  a.cmask = op.cmask;
+  std::vector<int> sb(op.bits, op.bits + op.k);
+  std::sort(sb.begin(), sb.end());
+  for (int q = 0; q < op.k; ++q) a.sorted_bits[q] = (uint8_t)sb[q];
+  return a;
+}
+
+bool launch_standalone_instances(int prec, uint64_t dim, void* amp, const FastOp& op, const uint8_t* dblob,
+                                 const Loc& l, hipStream_t s, const Instances& in) {
+  if (op.kind == FK_DENSEK && op.k >= 2 && op.k <= 4) {  // the group fits in registers
+    hip_check(launch_densek_reg(prec, amp, dim >> op.k, densek_args(op), (const double2*)(dblob + l.coefs),
+                                (const uint64_t*)(dblob + l.off), s, in),
+              "densek");
+    return true;
+  }
+  if (op.kind != FK_DIAGK) return false;
+  DiagKArgs a{};
+  a.k = op.k;
+  a.cmask = op.cmask;
+  for (int q = 0; q < op.k; ++q) a.bits[q] = (uint8_t)op.bits[q];
+  hip_check(launch_diagk(prec, amp, dim, a, (const double2*)(dblob + l.coefs), s, in), "diagk");
+  return true;
+}
+
 void launch_standalone_raw(int prec, uint64_t dim, void* amp, DevBuf& tmp, const FastOp& op, const uint8_t* dblob,
                            const Loc& l, hipStream_t s) {
   switch (op.kind) {
@@ -289,20 +387,10 @@ void launch_standalone_raw(int prec, uint64_t dim, void* amp, DevBuf& tmp, const
                 "diag1");
       break;
     case FK_DENSEK: {
-      DenseKArgs a{};
-      a.k = op.k;
-      a.cmask = op.cmask;
-      std::vector<int> sb(op.bits, op.bits + op.k);
-      std::sort(sb.begin(), sb.end());
-      for (int q = 0; q < op.k; ++q) a.sorted_bits[q] = (uint8_t)sb[q];
+      if (launch_standalone_instances(prec, dim, amp, op, dblob, l, s, Instances())) break;
+      const DenseKArgs a = densek_args(op);
       const uint64_t dimk = 1ull << op.k;
       const uint64_t ngroups = dim >> op.k;
-      if (op.k >= 2 && op.k <= 4) {  // the group fits in registers
-        hip_check(launch_densek_reg(prec, amp, ngroups, a, (const double2*)(dblob + l.coefs),
-                                    (const uint64_t*)(dblob + l.off), s),
-                  "densek");
-        break;
-      }
       uint64_t tg = std::min<uint64_t>(ngroups, std::max<uint64_t>(256, (64ull << 20) / (dimk * 16)));
       tg = std::max<uint64_t>(tg / 256, 1) * 256;
       if (ngroups < 256) tg = ngroups;
@@ -312,14 +400,9 @@ void launch_standalone_raw(int prec, uint64_t dim, void* amp, DevBuf& tmp, const
                 "densek");
       break;
     }
-    case FK_DIAGK: {
-      DiagKArgs a{};
-      a.k = op.k;
-      a.cmask = op.cmask;
-      for (int q = 0; q < op.k; ++q) a.bits[q] = (uint8_t)op.bits[q];
-      hip_check(launch_diagk(prec, amp, dim, a, (const double2*)(dblob + l.coefs), s), "diagk");
+    case FK_DIAGK:
+      (void)launch_standalone_instances(prec, dim, amp, op, dblob, l, s, Instances());
       break;
-    }
     default:
       throw Error{QR_ERR_UNSUPPORTED, "internal error: op kind has no standalone kernel"};
   }
@@ -681,7 +764,7 @@ qr_state* new_state(uint32_t n, qr_precision p) {
   hip_check(hipGetDevice(&st->device), "hipGetDevice");
   hip_check(hipStreamCreateWithFlags(&st->stream, hipStreamNonBlocking), "hipStreamCreate");
   const size_t bytes = st->dim * st->bytes_per_amp();
-  hipError_t e = hipMalloc(&st->amp, bytes);
+  hipError_t e = device_malloc(&st->amp, bytes);
   if (e != hipSuccess) {
     st->amp = nullptr;
     (void)hipGetLastError();

@@ -26,6 +26,28 @@ inline void hip_check(hipError_t e, const char* what) {
   throw Error{QR_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e)};
 }
 
+// Device memory with what the library keeps for later calls given back before it fails.
+hipError_t device_malloc(void** p, size_t bytes);
+
+// A block of device memory held for one call without a state of its own. Blocks are kept for later
+// calls (allocating and freeing them took longer than the call's kernels): at most 8 of them and
+// 256 MB; larger ones are not kept, and all are given back when an allocation would fail. The
+// holder's work on the block is done before it lets go.
+class DeviceLease {
+ public:
+  DeviceLease() = default;
+  ~DeviceLease();
+  DeviceLease(const DeviceLease&) = delete;
+  DeviceLease& operator=(const DeviceLease&) = delete;
+  void reserve(size_t bytes);  // at least this size; what it held is lost
+  void* p = nullptr;
+
+ private:
+  void release();
+  size_t cap_ = 0;
+  int device_ = 0;
+};
+
 // Device buffer that grows on demand.
 struct DevBuf {
   void* p = nullptr;
@@ -36,7 +58,7 @@ struct DevBuf {
     p = nullptr;
     cap = 0;
     size_t want = std::max<size_t>(bytes, 1 << 16);
-    hip_check(hipMalloc(&p, want), "hipMalloc (workspace)");
+    hip_check(device_malloc(&p, want), "hipMalloc (workspace)");
     cap = want;
   }
   ~DevBuf() {
@@ -46,7 +68,7 @@ struct DevBuf {
 
 // A block of pinned host memory, which kernels and copies reach directly, held for one call.
 // Blocks are kept for later calls (pinning a new one takes longer than a small call): at most
-// 8 of them and 64 MB, none once no state is left.
+// 8 of them and 64 MB, given back when the last state is destroyed.
 class PinnedLease {
  public:
   PinnedLease() = default;
@@ -232,6 +254,10 @@ TileArgs tile_args_at(uint32_t n, const Stage& s, const uint8_t* dblob, const Lo
 // One standalone op on a state of 2^n amplitudes (tmp: staging for wide dense gates).
 void launch_standalone_raw(int prec, uint64_t dim, void* amp, DevBuf& tmp, const FastOp& op, const uint8_t* dblob,
                            const Loc& loc, hipStream_t s);
+// The same op with each instance's own table on several states in one launch; false if its kernel
+// takes one state at a time.
+bool launch_standalone_instances(int prec, uint64_t dim, void* amp, const FastOp& op, const uint8_t* dblob,
+                                 const Loc& loc, hipStream_t s, const Instances& in);
 
 // ---- execution ------------------------------------------------------------------------------
 qr_state* new_state(uint32_t n, qr_precision p);

@@ -87,7 +87,9 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
     hipStream_t s;
     ~StreamGuard() { (void)hipStreamDestroy(s); }
   } guard{s};
-  DevBuf states, blobs, tmp, dev_u, dev_off, dev_out;
+  DeviceLease states, blobs, draws_dev;
+  PinnedLease host, small;
+  DevBuf tmp;
   for (const auto& key : order) {
     const std::vector<uint64_t>& members = groups[key];
     std::shared_ptr<CachedPlan> cp = get_plan_for(n, prec, pr[members[0]].ops, pp, true, false, false);
@@ -101,13 +103,13 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
     for (size_t c0 = 0; c0 < members.size(); c0 += per_chunk) {
       const uint64_t cnt = std::min<uint64_t>(per_chunk, members.size() - c0);
       // coefficient blobs of the chunk's programs, back to back (same layout: same plan)
-      std::vector<uint8_t> host(cnt * blob_stride, 0);
+      host.reserve(std::max<size_t>(cnt * blob_stride, 1));
       parallel_for(cnt, [&](uint64_t y) {
         std::memcpy(host.data() + y * blob_stride, cp->image.bytes.data(), blob_size);
         write_values(pr[members[c0 + y]].ops, stages, loc, host.data() + y * blob_stride);
       });
-      blobs.reserve(host.size());
-      hip_check(hipMemcpyAsync(blobs.p, host.data(), host.size(), hipMemcpyHostToDevice, s), "H2D");
+      blobs.reserve(std::max<size_t>(cnt * blob_stride, 1));
+      hip_check(hipMemcpyAsync(blobs.p, host.data(), cnt * blob_stride, hipMemcpyHostToDevice, s), "H2D");
       states.reserve(cnt * dim * B);
       hip_check(launch_init_instances(prec, states.p, dim, cnt, s), "init states");
       const uint8_t* db = (const uint8_t*)blobs.p;
@@ -119,7 +121,9 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
           hip_check(jit_launch(cp->fns[si], st.k, pp.reg_bits, false, states.p, a.coefs, a.ntiles, a.nontile_mask, s,
                                ord, (uint32_t)cnt, dim, blob_stride / sizeof(double2)),
                     "compiled tile kernel (programs)");
-        } else {
+        } else if (!launch_standalone_instances(
+                       prec, dim, states.p, pr[members[c0]].ops[st.standalone], db, loc[si], s,
+                       Instances{(uint32_t)cnt, dim, blob_stride / sizeof(double2)})) {
           for (uint64_t y = 0; y < cnt; ++y)
             launch_standalone_raw(prec, dim, (uint8_t*)states.p + y * dim * B, tmp,
                                   pr[members[c0 + y]].ops[st.standalone], db + y * blob_stride, loc[si], s);
@@ -140,20 +144,19 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
         off[y + 1] = uu.size();
       }
       if (!uu.empty()) {
-        dev_u.reserve(uu.size() * sizeof(double));
-        dev_off.reserve(off.size() * sizeof(uint64_t));
-        dev_out.reserve(uu.size() * sizeof(uint64_t));
-        hip_check(hipMemcpyAsync(dev_u.p, uu.data(), uu.size() * sizeof(double), hipMemcpyHostToDevice, s), "H2D");
-        hip_check(hipMemcpyAsync(dev_off.p, off.data(), off.size() * sizeof(uint64_t), hipMemcpyHostToDevice, s),
-                  "H2D");
-        hip_check(launch_sample_fold_instances(prec, states.p, dim, cnt, (const double*)dev_u.p,
-                                               (const uint64_t*)dev_off.p, (uint64_t*)dev_out.p, s),
+        // draws and offsets go up in one copy; the bins are written to pinned memory
+        const size_t ub = uu.size() * sizeof(double), ob = off.size() * sizeof(uint64_t);
+        small.reserve(2 * ub + ob);
+        std::memcpy(small.data(), uu.data(), ub);
+        std::memcpy(small.data() + ub, off.data(), ob);
+        const uint64_t* got = (const uint64_t*)(small.data() + ub + ob);
+        draws_dev.reserve(ub + ob);
+        hip_check(hipMemcpyAsync(draws_dev.p, small.data(), ub + ob, hipMemcpyHostToDevice, s), "H2D");
+        hip_check(launch_sample_fold_instances(prec, states.p, dim, cnt, (const double*)draws_dev.p,
+                                               (const uint64_t*)((const uint8_t*)draws_dev.p + ub), (uint64_t*)got, s),
                   "sample fold (programs)");
-        std::vector<uint64_t> got(uu.size());
-        hip_check(hipMemcpyAsync(got.data(), dev_out.p, got.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, s),
-                  "D2H");
         hip_check(hipStreamSynchronize(s), "sync");
-        for (size_t q = 0; q < got.size(); ++q) out[perm[q]] = got[q];
+        for (size_t q = 0; q < uu.size(); ++q) out[perm[q]] = got[q];
       } else {
         hip_check(hipStreamSynchronize(s), "sync");
       }
