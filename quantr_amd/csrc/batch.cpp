@@ -30,7 +30,8 @@ using namespace qr;
 
 namespace {
 
-constexpr int kDotBlocks = 64;
+// Instances of fewer qubits than this start from |0...0> in one launch for all of them.
+constexpr uint32_t kInitTogether = 18;
 constexpr size_t kAlign = 256;
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -45,7 +46,7 @@ struct Inst {
   std::shared_ptr<CachedPlan> pf, pb;
   size_t blob_f = 0, blob_b = 0;  // offsets of the two plan blobs in the batch blob
   size_t obs_groups = 0, obs_terms = 0;  // byte offsets of the observable's tables in the blob
-  int ngroups = 0;
+  int ngroups = 0, nplain = 0;
   uint64_t nparams = 0, nslots = 0;
   std::vector<int> gens;      // generator of each parameter (4 = global phase)
   size_t psi = 0, lam = 0;    // byte offsets in the state pool
@@ -159,7 +160,7 @@ void launch_instance(qr_batch* b, const Inst& I, hipStream_t s, uint64_t* stamps
   const uint8_t* dblob = (const uint8_t*)b->blob.p;
   double* work = (double*)b->work.p;
   double* outd = (double*)b->out.p;
-  hip_check(launch_init_basis(prec, psi, I.dim, 0, s), "init");
+  if (I.n >= kInitTogether) hip_check(launch_init_basis(prec, psi, I.dim, 0, s), "init");
   // forward
   for (size_t si = 0; si < I.pf->stages.size(); ++si) {
     const Stage& st = I.pf->stages[si];
@@ -171,12 +172,10 @@ void launch_instance(qr_batch* b, const Inst& I, hipStream_t s, uint64_t* stamps
       launch_standalone_raw(prec, I.dim, psi, b->tmp[I.stream], I.fwd[st.standalone], dblob + I.blob_f, I.pf->image.loc[si], s);
     }
   }
-  // lam = O psi (one pass), E = Re <psi|lam>
-  hip_check(launch_pauli_sum(prec, lam, psi, I.dim, (const PauliGroup*)(dblob + I.obs_groups), I.ngroups,
-                             (const PauliZTerm*)(dblob + I.obs_terms), s),
+  // lam = O psi and the partial sums of E = Re <psi|lam> in one pass
+  hip_check(launch_pauli_sum(prec, lam, psi, I.dim, (const PauliGroup*)(dblob + I.obs_groups), I.ngroups, I.nplain,
+                             (const PauliZTerm*)(dblob + I.obs_terms), s, work + I.dot),
             "pauli sum");
-  hip_check(launch_dot_re_partial(prec, psi, lam, I.dim, work + I.dot, kDotBlocks, s), "dot");
-  hip_check(launch_sum_rows(work + I.dot, kDotBlocks, 1, outd + idx, s), "expectation sum");
   // reverse sweep
   for (size_t si = 0; si < I.pb->stages.size(); ++si) {
     const Stage& st = I.pb->stages[si];
@@ -192,9 +191,9 @@ void launch_instance(qr_batch* b, const Inst& I, hipStream_t s, uint64_t* stamps
     }
   }
   const size_t m = b->inst.size();
-  if (I.nparams)
-    hip_check(launch_sum_rows(work + I.part, I.nslots, (uint32_t)I.nparams, outd + m + I.grad, s), "gradient sums");
-  hip_check(launch_stamp(stamps + 1 + idx, s), "stamp");
+  hip_check(launch_finish_instance(work + I.part, I.nslots, (uint32_t)I.nparams, outd + m + I.grad, work + I.dot,
+                                   pauli_sum_partials(I.dim), outd + idx, stamps + 1 + idx, s),
+            "gradient sums");
 }
 
 
@@ -296,6 +295,7 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
       std::vector<PauliGroup> groups;
       std::vector<PauliZTerm> flat;
       pauli_tables(I.terms, groups, flat);
+      I.nplain = pauli_plain_first(groups, flat);
       I.ngroups = (int)groups.size();
       I.obs_groups = blob_size = align_up(blob_size, 16);
       blob_size += groups.size() * sizeof(PauliGroup);
@@ -309,10 +309,20 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
     I.part = work_doubles;
     work_doubles += std::max<uint64_t>(I.nparams, 1) * I.nslots;
     I.dot = work_doubles;
-    work_doubles += kDotBlocks;
+    work_doubles += pauli_sum_partials(I.dim);
     I.grad = b->total_params;
     b->total_params += I.nparams;
   }
+  // the states that start together: pool offsets, then qubit counts
+  std::vector<uint64_t> init_base;
+  std::vector<uint32_t> init_bits;
+  for (const Inst& I : b->inst)
+    if (I.n < kInitTogether) {
+      init_base.push_back(I.psi);
+      init_bits.push_back(I.n);
+    }
+  const size_t init_at = blob_size = align_up(blob_size, kAlign);
+  blob_size += init_base.size() * (sizeof(uint64_t) + sizeof(uint32_t));
   b->host_blob.reserve(std::max<size_t>(blob_size, 1));
   b->host_blob_size = blob_size;
   for (Inst& I : b->inst) {  // standalone and observable tables (fixed for the batch's lifetime)
@@ -321,11 +331,17 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
     std::vector<PauliGroup> groups;
     std::vector<PauliZTerm> flat;
     pauli_tables(I.terms, groups, flat);
+    (void)pauli_plain_first(groups, flat);
     if (!groups.empty())
       std::memcpy(b->host_blob.data() + I.obs_groups, groups.data(), groups.size() * sizeof(PauliGroup));
     if (!flat.empty()) std::memcpy(b->host_blob.data() + I.obs_terms, flat.data(), flat.size() * sizeof(PauliZTerm));
   }
   for (const Inst& I : b->inst) fill_blob(b.get(), I);
+  if (!init_base.empty()) {
+    std::memcpy(b->host_blob.data() + init_at, init_base.data(), init_base.size() * sizeof(uint64_t));
+    std::memcpy(b->host_blob.data() + init_at + init_base.size() * sizeof(uint64_t), init_bits.data(),
+                init_bits.size() * sizeof(uint32_t));
+  }
   const size_t out_doubles = m + b->total_params;
   b->states.reserve(std::max<size_t>(state_bytes, 1));
   b->blob.reserve(std::max<size_t>(blob_size, 1));
@@ -334,6 +350,9 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
   // ---- streams: largest instances first, each to the least loaded stream ---------------------
   const int S = (int)std::min<uint64_t>((uint64_t)nstreams, m);
   hip_check(hipStreamCreateWithFlags(&b->origin, hipStreamNonBlocking), "hipStreamCreate");
+  // the instances' stamps only rise: they start at zero (before the capture, ordered on its stream)
+  hip_check(hipMemsetAsync(b->out.p, 0, out_doubles * sizeof(double) + (m + 1) * sizeof(uint64_t) + kAlign, b->origin),
+            "hipMemsetAsync");
   b->streams.resize(S);
   b->tmp.resize(S);
   for (int s = 0; s < S; ++s) hip_check(hipStreamCreateWithFlags(&b->streams[s], hipStreamNonBlocking), "hipStreamCreate");
@@ -369,6 +388,12 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
   hip_check(hipStreamBeginCapture(b->origin, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
   try {
     hip_check(launch_stamp(stamps, b->origin), "stamp");
+    for (size_t i0 = 0; i0 < init_base.size(); i0 += 65535) {
+      const uint64_t* base = (const uint64_t*)((const uint8_t*)b->blob.p + init_at);
+      hip_check(launch_init_batch(b->prec, b->states.p, base + i0, (const uint32_t*)(base + init_base.size()) + i0,
+                                  (uint32_t)std::min<size_t>(65535, init_base.size() - i0), b->origin),
+                "init");
+    }
     hip_check(hipEventRecord(b->events[S], b->origin), "hipEventRecord");
     for (int s = 0; s < S; ++s) {
       hip_check(hipStreamWaitEvent(b->streams[s], b->events[S], 0), "hipStreamWaitEvent");

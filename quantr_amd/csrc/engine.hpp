@@ -156,6 +156,8 @@ PauliZTerm z_term(const PauliMasks& tm);
 // The observable as device tables: terms grouped by X mask (i^ny folded into coefficients).
 void pauli_tables(const std::vector<PauliMasks>& terms, std::vector<PauliGroup>& groups,
                   std::vector<PauliZTerm>& flat);
+// Puts the groups that are one real term without signs first; returns how many there are.
+int pauli_plain_first(std::vector<PauliGroup>& groups, const std::vector<PauliZTerm>& flat);
 // Orders an observable's G groups into expectation passes (no allocation): groups whose X
 // masks fit one tile are packed first-fit, widest first, into passes of one state read each;
 // groups too wide for a tile form a last, direct pass. Writes each group's X mask in its

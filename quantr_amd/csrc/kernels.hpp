@@ -135,9 +135,18 @@ struct PauliGroup {
   uint32_t first, count;
 };
 // lam[o] = sum over groups g, terms t of g: c_t (-1)^{popcount(j & zm_t)} psi[j], j = o ^ xm_g
-// (the whole observable in one pass).
+// (the whole observable in one pass). The first nplain groups have one term, with zm = 0 and ci = 0.
+// With `part`, part[0 .. pauli_sum_partials(dim)) = partial sums of Re <psi|lam>.
 hipError_t launch_pauli_sum(int prec, void* lam, const void* psi, uint64_t dim, const PauliGroup* groups, int ngroups,
-                            const PauliZTerm* terms, hipStream_t s);
+                            int nplain, const PauliZTerm* terms, hipStream_t s, double* part = nullptr);
+unsigned pauli_sum_partials(uint64_t dim);
+// |0...0> in `count` states of a pool: state y starts at byte base[y] and has 2^bits[y] amplitudes.
+hipError_t launch_init_batch(int prec, void* pool, const uint64_t* base, const uint32_t* bits, uint32_t count,
+                             hipStream_t s);
+// grads[r] = sum of part[r * ncols ..], r < nrows; energy[0] = sum of dot[0 .. ndot); stamp[0] = the
+// device clock when both are done.
+hipError_t launch_finish_instance(const double* part, uint64_t ncols, uint32_t nrows, double* grads, const double* dot,
+                                  uint64_t ndot, double* energy, uint64_t* stamp, hipStream_t s);
 // |0...0> in each of `count` states of dim amplitudes stored back to back.
 hipError_t launch_init_instances(int prec, void* psi, uint64_t dim, uint64_t count, hipStream_t s);
 // For each of `count` states stored back to back: its draws u[off[y] .. off[y+1]) (ascending)
@@ -205,9 +214,6 @@ int pauli_expect_partials(uint64_t dim);
 hipError_t launch_pauli_expect_passes(int prec, const void* psi, uint64_t dim, const void* groups, const void* terms,
                                       const PauliTilePass* passes, int npasses, const uint32_t* diag_count,
                                       double* part, hipStream_t s);
-// part[b] = partial sums of Re sum_j conj(a_j) b_j over nblocks blocks.
-hipError_t launch_dot_re_partial(int prec, const void* a, const void* b, uint64_t dim, double* part, int nblocks,
-                                 hipStream_t s);
 // psi[i] *= f for every amplitude, in place (the streaming ceiling of a sweep).
 hipError_t launch_stream_scale(int prec, void* psi, uint64_t dim, double f, hipStream_t s);
 // out[0] = the device wall clock (constant-rate counter).

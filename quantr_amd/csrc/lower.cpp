@@ -723,6 +723,11 @@ void pauli_tile_tables(int prec, const PauliGroup* groups, const uint32_t* lxm, 
   tt[nt] = PauliTileTerm{0, 0.0, 0, 0};
 }
 
+int pauli_plain_first(std::vector<PauliGroup>& groups, const std::vector<PauliZTerm>& flat) {
+  auto plain = [&](const PauliGroup& g) { return g.count == 1 && flat[g.first].zm == 0 && flat[g.first].ci == 0.0; };
+  return (int)(std::stable_partition(groups.begin(), groups.end(), plain) - groups.begin());
+}
+
 void pauli_tables(const std::vector<PauliMasks>& terms, std::vector<PauliGroup>& groups,
                   std::vector<PauliZTerm>& flat) {
   // terms grouped by X mask; Z masks and i^ny folded into per-term complex coefficients

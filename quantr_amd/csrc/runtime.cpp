@@ -845,6 +845,7 @@ void apply_observable(int prec, void* lam, const void* psi, uint64_t dim, const 
   std::vector<PauliGroup> groups;
   std::vector<PauliZTerm> flat;
   pauli_tables(terms, groups, flat);
+  const int nplain = pauli_plain_first(groups, flat);
   const size_t gb = groups.size() * sizeof(PauliGroup), tb = flat.size() * sizeof(PauliZTerm);
   scratch.reserve(gb + tb + 16);
   if (gb + tb) {
@@ -853,7 +854,7 @@ void apply_observable(int prec, void* lam, const void* psi, uint64_t dim, const 
     std::memcpy(blob + gb, flat.data(), tb);
     up.send(scratch.p, gb + tb, s);
   }
-  hip_check(launch_pauli_sum(prec, lam, psi, dim, (const PauliGroup*)scratch.p, (int)groups.size(),
+  hip_check(launch_pauli_sum(prec, lam, psi, dim, (const PauliGroup*)scratch.p, (int)groups.size(), nplain,
                              (const PauliZTerm*)((uint8_t*)scratch.p + gb), s),
             "pauli sum");
 }
