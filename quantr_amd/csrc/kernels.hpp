@@ -109,9 +109,17 @@ hipError_t launch_tile(int prec, int K, int RB, bool prefetch, void* psi, const 
 hipError_t launch_sample_fold(int prec, const void* psi, uint64_t dim, const double* u, uint64_t shots,
                               uint64_t* out, hipStream_t s);
 hipError_t launch_block_mass(int prec, const void* psi, uint64_t dim, int bb, double* mass, hipStream_t s);
+// Where blocks with a halfway case leave their probabilities: place p holds block[p]'s 2^bb from
+// probs[p * 2^bb] on. *count (device memory, zero at the start) may end above `most`.
+struct TieBlocks {
+  uint32_t* count;
+  uint32_t most;
+  uint64_t* block;
+  double* probs;
+};
 // Exact sums of rint(p_i * 2^(52-e)) per block for e = ebase[b] + 0..2, and halfway flags.
 hipError_t launch_block_exact_sums(int prec, const void* psi, uint64_t dim, int bb, const int32_t* ebase,
-                                   double* sums, uint32_t* flags, hipStream_t s);
+                                   double* sums, uint32_t* flags, const TieBlocks& tie, hipStream_t s);
 // out[y * 2^bb + q] = re^2 + im^2 (no fused operations) of amplitude q of block list[y] (block y if
 // list is null), y < count; out and list may be pinned host memory.
 hipError_t launch_gather_probs(int prec, const void* psi, int bb, const uint64_t* list, uint32_t count, double* out,

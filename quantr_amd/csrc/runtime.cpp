@@ -35,18 +35,34 @@ std::mutex g_pin_mu;
 std::vector<PinnedBlock> g_pinned;  // kept blocks, none in use
 uint64_t g_pin_states = 0;
 
+// Adds a block to the kept ones and takes out the smallest until no more than `keep` of at most
+// `bytes` are left (a large block is the one that costs most to make again); returns those.
+template <class Block>
+std::vector<Block> keep_block(std::vector<Block>& kept, const Block& b, size_t keep, size_t bytes) {
+  std::vector<Block> drop;
+  if (b.cap > bytes) {
+    drop.push_back(b);
+    return drop;
+  }
+  kept.push_back(b);
+  size_t held = 0;
+  for (const Block& x : kept) held += x.cap;
+  while (kept.size() > keep || held > bytes) {
+    auto least = std::min_element(kept.begin(), kept.end(), [](const Block& x, const Block& y) { return x.cap < y.cap; });
+    held -= least->cap;
+    drop.push_back(*least);
+    kept.erase(least);
+  }
+  return drop;
+}
+
 void pinned_give_back(void* p, size_t cap) {
-  void* drop = p;
+  std::vector<PinnedBlock> drop;
   {
     std::lock_guard<std::mutex> lk(g_pin_mu);
-    size_t held = cap;
-    for (const PinnedBlock& b : g_pinned) held += b.cap;
-    if (g_pinned.size() < kPinnedKeep && held <= kPinnedBytes) {
-      g_pinned.push_back({p, cap});
-      drop = nullptr;
-    }
+    drop = keep_block(g_pinned, PinnedBlock{p, cap}, kPinnedKeep, kPinnedBytes);
   }
-  if (drop) (void)hipHostFree(drop);
+  for (const PinnedBlock& b : drop) (void)hipHostFree(b.p);
 }
 }  // namespace
 
@@ -148,17 +164,12 @@ void DeviceLease::reserve(size_t bytes) {
 
 void DeviceLease::release() {
   if (!p) return;
-  void* drop = p;
+  std::vector<DeviceBlock> drop(1, DeviceBlock{p, cap_, device_});
   if (!std::uncaught_exceptions()) {  // after an error, hipFree waits for what may still run
     std::lock_guard<std::mutex> lk(g_dev_mu);
-    size_t held = cap_;
-    for (const DeviceBlock& b : g_device_blocks) held += b.cap;
-    if (g_device_blocks.size() < kDeviceKeep && held <= kDeviceBytes) {
-      g_device_blocks.push_back({p, cap_, device_});
-      drop = nullptr;
-    }
+    drop = keep_block(g_device_blocks, drop[0], kDeviceKeep, kDeviceBytes);
   }
-  if (drop) (void)hipFree(drop);
+  for (const DeviceBlock& b : drop) (void)hipFree(b.p);
   p = nullptr;
   cap_ = 0;
 }

@@ -7,7 +7,8 @@
 //  1. block masses (any order) give approximate block starts and so the binade e in which each
 //     block's fold most likely runs, and which blocks cross into the next one;
 //  2. per block, exact integer sums of rint(p_i / 2^(e-52)) for e and its two neighbours; the
-//     probabilities of the crossing blocks go to the host in the same step;
+//     probabilities of the crossing blocks and of those with a halfway case go to the host in
+//     the same step;
 //  3. on the host, the exact start of every block, in order: while a block's fold stays in the
 //     binade of its start, fl(S + p) = S + rint(p / U) * U exactly (U = 2^(e-52)), so its end is
 //     its start plus the integer sum. Blocks that cross into the next binade, hold a halfway
@@ -146,7 +147,7 @@ void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vec
   // leaves its binade, give or take the masses' rounding; then exact unit sums and these blocks'
   // probabilities
   constexpr uint64_t kMostFolds = 128;  // far above one per binade; further ones are fetched singly
-  PinnedLease pin(nblk * (4 + 3 * 8 + 4) + 64 + kMostFolds * 8);
+  PinnedLease pin(nblk * (4 + 3 * 8 + 4) + 64 + kMostFolds * 8 + 4);
   double* sums = (double*)pin.data();
   uint64_t* list = (uint64_t*)(sums + 3 * nblk);
   uint32_t* flags = (uint32_t*)(list + kMostFolds);
@@ -174,14 +175,21 @@ void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vec
       if (mass[b] != 0.0 && !inside && folds < kMostFolds) list[folds++] = b;
     }
   }
-  PinnedLease pin_probs(folds * len * 8 + 8);
+  // blocks with a halfway case: their number isn't known before the kernel runs
+  constexpr uint32_t kMostTies = 48;
+  PinnedLease pin_probs((folds + kMostTies) * len * 8 + kMostTies * 8);
   const double* probs = (const double*)pin_probs.data();
-  st->aux.reserve(nblk * 4);
-  hip_check(hipMemcpyAsync(st->aux.p, ebase, nblk * 4, hipMemcpyHostToDevice, st->stream), "H2D");
+  const double* tie_probs = probs + folds * len;
+  uint64_t* tie_block = (uint64_t*)(tie_probs + kMostTies * len);
+  std::fill(tie_block, tie_block + kMostTies, ~0ull);
+  ebase[nblk] = 0;  // their counter travels behind the binades
+  st->aux.reserve((nblk + 1) * 4);
+  hip_check(hipMemcpyAsync(st->aux.p, ebase, (nblk + 1) * 4, hipMemcpyHostToDevice, st->stream), "H2D");
+  const TieBlocks tie{(uint32_t*)st->aux.p + nblk, kMostTies, tie_block, (double*)tie_probs};
   {
     ProfScope ps_(st, "block_exact_sums", (double)st->dim * st->bytes_per_amp());
     hip_check(launch_block_exact_sums(st->prec, st->amp, st->dim, bb, (const int32_t*)st->aux.p, sums, flags,
-                                      st->stream),
+                                      tie, st->stream),
               "block exact sums");
   }
   hip_check(launch_gather_probs(st->prec, st->amp, bb, list, (uint32_t)folds, (double*)pin_probs.data(), st->stream),
@@ -195,6 +203,8 @@ void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vec
   auto probs_of = [&](uint64_t b) -> const double* {
     const uint64_t* at = std::lower_bound(list, list + folds, b);
     if (at != list + folds && *at == b) return probs + (at - list) * len;
+    const uint64_t* t = std::find(tie_block, tie_block + kMostTies, b);
+    if (t != tie_block + kMostTies) return tie_probs + (t - tie_block) * len;
     pin_one.reserve(len * 8 + 8);
     uint64_t* one = (uint64_t*)(pin_one.data() + len * 8);
     *one = b;
