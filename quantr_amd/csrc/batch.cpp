@@ -103,7 +103,7 @@ PlanParams fwd_params(uint32_t n, int prec, int k = 0) {
 PlanParams dual_params(uint32_t n, int prec, int k = 0) {
   PlanParams pp;
   pp.tile_bits = std::min<int>(k ? k : (prec == 0 ? 10 : 11), (int)n);
-  pp.reg_bits = std::min(4, pp.tile_bits);
+  pp.reg_bits = dual_reg_bits(pp.tile_bits);  // 32 instances of 10..18 qubits: 2.65 -> 2.50 ms per run
   pp.low_bits = prec == 0 ? 3 : 4;
   if (pp.tile_bits == (int)n) pp.max_ops = kWholeStateStageOps;
   return pp;

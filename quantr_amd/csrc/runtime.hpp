@@ -186,6 +186,7 @@ PlanParams plan_params(const qr_state* st);       // forward sweeps
 // The same for a state of n qubits, precision prec (0 = complex128) and options opt.
 PlanParams plan_params(uint32_t n, int prec, const qr_options& opt);
 PlanParams dual_plan_params(const qr_state* st);  // adjoint sweeps (psi and lam per tile)
+int dual_reg_bits(int tile_bits);                 // register bits of adjoint tiles
 
 // Offsets of one stage's data in a packed plan blob.
 struct Loc {

@@ -800,7 +800,7 @@ def test_expectation_arrangements(precision, n):
 
 
 @pytest.mark.parametrize("precision,tol", [(_capi.QR_C128, 1e-11), (_capi.QR_C64, 2e-5)])
-@pytest.mark.parametrize("tile_bits", [6, 10, 11, 12, 13])
+@pytest.mark.parametrize("tile_bits", [5, 7, 8, 9, 10, 11, 12, 13])
 def test_adjoint_tap_rows(tile_bits, precision, tol):
     """Gradient taps summed through LDS rows (workgroups of one to eight wavefronts, stages with
     more taps than rows) and singly (smaller workgroups), with angles beyond the shears' range and
