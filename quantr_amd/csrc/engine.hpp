@@ -64,6 +64,8 @@ enum TileForm : int {
   TF_NEGSWAP = 6, // [[0,-1],[1,0]] (Y, Y90, MY90 with their scalar factored out)
   TF_RROT = 7,    // real rotation as three shears, al = c[0], be = c[1] (Ry; magnitude folded out)
   TF_XROT = 8,    // the same for [[c,-is],[-is,c]], the rotation of (x, i y) (Rx)
+  TF_RROT_Y = 9,  // TF_RROT and TF_XROT with the shears on the |1> half first (adjoint sweeps)
+  TF_XROT_Y = 10,
 };
 
 // Exact value classes of an op, used to factor scalars out of uncontrolled gates.

@@ -218,7 +218,7 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
     switch (op.code) {
       case TC_U1: {
         const uint64_t outside = op.lane_cmask & ~tile_mask, inside = op.lane_cmask & tile_mask;
-        const uint32_t form = op.fold == FOLD_DROP_RROT ? (uint32_t)TF_RROT : op.fold == FOLD_DROP_XROT ? (uint32_t)TF_XROT : op.b;
+        const uint32_t form = op.fold == FOLD_DROP_RROT ? (uint32_t)TF_RROT_Y : op.fold == FOLD_DROP_XROT ? (uint32_t)TF_XROT_Y : op.b;
         if (inside == 0) {
           // controls outside the tile are the same for the whole workgroup: a scalar branch
           if (outside) o << "  if ((base & " << hex64(outside) << ") == " << hex64(outside) << ")";

@@ -197,15 +197,15 @@ void Uploader::send(void* dst, size_t bytes, hipStream_t s) {
 }
 
 // Default tile shape: 2^12 complex128 / 2^13 complex64 amplitudes (64 KB of LDS, two
-// workgroups per CU), 16 amplitudes per thread. States of up to 19 qubits leave most CUs without
-// such a tile: 2^11 amplitudes give two to four times the workgroups, which pays for a sweep
-// more or less (brickwork of 20 layers, complex128, 12 / 13 / 16 / 19 qubits: 95 / 98 / 121 / 165 us
-// with 2^12, 83 / 87 / 106 / 148 with 2^11; complex64 ansatz, 15 / 17 qubits: 132 / 152 -> 114 / 130;
-// at 20 qubits 268 -> 301). A complex64 state of 13 qubits stays in one tile (3 sweeps
-// instead of 8: 102 against 108 us).
+// workgroups per CU), 16 amplitudes per thread. Complex128 states of up to 19 qubits leave most CUs
+// without such a tile: 2^11 amplitudes give twice the workgroups, which pays for a sweep more or
+// less (brickwork of 20 layers, 12 / 13 / 16 / 19 qubits: 95 / 98 / 121 / 165 us with 2^12,
+// 83 / 87 / 106 / 148 with 2^11; an ansatz of 20 qubits 268 -> 301). Complex64 states keep 2^13: more
+// sweeps mean more factored scalars applied, and the energies of an 18-qubit ansatz were 1.4
+// times further from 64 bits with 2^11.
 int pick_tile_bits(const qr_state* st) {
   int k = st->prec == 0 ? 12 : 13;
-  if (st->n <= 19 && (int)st->n != (st->prec == 0 ? 11 : 13)) k = 11;
+  if (st->prec == 0 && st->n <= 19) k = 11;
   if (st->opt.tile_bits) k = std::min<int>(tile_max_bits(st->prec), (int)st->opt.tile_bits);
   return std::min<int>(k, (int)st->n);
 }

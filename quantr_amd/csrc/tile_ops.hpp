@@ -93,6 +93,41 @@ __device__ __forceinline__ void rot_x(Regs<R, RB>& a, R al, R be, uint32_t ns) {
   }
 }
 
+// The same rotations with the shears on y first and last: y is rounded twice and x once. Used by the
+// adjoint sweeps, whose states end near |0...0> and start near it in training, where x holds the
+// large amplitudes (complex64 gradients of 13 qubits and 6 layers, rms error against 64 bits:
+// 1.07e-6 with x first, 0.84e-6 with y first).
+template <typename R, int RB, int J, bool HAS_NS>
+__device__ __forceinline__ void rot_real_y(Regs<R, RB>& a, R al, R be, uint32_t ns) {
+#pragma unroll
+  for (int m0 = 0; m0 < (1 << RB); ++m0) {
+    if (m0 & (1 << J)) continue;
+    if (HAS_NS && ((uint32_t)m0 & ns) != ns) continue;
+    const int m1 = m0 | (1 << J);
+    R xr = a.v[m0].x, xi = a.v[m0].y, yr = a.v[m1].x, yi = a.v[m1].y;
+    yr = fma(-al, xr, yr); yi = fma(-al, xi, yi);
+    xr = fma(-be, yr, xr); xi = fma(-be, yi, xi);
+    yr = fma(-al, xr, yr); yi = fma(-al, xi, yi);
+    a.v[m0].x = xr; a.v[m0].y = xi;
+    a.v[m1].x = yr; a.v[m1].y = yi;
+  }
+}
+template <typename R, int RB, int J, bool HAS_NS>
+__device__ __forceinline__ void rot_x_y(Regs<R, RB>& a, R al, R be, uint32_t ns) {
+#pragma unroll
+  for (int m0 = 0; m0 < (1 << RB); ++m0) {
+    if (m0 & (1 << J)) continue;
+    if (HAS_NS && ((uint32_t)m0 & ns) != ns) continue;
+    const int m1 = m0 | (1 << J);
+    R xr = a.v[m0].x, xi = a.v[m0].y, yr = a.v[m1].x, yi = a.v[m1].y;
+    yi = fma(al, xr, yi); yr = fma(-al, xi, yr);
+    xr = fma(be, yi, xr); xi = fma(-be, yr, xi);
+    yi = fma(al, xr, yi); yr = fma(-al, xi, yr);
+    a.v[m0].x = xr; a.v[m0].y = xi;
+    a.v[m1].x = yr; a.v[m1].y = yi;
+  }
+}
+
 // 2x2 on register slot J for every register pair whose register-held controls (ns) are 1.
 template <typename R, int RB, int J, int FORM, bool HAS_NS>
 __device__ __forceinline__ void u1_slot(Regs<R, RB>& a, const Coef4 u, uint32_t ns) {
@@ -101,6 +136,11 @@ __device__ __forceinline__ void u1_slot(Regs<R, RB>& a, const Coef4 u, uint32_t 
   if (FORM == 7 || FORM == 8) {  // rotations as shears: al in c[0], be in c[1]
     if (FORM == 7) rot_real<R, RB, J, HAS_NS>(a, u00r, u01r, ns);
     else rot_x<R, RB, J, HAS_NS>(a, u00r, u01r, ns);
+    return;
+  }
+  if (FORM == 9 || FORM == 10) {
+    if (FORM == 9) rot_real_y<R, RB, J, HAS_NS>(a, u00r, u01r, ns);
+    else rot_x_y<R, RB, J, HAS_NS>(a, u00r, u01r, ns);
     return;
   }
 #pragma unroll
