@@ -71,15 +71,6 @@ void pinned_state_created() {
   ++g_pin_states;
 }
 
-void pinned_state_destroyed() {
-  std::vector<PinnedBlock> drop;
-  {
-    std::lock_guard<std::mutex> lk(g_pin_mu);
-    if (--g_pin_states == 0) drop.swap(g_pinned);
-  }
-  for (const PinnedBlock& b : drop) (void)hipHostFree(b.p);
-}
-
 void PinnedLease::reserve(size_t bytes) {
   if (bytes <= cap_) return;
   if (p_) pinned_give_back(p_, cap_);
@@ -121,6 +112,20 @@ struct DeviceBlock {
 std::mutex g_dev_mu;
 std::vector<DeviceBlock> g_device_blocks;  // kept blocks, none in use
 }  // namespace
+
+void pinned_state_destroyed() {
+  std::vector<PinnedBlock> drop;
+  std::vector<DeviceBlock> drop_dev;
+  {
+    std::scoped_lock lk(g_pin_mu, g_dev_mu);
+    if (--g_pin_states == 0) {
+      drop.swap(g_pinned);
+      drop_dev.swap(g_device_blocks);
+    }
+  }
+  for (const PinnedBlock& b : drop) (void)hipHostFree(b.p);
+  for (const DeviceBlock& b : drop_dev) (void)hipFree(b.p);
+}
 
 hipError_t device_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);

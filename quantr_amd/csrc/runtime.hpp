@@ -31,8 +31,8 @@ hipError_t device_malloc(void** p, size_t bytes);
 
 // A block of device memory held for one call without a state of its own. Blocks are kept for later
 // calls (allocating and freeing them took longer than the call's kernels): at most 8 of them and
-// 256 MB; larger ones are not kept, and all are given back when an allocation would fail. The
-// holder's work on the block is done before it lets go.
+// 256 MB; larger ones are not kept, and all are given back when an allocation would fail and with the
+// last state. The holder's work on the block is done before it lets go.
 class DeviceLease {
  public:
   DeviceLease() = default;
@@ -84,7 +84,7 @@ class PinnedLease {
   size_t cap_ = 0;
 };
 void pinned_state_created();    // one more state lives
-void pinned_state_destroyed();  // one less; the last one frees the kept blocks
+void pinned_state_destroyed();  // one less; the last one frees the kept blocks, host and device
 
 // Uploads of small host data onto a stream without waiting for it: two pinned blocks in turn, each
 // reused once its last copy is done. The owner's stream is idle before it is destroyed.
