@@ -73,7 +73,11 @@ struct qr_batch {
   size_t host_blob_size = 0;
   uint64_t total_params = 0;
   double clock_khz = 0.0;
+  qr_batch() { qr::pinned_state_created(); }
   ~qr_batch() {
+    if (origin) (void)hipStreamSynchronize(origin);
+    host_blob.release();
+    qr::pinned_state_destroyed();
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     for (auto e : events) (void)hipEventDestroy(e);

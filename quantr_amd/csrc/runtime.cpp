@@ -94,11 +94,13 @@ void PinnedLease::reserve(size_t bytes) {
   cap_ = want;
 }
 
-PinnedLease::~PinnedLease() {
+void PinnedLease::release() {
   if (!p_) return;
   // a call that ends in an error may leave work in flight on the block: hipHostFree waits for it
   if (std::uncaught_exceptions()) (void)hipHostFree(p_);
   else pinned_give_back(p_, cap_);
+  p_ = nullptr;
+  cap_ = 0;
 }
 
 // ---- device memory kept between calls -----------------------------------------------------

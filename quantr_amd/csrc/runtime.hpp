@@ -32,7 +32,7 @@ hipError_t device_malloc(void** p, size_t bytes);
 // A block of device memory held for one call without a state of its own. Blocks are kept for later
 // calls (allocating and freeing them took longer than the call's kernels): at most 8 of them and
 // 256 MB; larger ones are not kept, and all are given back when an allocation would fail and with the
-// last state. The holder's work on the block is done before it lets go.
+// last state or batch. The holder's work on the block is done before it lets go.
 class DeviceLease {
  public:
   DeviceLease() = default;
@@ -68,23 +68,24 @@ struct DevBuf {
 
 // A block of pinned host memory, which kernels and copies reach directly, held for one call.
 // Blocks are kept for later calls (pinning a new one takes longer than a small call): at most
-// 8 of them and 64 MB, given back when the last state is destroyed.
+// 8 of them and 64 MB, given back when the last state or batch is destroyed.
 class PinnedLease {
  public:
   PinnedLease() = default;
   explicit PinnedLease(size_t bytes) { reserve(bytes); }
-  ~PinnedLease();
+  ~PinnedLease() { release(); }
   PinnedLease(const PinnedLease&) = delete;
   PinnedLease& operator=(const PinnedLease&) = delete;
   void reserve(size_t bytes);  // at least this size; what it held is lost
+  void release();              // back to the kept blocks
   uint8_t* data() const { return (uint8_t*)p_; }
 
  private:
   void* p_ = nullptr;
   size_t cap_ = 0;
 };
-void pinned_state_created();    // one more state lives
-void pinned_state_destroyed();  // one less; the last one frees the kept blocks, host and device
+void pinned_state_created();    // one more state or batch lives
+void pinned_state_destroyed();  // one less; the last one, its own blocks let go of, frees the kept blocks, host and device
 
 // Uploads of small host data onto a stream without waiting for it: two pinned blocks in turn, each
 // reused once its last copy is done. The owner's stream is idle before it is destroyed.
@@ -94,6 +95,11 @@ class Uploader {
   // A block of `bytes` to fill, then send() it to dst on stream s.
   uint8_t* begin(size_t bytes);
   void send(void* dst, size_t bytes, hipStream_t s);
+  // Lets go of both blocks; their copies are done.
+  void release() {
+    for (PinnedLease& b : buf_) b.release();
+    busy_[0] = busy_[1] = false;
+  }
 
  private:
   PinnedLease buf_[2];
@@ -130,6 +136,7 @@ struct qr_state {
   size_t bytes_per_amp() const { return prec == 0 ? 16 : 8; }
   ~qr_state() {
     if (stream) (void)hipStreamSynchronize(stream);
+    up.release();
     if (counted) qr::pinned_state_destroyed();
     for (auto& r : prof) {
       (void)hipEventDestroy(r.a);
