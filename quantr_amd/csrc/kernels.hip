@@ -870,6 +870,8 @@ __device__ __forceinline__ void lds_pairs(const T (&a)[16], const T (&y)[8], boo
 
 // In-place Walsh-Hadamard transform: w[p] becomes sum_i (-1)^{popcount(i & p)} w[i], the sum of
 // the values under every sign pattern p at once.
+// The results are opaque: the compiler would else move the last additions to each pattern's use, and
+// hold (and spill) the values of every step until then.
 template <int N>
 __device__ __forceinline__ void walsh(double (&w)[N]) {
 #pragma unroll
@@ -881,6 +883,8 @@ __device__ __forceinline__ void walsh(double (&w)[N]) {
         w[i] = x + y;
         w[i | h] = x - y;
       }
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(w[i]));
 }
 __device__ __forceinline__ double at_pattern(const double (&w)[8], uint32_t p) {
   double v;
@@ -895,6 +899,18 @@ __device__ __forceinline__ double at_pattern(const double (&w)[8], uint32_t p) {
     default: v = w[7]; break;
   }
   return v;
+}
+
+// Records at uniform addresses, through scalar loads: the constant address space says that nothing
+// writes them while the kernel runs. From plain pointers the compiler made vector loads (it takes a
+// barrier for a possible write), and a wavefront waited for each record behind its tile's loads.
+__device__ __forceinline__ PauliTileTerm load_term(const PauliTileTerm* p) {
+  const auto q = (const __attribute__((address_space(4))) uint64_t*)p;
+  return PauliTileTerm{q[0], __longlong_as_double((long long)q[1]), (uint32_t)q[2], (uint32_t)(q[2] >> 32)};
+}
+__device__ __forceinline__ PauliTileGroup load_group(const PauliTileGroup* p) {
+  const auto q = (const __attribute__((address_space(4))) uint32_t*)p;
+  return PauliTileGroup{q[0], q[1], q[2], q[3]};
 }
 
 // A term's coefficient with its sign (-1)^{parity}: the parity of the tile's bits is uniform, the
@@ -913,7 +929,7 @@ __device__ __forceinline__ double signed_terms(const double (&w)[8], const Pauli
                                                uint32_t count, PauliTileTerm& t, uint64_t base, uint32_t pt) {
   double acc = 0.0;
   for (; count; --count) {
-    const PauliTileTerm next = *tp++;
+    const PauliTileTerm next = load_term(tp++);
     acc = fma(signed_coeff(t, base, pt), at_pattern(w, t.pat), acc);
     t = next;
   }
@@ -927,11 +943,93 @@ template <typename T, int M>
 __device__ __forceinline__ void plain_groups(const T (&a)[16], uint32_t plain, const PauliTileTerm* __restrict__& tp,
                                              PauliTileTerm& t, uint64_t base, uint32_t pt, double& acc) {
   if ((plain >> M) & 1u) {
-    const PauliTileTerm next = *tp++;
+    const PauliTileTerm next = load_term(tp++);
     acc = fma(signed_coeff(t, base, pt), pairs_sum<T, M>(a), acc);
     t = next;
   }
   if constexpr (M < 15) plain_groups<T, M + 1>(a, plain, tp, t, base, pt, acc);
+}
+
+// LDS slot of a tile's element p (see k_pauli_expect_tiles).
+template <int K>
+__device__ __forceinline__ uint32_t pauli_slot(uint32_t p) {
+  constexpr int LN = K - 12;
+  return p ^ (((p >> (LN + 4)) & 15u) << LN);
+}
+// Tile position of a thread's register 0 in arrangement A.
+template <int K, int A>
+__device__ __forceinline__ uint32_t pauli_thread(uint32_t lane) {
+  constexpr uint32_t nb = (uint32_t)pauli_arrangement_bit(K, A);
+  return (lane & ((1u << nb) - 1u)) | ((lane >> nb) << (nb + 4));
+}
+
+// A thread's 16 amplitudes from arrangement A - 1 to arrangement A, real parts and then imaginary
+// parts through an LDS array of 2^K reals.
+template <typename R, int K, int A, typename T>
+__device__ __forceinline__ void rearrange(T (&a)[16], R* lds, uint32_t lane) {
+  constexpr int from = pauli_arrangement_bit(K, A - 1), to = pauli_arrangement_bit(K, A);
+  // the thread's place, opaque: addresses are computed for each round, not kept in registers
+  auto place = [&]() {
+    uint32_t l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  __syncthreads();  // the reads before are over
+  uint32_t p = pauli_thread<K, A - 1>(place());
+#pragma unroll
+  for (uint32_t r = 0; r < 16; ++r) lds[pauli_slot<K>(p | (r << from))] = a[r].x;
+  __syncthreads();
+  p = pauli_thread<K, A>(place());
+#pragma unroll
+  for (uint32_t r = 0; r < 16; ++r) a[r].x = lds[pauli_slot<K>(p | (r << to))];
+  __syncthreads();
+  p = pauli_thread<K, A - 1>(place());
+#pragma unroll
+  for (uint32_t r = 0; r < 16; ++r) lds[pauli_slot<K>(p | (r << from))] = a[r].y;
+  __syncthreads();
+  p = pauli_thread<K, A>(place());
+#pragma unroll
+  for (uint32_t r = 0; r < 16; ++r) a[r].y = lds[pauli_slot<K>(p | (r << to))];
+}
+
+// X mask 0 of a tile in arrangement 0: terms sorted by pattern, diag_count[p] of each.
+template <typename T>
+__device__ __forceinline__ void diag_group(const T (&a)[16], const uint32_t (&diag_count)[16],
+                                           const PauliTileTerm* __restrict__& tp, PauliTileTerm& tm, uint64_t base,
+                                           uint32_t pt, double& acc) {
+  double w[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) w[r] = fma((double)a[r].x, (double)a[r].x, (double)a[r].y * (double)a[r].y);
+  walsh<16>(w);
+#pragma unroll
+  for (int p = 0; p < 16; ++p) {
+    uint32_t count = diag_count[p];
+    if (count == 0) continue;
+    double f = 0.0;
+    for (; count; --count) {
+      const PauliTileTerm tn = load_term(tp++);
+      f += signed_coeff(tm, base, pt);
+      tm = tn;
+    }
+    acc = fma(f, w[p], acc);
+  }
+}
+
+// X mask 0 and the plain groups of arrangements A and up.
+template <typename R, int K, int A, typename T>
+__device__ __forceinline__ void plain_arrangements(T (&a)[16], R* lds, uint32_t lane, const PauliTilePass& ps,
+                                                   const uint32_t (&diag_count)[16],
+                                                   const PauliTileTerm* __restrict__& tp, PauliTileTerm& tm,
+                                                   uint64_t base, double& acc) {
+  if ((ps.arrs >> A) == 0) return;
+  if constexpr (A > 0) rearrange<R, K, A>(a, lds, lane);
+  const uint32_t pt = pauli_thread<K, A>(lane);
+  if constexpr (A == 0) {
+    if (ps.diag) diag_group(a, diag_count, tp, tm, base, pt, acc);
+  }
+  if (ps.plain[A]) plain_groups<T, 1>(a, ps.plain[A], tp, tm, base, pt, acc);
+  if constexpr (A + 1 < kPauliArrangements)
+    plain_arrangements<R, K, A + 1>(a, lds, lane, ps, diag_count, tp, tm, base, acc);
 }
 
 // Partial sums of Re <psi|O|psi> for groups whose X masks lie in tiles of 2^K amplitudes (tile
@@ -946,23 +1044,31 @@ __device__ __forceinline__ void plain_groups(const T (&a)[16], uint32_t plain, c
 //  * signs: a Walsh-Hadamard transform of the 8 pair products (16 probabilities for X mask 0)
 //    holds the sum under every pattern of register bits, so a term takes one multiply-add for
 //    all of a thread's amplitudes instead of one add for each.
+//  * without general groups (Ising and the like), the exchange between arrangements moves real
+//    parts and then imaginary parts through half the LDS, and complex128 fits four workgroups on a
+//    CU in place of two: one's loads run under the others' arithmetic. Complex64 is held to two by
+//    its registers (111 at 512 threads), and keeps the exchange of whole amplitudes.
 // What it measured against one LDS read and a signed add per amplitude, group and term: the Ising
-// observable of 29 qubits, complex128 (57 terms, 29 X masks, 3 passes), 13.5 -> 5.6 ms, 1.9 ms a
-// pass = 4.6 TB/s; complex64, 28 qubits, 6.5 -> 1.7 ms; 120 strings of up to 4 factors on 22
-// qubits 506 -> 367 us. Fetching the next tile ahead took longer (5.9 ms: its registers spill).
+// observable of 29 qubits, complex128 (57 terms, 29 X masks, 3 passes), 13.5 -> 4.2 ms = 6.1 TB/s
+// (5.6 ms with vector loads of the records and two workgroups per CU); a pass of Z terms alone 6.9
+// TB/s, one of twelve contiguous X masks 6.1, one of nine X masks 2^12 and up in 128-byte segments
+// 5.0. Complex64, 28 qubits, 6.5 -> 1.6 ms (2.1 with vector loads); 120 strings of up to 4 factors on 22 qubits
+// 520 -> 335 us (355). Fetching the next tile ahead took longer (5.9 ms: its registers spill).
 // Element p of the tile sits at LDS slot p ^ (bits above the lowest arrangement's nibble, at its
 // place): consecutive lanes hit distinct slots in all three arrangements.
 template <typename R, int K, bool NT, bool GENERAL>
-__global__ __launch_bounds__(1 << (K - 4), K == 12 ? 2 : 4) void k_pauli_expect_tiles(
+__global__ __launch_bounds__(1 << (K - 4), K == 12 && GENERAL ? 2 : 4) void k_pauli_expect_tiles(
     const typename CT<R>::T* __restrict__ psi, uint64_t dim, PauliTilePasses P,
     const PauliTileGroup* __restrict__ groups, const PauliTileTerm* __restrict__ terms, double* __restrict__ part,
     int accumulate) {
   using T = typename CT<R>::T;
-  constexpr int TB = K - 4, LN = K - 12;  // thread bits; the lowest arrangement's first bit
-  __shared__ T lds[1 << K];
+  constexpr int TB = K - 4;  // thread bits
+  constexpr bool HALF = !GENERAL && K == 12;
+  __shared__ __align__(16) R lds_reals[(HALF ? 1 : 2) << K];
+  T* const lds = reinterpret_cast<T*>(lds_reals);
   const uint32_t tid = threadIdx.x;
   const uint32_t ntiles = (uint32_t)(dim >> K);  // 2^28 at most
-  auto slot = [](uint32_t p) { return p ^ (((p >> (LN + 4)) & 15u) << LN); };
+  auto slot = [](uint32_t p) { return pauli_slot<K>(p); };
   double acc = 0.0;
   uint32_t t = blockIdx.x;  // this workgroup's next (pass, tile), counted through all passes
   for (uint32_t ip = 0; ip < P.count; ++ip) {
@@ -1009,8 +1115,12 @@ __global__ __launch_bounds__(1 << (K - 4), K == 12 ? 2 : 4) void k_pauli_expect_
       // records and terms in the order of their use, each fetched one ahead
       const PauliTileGroup* __restrict__ gp = groups + ps.first;
       const PauliTileTerm* __restrict__ tp = terms + ps.term0;
-      PauliTileGroup gr = *gp++;
-      PauliTileTerm tm = *tp++;
+      PauliTileGroup gr = load_group(gp++);
+      PauliTileTerm tm = load_term(tp++);
+      if constexpr (HALF) {
+        plain_arrangements<R, K, 0>(a, lds_reals, lane, ps, P.diag_count, tp, tm, base, acc);
+        continue;
+      }
       if (ps.lds) {
         __syncthreads();  // the previous tile's reads are over
 #pragma unroll
@@ -1034,29 +1144,11 @@ __global__ __launch_bounds__(1 << (K - 4), K == 12 ? 2 : 4) void k_pauli_expect_
             a[r].y = d.y;
           }
         }
-        if (arr == 0 && ps.diag) {  // X mask 0: terms sorted by pattern
-          double w[16];
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            w[r] = fma((double)a[r].x, (double)a[r].x, (double)a[r].y * (double)a[r].y);
-          walsh<16>(w);
-#pragma unroll
-          for (int p = 0; p < 16; ++p) {
-            uint32_t count = P.diag_count[p];
-            if (count == 0) continue;
-            double f = 0.0;
-            for (; count; --count) {
-              const PauliTileTerm tn = *tp++;
-              f += signed_coeff(tm, base, pt);
-              tm = tn;
-            }
-            acc = fma(f, w[p], acc);
-          }
-        }
+        if (arr == 0 && ps.diag) diag_group(a, P.diag_count, tp, tm, base, pt, acc);
         if (ps.plain[arr]) plain_groups<T, 1>(a, ps.plain[arr], tp, tm, base, pt, acc);
 #pragma unroll 1
         for (uint32_t left = GENERAL ? ps.cnt[arr] : 0; left; --left) {
-          const PauliTileGroup next = *gp++;
+          const PauliTileGroup next = load_group(gp++);
           const uint32_t op = gr.op, nre = gr.nre, nim = gr.nim, lx = gr.lx;
           gr = next;
           // products of the loop-invariant amplitudes must not move out of the group loop: the
@@ -1110,7 +1202,7 @@ __global__ __launch_bounds__(1 << (K - 4), K == 12 ? 2 : 4) void k_pauli_expect_
     t -= ntiles;
   }
   __syncthreads();
-  double* red = reinterpret_cast<double*>(lds);
+  double* red = reinterpret_cast<double*>(lds_reals);
   red[tid] = acc;
   __syncthreads();
   for (uint32_t w = 1u << (TB - 1); w > 0; w >>= 1) {

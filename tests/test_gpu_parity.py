@@ -799,6 +799,36 @@ def test_expectation_arrangements(precision, n):
     st.close()
 
 
+@pytest.mark.parametrize("n,precision", [(12, _capi.QR_C128), (13, _capi.QR_C64), (17, _capi.QR_C128),
+                                         (18, _capi.QR_C64)])
+def test_expectation_plain_groups(n, precision):
+    """Observables without general groups, whose tiles pass from one arrangement of register bits
+    to the next: X masks in the first, second or third arrangement alone, with the ones between
+    left out, with Z strings, and of several passes. Tolerance as for every arrangement above."""
+    rng = np.random.default_rng(4300 + n)
+    st = _capi.State(n, precision)
+    st.apply(W.to_program(W.brickwork(n, depth=7, seed=n + 2)))
+    psi = st.amplitudes()
+    k = 12 if precision == _capi.QR_C128 else 13
+    nibbles = [[b for b in range(max(k - 4 - 4 * a, 0), k - 4 * a)] for a in range(4) if k - 4 * a > 0]
+
+    def xs(bits):
+        return [(float(rng.uniform(-1, 1)), [(n - 1 - b, "X")]) for b in bits]
+
+    def pair(bits):
+        return [(float(rng.uniform(-1, 1)), [(n - 1 - b, "X") for b in bits[:2]])]
+
+    zs = [(float(rng.uniform(-1, 1)), [(n - 1 - b, "Z"), (n - 1 - (b + 3) % n, "Z")]) for b in range(n)]
+    sets = [zs] + [xs(b) for b in nibbles] + [pair(b) + zs for b in nibbles if len(b) > 1]
+    sets += [xs(nibbles[0]) + pair(nibbles[2]), xs(range(k)) + zs, xs(range(n)) + zs]
+    for terms in sets:
+        obs = _capi.Observable(terms)
+        got = st.expectation(obs)
+        want = H.oracle_expectation(n, psi, obs)
+        assert abs(got - want) < 16 * n * 2.0 ** -52 * sum(abs(c) for c, _ in terms)
+    st.close()
+
+
 @pytest.mark.parametrize("precision,tol", [(_capi.QR_C128, 1e-11), (_capi.QR_C64, 2e-5)])
 @pytest.mark.parametrize("tile_bits", [5, 7, 8, 9, 10, 11, 12, 13])
 def test_adjoint_tap_rows(tile_bits, precision, tol):
