@@ -916,9 +916,8 @@ __device__ __forceinline__ PauliTileGroup load_group(const PauliTileGroup* p) {
 // A term's coefficient with its sign (-1)^{parity}: the parity of the tile's bits is uniform, the
 // thread's comes from its tile position pt.
 __device__ __forceinline__ double signed_coeff(const PauliTileTerm& t, uint64_t base, uint32_t pt) {
-  uint32_t hi = (uint32_t)__double2hiint(t.c);
-  hi ^= (uint32_t)__popcll(base & t.zout) << 31;
-  hi ^= (uint32_t)__popc(pt & t.lz) << 31;
+  const uint32_t ones = (uint32_t)__popc(pt & t.lz) + (uint32_t)__popcll(base & t.zout);
+  const uint32_t hi = (uint32_t)__double2hiint(t.c) + (ones << 31);  // an odd count flips the sign bit
   return __hiloint2double((int)hi, __double2loint(t.c));
 }
 
@@ -987,33 +986,44 @@ __device__ __forceinline__ uint32_t pauli_thread(uint32_t lane) {
   return (lane & ((1u << nb) - 1u)) | ((lane >> nb) << (nb + 4));
 }
 
+// The LDS slot of a thread's register r in arrangement A. Slots are linear: the thread's part, at byte
+// offset `first`, meets the register's constant one in the lowest nibble only, so an access takes at
+// most one xor, and the rest is its immediate offset.
+template <typename R, int K, int A>
+__device__ __forceinline__ R& pauli_at(R* lds, uint32_t first, uint32_t r) {
+  const uint32_t s = pauli_slot<K>(r << pauli_arrangement_bit(K, A)), low = s & (15u << (K - 12));
+  return *reinterpret_cast<R*>(reinterpret_cast<char*>(lds) + ((first ^ (low * sizeof(R))) + (s - low) * sizeof(R)));
+}
+
 // A thread's 16 amplitudes from arrangement A - 1 to arrangement A, real parts and then imaginary
 // parts through an LDS array of 2^K reals.
 template <typename R, int K, int A, typename T>
 __device__ __forceinline__ void rearrange(T (&a)[16], R* lds, uint32_t lane) {
-  constexpr int from = pauli_arrangement_bit(K, A - 1), to = pauli_arrangement_bit(K, A);
+  static_assert(K == 12, "arrangements of whole nibbles");
   // the thread's place, opaque: addresses are computed for each round, not kept in registers
-  auto place = [&]() {
+  auto place = [&](auto arrangement) {
     uint32_t l = lane;
     asm volatile("" : "+v"(l));
-    return l;
+    return pauli_slot<K>(pauli_thread<K, decltype(arrangement)::value>(l)) * (uint32_t)sizeof(R);
   };
+  constexpr std::integral_constant<int, A - 1> from{};
+  constexpr std::integral_constant<int, A> to{};
   __syncthreads();  // the reads before are over
-  uint32_t p = pauli_thread<K, A - 1>(place());
+  uint32_t p = place(from);
 #pragma unroll
-  for (uint32_t r = 0; r < 16; ++r) lds[pauli_slot<K>(p | (r << from))] = a[r].x;
+  for (uint32_t r = 0; r < 16; ++r) pauli_at<R, K, A - 1>(lds, p, r) = a[r].x;
   __syncthreads();
-  p = pauli_thread<K, A>(place());
+  p = place(to);
 #pragma unroll
-  for (uint32_t r = 0; r < 16; ++r) a[r].x = lds[pauli_slot<K>(p | (r << to))];
+  for (uint32_t r = 0; r < 16; ++r) a[r].x = pauli_at<R, K, A>(lds, p, r);
   __syncthreads();
-  p = pauli_thread<K, A - 1>(place());
+  p = place(from);
 #pragma unroll
-  for (uint32_t r = 0; r < 16; ++r) lds[pauli_slot<K>(p | (r << from))] = a[r].y;
+  for (uint32_t r = 0; r < 16; ++r) pauli_at<R, K, A - 1>(lds, p, r) = a[r].y;
   __syncthreads();
-  p = pauli_thread<K, A>(place());
+  p = place(to);
 #pragma unroll
-  for (uint32_t r = 0; r < 16; ++r) a[r].y = lds[pauli_slot<K>(p | (r << to))];
+  for (uint32_t r = 0; r < 16; ++r) a[r].y = pauli_at<R, K, A>(lds, p, r);
 }
 
 // X mask 0 of a tile in arrangement 0: terms sorted by pattern, diag_count[p] of each.
@@ -1052,7 +1062,7 @@ __device__ __forceinline__ void plain_arrangements(T (&a)[16], R* lds, uint32_t 
     if (ps.diag) diag_group(a, diag_count, tp, tm, base, pt, acc);
   }
   if (ps.plain[A]) plain_groups<T, 1>(a, ps.plain[A], tp, tm, base, pt, acc);
-  if constexpr (A + 1 < kPauliArrangements)
+  if constexpr (pauli_arrangement_bit(K, A) > 0)  // the last one holds the lowest bits
     plain_arrangements<R, K, A + 1>(a, lds, lane, ps, diag_count, tp, tm, base, acc);
 }
 
@@ -1073,7 +1083,7 @@ __device__ __forceinline__ void plain_arrangements(T (&a)[16], R* lds, uint32_t 
 //    CU in place of two: one's loads run under the others' arithmetic. Complex64 is held to two by
 //    its registers (111 at 512 threads), and keeps the exchange of whole amplitudes.
 // What it measured against one LDS read and a signed add per amplitude, group and term: the Ising
-// observable of 29 qubits, complex128 (57 terms, 29 X masks, 3 passes), 13.5 -> 4.2 ms = 6.1 TB/s
+// observable of 29 qubits, complex128 (57 terms, 29 X masks, 3 passes), 13.5 -> 4.1 ms = 6.3 TB/s
 // (5.6 ms with vector loads of the records and two workgroups per CU); a pass of Z terms alone 6.9
 // TB/s, one of twelve contiguous X masks 6.1, one of nine X masks 2^12 and up in 128-byte segments
 // 5.0. Complex64, 28 qubits, 6.5 -> 1.6 ms (2.1 with vector loads); 120 strings of up to 4 factors on 22 qubits
