@@ -16,97 +16,9 @@
 
 #include "engine.hpp"
 #include "kernels.hpp"
+#include "workspace.hpp"
 
 namespace qr {
-
-inline void hip_check(hipError_t e, const char* what) {
-  if (e == hipSuccess) return;
-  if (e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation)
-    throw Error{QR_ERR_OOM, std::string(what) + ": " + hipGetErrorString(e)};
-  throw Error{QR_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e)};
-}
-
-// Device memory with what the library keeps for later calls given back before it fails.
-hipError_t device_malloc(void** p, size_t bytes);
-
-// A block of device memory held for one call without a state of its own. Blocks are kept for later
-// calls (allocating and freeing them took longer than the call's kernels): at most 8 of them and
-// 256 MB; larger ones are not kept, and all are given back when an allocation would fail and with the
-// last state or batch. The holder's work on the block is done before it lets go.
-class DeviceLease {
- public:
-  DeviceLease() = default;
-  ~DeviceLease();
-  DeviceLease(const DeviceLease&) = delete;
-  DeviceLease& operator=(const DeviceLease&) = delete;
-  void reserve(size_t bytes);  // at least this size; what it held is lost
-  void* p = nullptr;
-
- private:
-  void release();
-  size_t cap_ = 0;
-  int device_ = 0;
-};
-
-// Device buffer that grows on demand.
-struct DevBuf {
-  void* p = nullptr;
-  size_t cap = 0;
-  void reserve(size_t bytes) {
-    if (bytes <= cap) return;
-    if (p) hip_check(hipFree(p), "hipFree");
-    p = nullptr;
-    cap = 0;
-    size_t want = std::max<size_t>(bytes, 1 << 16);
-    hip_check(device_malloc(&p, want), "hipMalloc (workspace)");
-    cap = want;
-  }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
-};
-
-// A block of pinned host memory, which kernels and copies reach directly, held for one call.
-// Blocks are kept for later calls (pinning a new one takes longer than a small call): at most
-// 8 of them and 64 MB, given back when the last state or batch is destroyed.
-class PinnedLease {
- public:
-  PinnedLease() = default;
-  explicit PinnedLease(size_t bytes) { reserve(bytes); }
-  ~PinnedLease() { release(); }
-  PinnedLease(const PinnedLease&) = delete;
-  PinnedLease& operator=(const PinnedLease&) = delete;
-  void reserve(size_t bytes);  // at least this size; what it held is lost
-  void release();              // back to the kept blocks
-  uint8_t* data() const { return (uint8_t*)p_; }
-
- private:
-  void* p_ = nullptr;
-  size_t cap_ = 0;
-};
-void pinned_state_created();    // one more state or batch lives
-void pinned_state_destroyed();  // one less; the last one, its own blocks let go of, frees the kept blocks, host and device
-
-// Uploads of small host data onto a stream without waiting for it: two pinned blocks in turn, each
-// reused once its last copy is done. The owner's stream is idle before it is destroyed.
-class Uploader {
- public:
-  ~Uploader();
-  // A block of `bytes` to fill, then send() it to dst on stream s.
-  uint8_t* begin(size_t bytes);
-  void send(void* dst, size_t bytes, hipStream_t s);
-  // Lets go of both blocks; their copies are done.
-  void release() {
-    for (PinnedLease& b : buf_) b.release();
-    busy_[0] = busy_[1] = false;
-  }
-
- private:
-  PinnedLease buf_[2];
-  hipEvent_t ev_[2] = {nullptr, nullptr};
-  bool busy_[2] = {false, false};
-  int at_ = 0;
-};
 
 struct ProfRec {
   std::string name;
