@@ -4,49 +4,59 @@
 #include <algorithm>
 #include <exception>
 #include <mutex>
-#include <vector>
 
 namespace qr {
 
 // ---- pinned host memory -------------------------------------------------------------------
 namespace {
-constexpr size_t kPinnedKeep = 8, kPinnedBytes = 64ull << 20;
+constexpr size_t kKeep = 8, kPinnedBytes = 64ull << 20;
 struct PinnedBlock {
   void* p;
   size_t cap;
 };
 std::mutex g_pin_mu;
-std::vector<PinnedBlock> g_pinned;  // kept blocks, none in use
 uint64_t g_pin_states = 0;
 
-// Adds a block to the kept ones and takes out the smallest until no more than `keep` of at most
-// `bytes` are left (a large block is the one that costs most to make again); returns those.
+// Blocks nobody holds, at most kKeep of them between calls. Nothing here allocates: blocks come back
+// in destructors.
 template <class Block>
-std::vector<Block> keep_block(std::vector<Block>& kept, const Block& b, size_t keep, size_t bytes) {
-  std::vector<Block> drop;
-  if (b.cap > bytes) {
-    drop.push_back(b);
-    return drop;
+struct Kept {
+  Block block[kKeep + 1];
+  size_t count = 0, held = 0;
+  void take_out(size_t i) {
+    held -= block[i].cap;
+    block[i] = block[--count];
   }
-  kept.push_back(b);
-  size_t held = 0;
-  for (const Block& x : kept) held += x.cap;
-  while (kept.size() > keep || held > bytes) {
-    auto least = std::min_element(kept.begin(), kept.end(), [](const Block& x, const Block& y) { return x.cap < y.cap; });
-    held -= least->cap;
-    drop.push_back(*least);
-    kept.erase(least);
+  void add(const Block& b) {  // count <= kKeep
+    block[count++] = b;
+    held += b.cap;
   }
-  return drop;
-}
+  // Takes out blocks until no more than kKeep of at most `bytes` are left, the smallest first (a large
+  // block is the one that costs most to make again), or the largest first where little may stay
+  // (one of them would push out all that small calls use). drop[kKeep + 1] receives them.
+  size_t trim(size_t bytes, bool largest_first, Block* drop) {
+    size_t n = 0;
+    while (count > kKeep || held > bytes) {
+      size_t out = 0;
+      for (size_t i = 1; i < count; ++i)
+        if (largest_first ? block[i].cap > block[out].cap : block[i].cap < block[out].cap) out = i;
+      drop[n++] = block[out];
+      take_out(out);
+    }
+    return n;
+  }
+};
+Kept<PinnedBlock> g_pinned;
 
 void pinned_give_back(void* p, size_t cap) {
-  std::vector<PinnedBlock> drop;
-  {
+  PinnedBlock drop[kKeep + 1] = {{p, cap}};
+  size_t n = 1;
+  if (cap <= kPinnedBytes) {
     std::lock_guard<std::mutex> lk(g_pin_mu);
-    drop = keep_block(g_pinned, PinnedBlock{p, cap}, kPinnedKeep, kPinnedBytes);
+    g_pinned.add(drop[0]);
+    n = g_pinned.trim(kPinnedBytes, false, drop);
   }
-  for (const PinnedBlock& b : drop) (void)hipHostFree(b.p);
+  for (size_t i = 0; i < n; ++i) (void)hipHostFree(drop[i].p);
 }
 }  // namespace
 
@@ -62,13 +72,14 @@ void PinnedLease::reserve(size_t bytes) {
   cap_ = 0;
   {
     std::lock_guard<std::mutex> lk(g_pin_mu);
-    size_t best = g_pinned.size();
-    for (size_t i = 0; i < g_pinned.size(); ++i)
-      if (g_pinned[i].cap >= bytes && (best == g_pinned.size() || g_pinned[i].cap < g_pinned[best].cap)) best = i;
-    if (best < g_pinned.size()) {
-      p_ = g_pinned[best].p;
-      cap_ = g_pinned[best].cap;
-      g_pinned.erase(g_pinned.begin() + best);
+    size_t best = g_pinned.count;
+    for (size_t i = 0; i < g_pinned.count; ++i)
+      if (g_pinned.block[i].cap >= bytes && (best == g_pinned.count || g_pinned.block[i].cap < g_pinned.block[best].cap))
+        best = i;
+    if (best < g_pinned.count) {
+      p_ = g_pinned.block[best].p;
+      cap_ = g_pinned.block[best].cap;
+      g_pinned.take_out(best);
       return;
     }
   }
@@ -89,41 +100,43 @@ void PinnedLease::release() {
 
 // ---- device memory kept between calls -----------------------------------------------------
 namespace {
-constexpr size_t kDeviceKeep = 8, kDeviceBytes = 256ull << 20;
+constexpr size_t kDeviceBytes = 256ull << 20;
 struct DeviceBlock {
   void* p;
   size_t cap;
   int device;
 };
 std::mutex g_dev_mu;
-std::vector<DeviceBlock> g_device_blocks;  // kept blocks, none in use
+Kept<DeviceBlock> g_device_blocks;
 }  // namespace
 
 void pinned_state_destroyed() {
-  std::vector<PinnedBlock> drop;
-  std::vector<DeviceBlock> drop_dev;
+  PinnedBlock drop[kKeep + 1];
+  DeviceBlock drop_dev[kKeep + 1];
+  size_t n = 0, nd = 0;
   {
     std::scoped_lock lk(g_pin_mu, g_dev_mu);
     if (--g_pin_states == 0) {
-      drop.swap(g_pinned);
-      drop_dev.swap(g_device_blocks);
+      n = g_pinned.trim(kPinnedIdleBytes, true, drop);
+      nd = g_device_blocks.trim(0, true, drop_dev);
     }
   }
-  for (const PinnedBlock& b : drop) (void)hipHostFree(b.p);
-  for (const DeviceBlock& b : drop_dev) (void)hipFree(b.p);
+  for (size_t i = 0; i < n; ++i) (void)hipHostFree(drop[i].p);
+  for (size_t i = 0; i < nd; ++i) (void)hipFree(drop_dev[i].p);
 }
 
 hipError_t device_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory && e != hipErrorMemoryAllocation) return e;
-  std::vector<DeviceBlock> drop;
+  DeviceBlock drop[kKeep + 1];
+  size_t n = 0;
   {
     std::lock_guard<std::mutex> lk(g_dev_mu);
-    drop.swap(g_device_blocks);
+    n = g_device_blocks.trim(0, true, drop);
   }
-  if (drop.empty()) return e;
+  if (n == 0) return e;
   (void)hipGetLastError();
-  for (const DeviceBlock& b : drop) (void)hipFree(b.p);
+  for (size_t i = 0; i < n; ++i) (void)hipFree(drop[i].p);
   return hipMalloc(p, bytes);
 }
 
@@ -133,16 +146,17 @@ void DeviceLease::reserve(size_t bytes) {
   hip_check(hipGetDevice(&device_), "hipGetDevice");
   {
     std::lock_guard<std::mutex> lk(g_dev_mu);
-    size_t best = g_device_blocks.size();
-    for (size_t i = 0; i < g_device_blocks.size(); ++i) {
-      const DeviceBlock& b = g_device_blocks[i];
-      if (b.device == device_ && b.cap >= bytes && (best == g_device_blocks.size() || b.cap < g_device_blocks[best].cap))
+    size_t best = g_device_blocks.count;
+    for (size_t i = 0; i < g_device_blocks.count; ++i) {
+      const DeviceBlock& b = g_device_blocks.block[i];
+      if (b.device == device_ && b.cap >= bytes &&
+          (best == g_device_blocks.count || b.cap < g_device_blocks.block[best].cap))
         best = i;
     }
-    if (best < g_device_blocks.size()) {
-      p = g_device_blocks[best].p;
-      cap_ = g_device_blocks[best].cap;
-      g_device_blocks.erase(g_device_blocks.begin() + best);
+    if (best < g_device_blocks.count) {
+      p = g_device_blocks.block[best].p;
+      cap_ = g_device_blocks.block[best].cap;
+      g_device_blocks.take_out(best);
       return;
     }
   }
@@ -155,12 +169,14 @@ void DeviceLease::reserve(size_t bytes) {
 
 void DeviceLease::release() {
   if (!p) return;
-  std::vector<DeviceBlock> drop(1, DeviceBlock{p, cap_, device_});
-  if (!std::uncaught_exceptions()) {  // after an error, hipFree waits for what may still run
+  DeviceBlock drop[kKeep + 1] = {{p, cap_, device_}};
+  size_t n = 1;
+  if (cap_ <= kDeviceBytes && !std::uncaught_exceptions()) {  // after an error, hipFree waits for what may still run
     std::lock_guard<std::mutex> lk(g_dev_mu);
-    drop = keep_block(g_device_blocks, drop[0], kDeviceKeep, kDeviceBytes);
+    g_device_blocks.add(drop[0]);
+    n = g_device_blocks.trim(kDeviceBytes, false, drop);
   }
-  for (const DeviceBlock& b : drop) (void)hipFree(b.p);
+  for (size_t i = 0; i < n; ++i) (void)hipFree(drop[i].p);
   p = nullptr;
   cap_ = 0;
 }
