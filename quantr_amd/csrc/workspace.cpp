@@ -51,10 +51,14 @@ Kept<PinnedBlock> g_pinned;
 void pinned_give_back(void* p, size_t cap) {
   PinnedBlock drop[kKeep + 1] = {{p, cap}};
   size_t n = 1;
-  if (cap <= kPinnedBytes) {
+  {
     std::lock_guard<std::mutex> lk(g_pin_mu);
-    g_pinned.add(drop[0]);
-    n = g_pinned.trim(kPinnedBytes, false, drop);
+    const bool idle = g_pin_states == 0;
+    const size_t most = idle ? kPinnedIdleBytes : kPinnedBytes;
+    if (cap <= most) {
+      g_pinned.add(drop[0]);
+      n = g_pinned.trim(most, idle, drop);
+    }
   }
   for (size_t i = 0; i < n; ++i) (void)hipHostFree(drop[i].p);
 }
@@ -118,7 +122,7 @@ void pinned_state_destroyed() {
     std::scoped_lock lk(g_pin_mu, g_dev_mu);
     if (--g_pin_states == 0) {
       n = g_pinned.trim(kPinnedIdleBytes, true, drop);
-      nd = g_device_blocks.trim(0, true, drop_dev);
+      nd = g_device_blocks.trim(kDeviceIdleBytes, true, drop_dev);
     }
   }
   for (size_t i = 0; i < n; ++i) (void)hipHostFree(drop[i].p);
@@ -171,10 +175,14 @@ void DeviceLease::release() {
   if (!p) return;
   DeviceBlock drop[kKeep + 1] = {{p, cap_, device_}};
   size_t n = 1;
-  if (cap_ <= kDeviceBytes && !std::uncaught_exceptions()) {  // after an error, hipFree waits for what may still run
-    std::lock_guard<std::mutex> lk(g_dev_mu);
-    g_device_blocks.add(drop[0]);
-    n = g_device_blocks.trim(kDeviceBytes, false, drop);
+  if (!std::uncaught_exceptions()) {  // after an error, hipFree waits for what may still run
+    std::scoped_lock lk(g_pin_mu, g_dev_mu);
+    const bool idle = g_pin_states == 0;
+    const size_t most = idle ? kDeviceIdleBytes : kDeviceBytes;
+    if (cap_ <= most) {
+      g_device_blocks.add(drop[0]);
+      n = g_device_blocks.trim(most, idle, drop);
+    }
   }
   for (size_t i = 0; i < n; ++i) (void)hipFree(drop[i].p);
   p = nullptr;

@@ -63,6 +63,33 @@ void state_per_circuit() {
   expect(pinned.calls == after, "a large call pushed out the blocks of small ones");
 }
 
+// A call without a state (re-simulated shots) keeps no more than the idle bounds, also where the
+// last state went while it ran, and with a state alive its blocks are still there.
+void call_without_a_state() {
+  auto call = [] {
+    PinnedLease host(20u << 20), small(1000);
+    DeviceLease states, tables;
+    states.reserve(100u << 20);
+    tables.reserve(100000);
+  };
+  call();
+  expect(pinned.held <= kPinnedIdleBytes, "pinned blocks stay without a state");
+  expect(device.held <= kDeviceIdleBytes, "device blocks stay without a state");
+  pinned_state_created();
+  call();
+  const size_t calls = pinned.calls + device.calls;
+  call();
+  expect(pinned.calls + device.calls == calls, "blocks allocated anew while a state lives");
+  {
+    DeviceLease d;
+    d.reserve(100u << 20);
+    PinnedLease p(20u << 20);
+    pinned_state_destroyed();
+  }
+  expect(pinned.held <= kPinnedIdleBytes, "pinned blocks stay after the last state");
+  expect(device.held <= kDeviceIdleBytes, "device blocks stay after the last state");
+}
+
 }  // namespace
 
 extern "C" {
@@ -87,7 +114,7 @@ int main(int argc, char** argv) {
   struct {
     const char* name;
     void (*run)();
-  } const checks[] = {{"state_per_circuit", state_per_circuit}};
+  } const checks[] = {{"state_per_circuit", state_per_circuit}, {"call_without_a_state", call_without_a_state}};
   for (const auto& c : checks)
     if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
       c.run();
