@@ -138,10 +138,12 @@ hipError_t device_malloc(void** p, size_t bytes) {
     std::lock_guard<std::mutex> lk(g_dev_mu);
     n = g_device_blocks.trim(0, true, drop);
   }
+  (void)hipGetLastError();  // it is returned, not left for the check of the next launch
   if (n == 0) return e;
-  (void)hipGetLastError();
   for (size_t i = 0; i < n; ++i) (void)hipFree(drop[i].p);
-  return hipMalloc(p, bytes);
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 void DeviceLease::reserve(size_t bytes) {
@@ -167,7 +169,13 @@ void DeviceLease::reserve(size_t bytes) {
   size_t want = 1 << 16;
   while (want < bytes && want < kDeviceBytes) want *= 2;
   want = std::max(want, bytes);
-  hip_check(device_malloc(&p, want), "hipMalloc (workspace)");
+  hipError_t e = device_malloc(&p, want);
+  if (e != hipSuccess && want > bytes) {  // short of memory: no room for later calls then
+    want = bytes;
+    e = device_malloc(&p, want);
+  }
+  if (e != hipSuccess) p = nullptr;
+  hip_check(e, "hipMalloc (workspace)");
   cap_ = want;
 }
 

@@ -11,13 +11,15 @@ using namespace qr;
 
 namespace {
 
+hipError_t last_error = hipSuccess;
+
 struct Memory {
   std::map<void*, size_t> live;
   size_t held = 0, calls = 0;
   size_t limit = ~size_t(0);
   hipError_t get(void** p, size_t bytes) {
     ++calls;
-    if (bytes > limit - held) return hipErrorOutOfMemory;
+    if (bytes > limit - held) return last_error = hipErrorOutOfMemory;
     *p = std::malloc(bytes);
     live[*p] = bytes;
     held += bytes;
@@ -90,6 +92,28 @@ void call_without_a_state() {
   expect(device.held <= kDeviceIdleBytes, "device blocks stay after the last state");
 }
 
+// A workspace that fits is had, also where its rounded size doesn't fit.
+void short_of_device_memory() {
+  device.limit = 100u << 20;
+  {
+    DeviceLease a;
+    a.reserve(70u << 20);
+    expect(a.p != nullptr && device.held >= (70u << 20), "no workspace");
+    std::memset(a.p, 1, 70u << 20);
+  }
+  DeviceLease b;
+  bool refused = false;
+  try {
+    b.reserve(101u << 20);
+  } catch (const Error& e) {
+    refused = e.status == QR_ERR_OOM;
+  }
+  expect(refused, "a workspace beyond the device");
+  expect(last_error == hipSuccess, "the error is left for the next launch");
+  b.reserve(1000);
+  expect(b.p != nullptr, "no workspace after a refused one");
+}
+
 }  // namespace
 
 extern "C" {
@@ -98,7 +122,11 @@ hipError_t hipHostFree(void* p) { return pinned.put(p); }
 hipError_t hipMalloc(void** p, size_t bytes) { return device.get(p, bytes); }
 hipError_t hipFree(void* p) { return device.put(p); }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
 const char* hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipEventCreateWithFlags(hipEvent_t*, unsigned) { return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
@@ -114,7 +142,8 @@ int main(int argc, char** argv) {
   struct {
     const char* name;
     void (*run)();
-  } const checks[] = {{"state_per_circuit", state_per_circuit}, {"call_without_a_state", call_without_a_state}};
+  } const checks[] = {{"state_per_circuit", state_per_circuit}, {"call_without_a_state", call_without_a_state},
+                {"short_of_device_memory", short_of_device_memory}};
   for (const auto& c : checks)
     if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
       c.run();

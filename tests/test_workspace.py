@@ -19,7 +19,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["state_per_circuit", "call_without_a_state"])
+@pytest.mark.parametrize("check", ["state_per_circuit", "call_without_a_state", "short_of_device_memory"])
 def test_kept_blocks(exe, check):
     r = subprocess.run([exe, check], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
