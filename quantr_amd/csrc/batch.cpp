@@ -327,7 +327,7 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
     }
   const size_t init_at = blob_size = align_up(blob_size, kAlign);
   blob_size += init_base.size() * (sizeof(uint64_t) + sizeof(uint32_t));
-  b->host_blob.reserve(std::max<size_t>(blob_size, 1));
+  b->host_blob.reserve_for_copies(std::max<size_t>(blob_size, 1));
   b->host_blob_size = blob_size;
   for (Inst& I : b->inst) {  // standalone and observable tables (fixed for the batch's lifetime)
     std::memcpy(b->host_blob.data() + I.blob_f, I.pf->image.bytes.data(), I.pf->image.live);
@@ -441,7 +441,8 @@ void batch_run(qr_batch* b, const qr_program* programs, double* expvals, double*
   hip_check(hipGraphLaunch(b->exec, b->origin), "hipGraphLaunch");
   // results and stamps lie in one buffer: one copy
   const size_t stamp_off = align_up((m + b->total_params) * sizeof(double), kAlign);
-  PinnedLease pin(stamp_off + (m + 1) * sizeof(uint64_t));
+  PinnedLease pin;
+  pin.reserve_for_copies(stamp_off + (m + 1) * sizeof(uint64_t));
   const double* h = (const double*)pin.data();
   const uint64_t* st = (const uint64_t*)(pin.data() + stamp_off);
   hip_check(hipMemcpyAsync(pin.data(), b->out.p, stamp_off + (m + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, b->origin),

@@ -268,23 +268,34 @@ void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vec
     }
     d = last;
   }
-  if (jobs.empty()) return;
-  const size_t ub = shots * 8, jb = jobs.size() * sizeof(ExactJob);
-  PinnedLease pin_jobs(2 * ub + jb);
-  uint64_t* got = (uint64_t*)(pin_jobs.data() + ub + jb);
-  std::memcpy(pin_jobs.data(), us.data(), ub);
-  std::memcpy(pin_jobs.data() + ub, jobs.data(), jb);
-  st->aux.reserve(ub + jb);
-  const uint8_t* dblob = (const uint8_t*)st->aux.p;
-  hip_check(hipMemcpyAsync(st->aux.p, pin_jobs.data(), ub + jb, hipMemcpyHostToDevice, st->stream), "H2D");
-  {
-    ProfScope ps_(st, "sample_exact_blocks", (double)jobs.size() * (double)len * st->bytes_per_amp());
-    hip_check(launch_sample_exact_blocks(st->prec, st->amp, st->dim, bb, (const ExactJob*)(dblob + ub), jobs.size(),
-                                         (const double*)dblob, got, st->stream),
-              "sample exact blocks");
+  // a slice of the jobs at a time: their draws (and those between them) and bins are pinned
+  for (size_t j0 = 0, j1; j0 < jobs.size(); j0 = j1) {
+    const uint64_t d0 = jobs[j0].first;
+    for (j1 = j0 + 1; j1 < jobs.size() && jobs[j1].last - d0 <= kDrawSlice && j1 - j0 < kDrawSlice / 8;) ++j1;
+    const uint64_t count = jobs[j1 - 1].last - d0;
+    const size_t ub = count * 8, jb = (j1 - j0) * sizeof(ExactJob);
+    PinnedLease pin_jobs(2 * ub + jb);
+    uint64_t* got = (uint64_t*)(pin_jobs.data() + ub + jb);
+    std::memcpy(pin_jobs.data(), us.data() + d0, ub);
+    ExactJob* up = (ExactJob*)(pin_jobs.data() + ub);
+    for (size_t j = j0; j < j1; ++j) {
+      up[j - j0] = jobs[j];
+      up[j - j0].first -= d0;
+      up[j - j0].last -= d0;
+    }
+    st->aux.reserve(ub + jb);
+    const uint8_t* dblob = (const uint8_t*)st->aux.p;
+    hip_check(hipMemcpyAsync(st->aux.p, pin_jobs.data(), ub + jb, hipMemcpyHostToDevice, st->stream), "H2D");
+    {
+      ProfScope ps_(st, "sample_exact_blocks", (double)(j1 - j0) * (double)len * st->bytes_per_amp());
+      hip_check(launch_sample_exact_blocks(st->prec, st->amp, st->dim, bb, (const ExactJob*)(dblob + ub), j1 - j0,
+                                           (const double*)dblob, got, st->stream),
+                "sample exact blocks");
+    }
+    hip_check(hipStreamSynchronize(st->stream), "sync");
+    for (size_t j = j0; j < j1; ++j)
+      std::copy(got + (jobs[j].first - d0), got + (jobs[j].last - d0), res.begin() + jobs[j].first);
   }
-  hip_check(hipStreamSynchronize(st->stream), "sync");
-  for (const ExactJob& j : jobs) std::copy(got + j.first, got + j.last, res.begin() + j.first);
 }
 
 }  // namespace qr

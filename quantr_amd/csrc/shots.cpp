@@ -104,9 +104,9 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
     for (size_t c0 = 0; c0 < members.size(); c0 += per_chunk) {
       const uint64_t cnt = std::min<uint64_t>(per_chunk, members.size() - c0);
       // coefficient blobs of the chunk's programs, back to back (same layout: same plan)
-      host.reserve(std::max<size_t>(cnt * blob_stride, 1));
+      host.reserve_for_copies(std::max<size_t>(cnt * blob_stride, 1));
       parallel_for(cnt, [&](uint64_t y) {
-        std::memcpy(host.data() + y * blob_stride, cp->image.bytes.data(), blob_size);
+        if (blob_size) std::memcpy(host.data() + y * blob_stride, cp->image.bytes.data(), blob_size);
         write_values(pr[members[c0 + y]].ops, stages, loc, host.data() + y * blob_stride);
       });
       blobs.reserve(std::max<size_t>(cnt * blob_stride, 1));
@@ -144,23 +144,25 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
         }
         off[y + 1] = uu.size();
       }
-      if (!uu.empty()) {
-        // draws and offsets go up in one copy; the bins are written to pinned memory
-        const size_t ub = uu.size() * sizeof(double), ob = off.size() * sizeof(uint64_t);
+      // a slice of the draws at a time: draws and offsets go up in one copy, the bins are written to
+      // pinned memory
+      for (uint64_t d0 = 0; d0 < uu.size(); d0 += kDrawSlice) {
+        const uint64_t d1 = std::min<uint64_t>(uu.size(), d0 + kDrawSlice);
+        const size_t ub = (d1 - d0) * sizeof(double), ob = off.size() * sizeof(uint64_t);
         small.reserve(2 * ub + ob);
-        std::memcpy(small.data(), uu.data(), ub);
-        std::memcpy(small.data() + ub, off.data(), ob);
-        const uint64_t* got = (const uint64_t*)(small.data() + ub + ob);
+        std::memcpy(small.data(), uu.data() + d0, ub);
+        uint64_t* part = (uint64_t*)(small.data() + ub);
+        for (size_t y = 0; y < off.size(); ++y) part[y] = std::min(std::max(off[y], d0), d1) - d0;
+        uint64_t* got = part + off.size();
         draws_dev.reserve(ub + ob);
         hip_check(hipMemcpyAsync(draws_dev.p, small.data(), ub + ob, hipMemcpyHostToDevice, s), "H2D");
         hip_check(launch_sample_fold_instances(prec, states.p, dim, cnt, (const double*)draws_dev.p,
-                                               (const uint64_t*)((const uint8_t*)draws_dev.p + ub), (uint64_t*)got, s),
+                                               (const uint64_t*)((const uint8_t*)draws_dev.p + ub), got, s),
                   "sample fold (programs)");
         hip_check(hipStreamSynchronize(s), "sync");
-        for (size_t q = 0; q < uu.size(); ++q) out[perm[q]] = got[q];
-      } else {
-        hip_check(hipStreamSynchronize(s), "sync");
+        for (uint64_t q = d0; q < d1; ++q) out[perm[q]] = got[q - d0];
       }
+      if (uu.empty()) hip_check(hipStreamSynchronize(s), "sync");
     }
   }
 }

@@ -2,14 +2,16 @@
 #include "workspace.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 #include <exception>
 #include <mutex>
+#include <new>
 
 namespace qr {
 
 // ---- pinned host memory -------------------------------------------------------------------
 namespace {
-constexpr size_t kKeep = 8, kPinnedBytes = 64ull << 20;
+constexpr size_t kKeep = 8;
 struct PinnedBlock {
   void* p;
   size_t cap;
@@ -70,10 +72,8 @@ void pinned_state_created() {
 }
 
 void PinnedLease::reserve(size_t bytes) {
-  if (bytes <= cap_) return;
-  if (p_) pinned_give_back(p_, cap_);
-  p_ = nullptr;
-  cap_ = 0;
+  if (bytes <= cap_ && !plain_) return;
+  release();
   {
     std::lock_guard<std::mutex> lk(g_pin_mu);
     size_t best = g_pinned.count;
@@ -87,19 +87,61 @@ void PinnedLease::reserve(size_t bytes) {
       return;
     }
   }
+  // rounded, so that calls of about one size share a block: to a power of two, from 4 MB on to whole MB
+  constexpr size_t MB = 1 << 20;
   size_t want = 1 << 16;
-  while (want < bytes) want *= 2;
-  hip_check(hipHostMalloc(&p_, want, hipHostMallocPortable | hipHostMallocCoherent), "hipHostMalloc");
+  while (want < bytes && want < 4 * MB) want *= 2;
+  if (want < bytes) want = (bytes + MB - 1) / MB * MB;
+  hipError_t e = hipHostMalloc(&p_, want, hipHostMallocPortable | hipHostMallocCoherent);
+  if (e != hipSuccess) {  // without the blocks nobody holds, and no more than is asked for
+    (void)hipGetLastError();
+    PinnedBlock drop[kKeep + 1];
+    size_t n = 0;
+    {
+      std::lock_guard<std::mutex> lk(g_pin_mu);
+      n = g_pinned.trim(0, true, drop);
+    }
+    for (size_t i = 0; i < n; ++i) (void)hipHostFree(drop[i].p);
+    want = bytes;
+    e = hipHostMalloc(&p_, want, hipHostMallocPortable | hipHostMallocCoherent);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      p_ = nullptr;
+    }
+  }
+  hip_check(e, "hipHostMalloc");
   cap_ = want;
+}
+
+void PinnedLease::reserve_for_copies(size_t bytes) {
+  if (bytes <= cap_) return;
+  if (bytes <= kPinnedBytes) {
+    try {
+      reserve(bytes);
+      return;
+    } catch (const Error&) {  // pinned memory is short: copies take other memory too
+    }
+  }
+  release();
+  p_ = std::malloc(bytes);
+  if (!p_) throw std::bad_alloc();
+  cap_ = bytes;
+  plain_ = true;
 }
 
 void PinnedLease::release() {
   if (!p_) return;
   // a call that ends in an error may leave work in flight on the block: hipHostFree waits for it
-  if (std::uncaught_exceptions()) (void)hipHostFree(p_);
-  else pinned_give_back(p_, cap_);
+  if (plain_) {
+    if (std::uncaught_exceptions()) (void)hipDeviceSynchronize();
+    std::free(p_);
+  } else if (std::uncaught_exceptions())
+    (void)hipHostFree(p_);
+  else
+    pinned_give_back(p_, cap_);
   p_ = nullptr;
   cap_ = 0;
+  plain_ = false;
 }
 
 // ---- device memory kept between calls -----------------------------------------------------
@@ -208,7 +250,7 @@ uint8_t* Uploader::begin(size_t bytes) {
   at_ ^= 1;
   if (busy_[at_]) hip_check(hipEventSynchronize(ev_[at_]), "hipEventSynchronize");
   busy_[at_] = false;
-  buf_[at_].reserve(std::max<size_t>(bytes, 1));
+  buf_[at_].reserve_for_copies(std::max<size_t>(bytes, 1));
   return buf_[at_].data();
 }
 

@@ -64,11 +64,13 @@ struct DevBuf {
 
 // A block of pinned host memory, which kernels and copies reach directly, held for one call.
 // Blocks are kept for later calls (pinning a new one takes longer than a small call): at most 8 of
-// them and 64 MB, or kPinnedIdleBytes while no state or batch lives: programs that make a state for
+// them and kPinnedBytes, or kPinnedIdleBytes while no state or batch lives: programs that make a state for
 // each circuit would else pin and free its blocks every time (create, apply, 500 draws, destroy,
 // complex128, 10 / 16 / 20 qubits: 147 / 412 / 510 us without them, 112 / 256 / 355 with; an
 // expectation in place of the draws, 12 qubits: 360 and 256).
-constexpr size_t kPinnedIdleBytes = 4ull << 20;
+// Nor is more pinned for a call's data: draws are taken in slices, and blocks that only copies reach
+// are ordinary memory beyond kPinnedBytes.
+constexpr size_t kPinnedBytes = 64ull << 20, kPinnedIdleBytes = 4ull << 20;
 class PinnedLease {
  public:
   PinnedLease() = default;
@@ -77,18 +79,22 @@ class PinnedLease {
   PinnedLease(const PinnedLease&) = delete;
   PinnedLease& operator=(const PinnedLease&) = delete;
   void reserve(size_t bytes);  // at least this size; what it held is lost
-  void release();              // back to the kept blocks
+  // The same for a block that only copies reach: ordinary memory beyond kPinnedBytes, and where no
+  // more can be pinned.
+  void reserve_for_copies(size_t bytes);
+  void release();  // back to the kept blocks
   uint8_t* data() const { return (uint8_t*)p_; }
 
  private:
   void* p_ = nullptr;
   size_t cap_ = 0;
+  bool plain_ = false;  // ordinary memory
 };
 void pinned_state_created();    // one more state or batch lives
 void pinned_state_destroyed();  // one less; the last one, its own blocks let go of, leaves the idle bounds
 
-// Uploads of small host data onto a stream without waiting for it: two pinned blocks in turn, each
-// reused once its last copy is done. The owner's stream is idle before it is destroyed.
+// Uploads of host data onto a stream without waiting for it: two blocks in turn, each reused once its
+// last copy is done. The owner's stream is idle before it is destroyed.
 class Uploader {
  public:
   ~Uploader();

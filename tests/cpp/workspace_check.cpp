@@ -1,38 +1,17 @@
 // workspace_check.cpp — the blocks kept between calls (workspace.cpp) over a HIP runtime of stubs
 // that counts what is allocated; no GPU is used. The argument names the check.
 #include <cstdio>
-#include <cstdlib>
 #include <cstring>
-#include <map>
 
+#include "hip_stubs.hpp"
 #include "workspace.hpp"
 
 using namespace qr;
+using stub::device;
+using stub::last_error;
+using stub::pinned;
 
 namespace {
-
-hipError_t last_error = hipSuccess;
-
-struct Memory {
-  std::map<void*, size_t> live;
-  size_t held = 0, calls = 0;
-  size_t limit = ~size_t(0);
-  hipError_t get(void** p, size_t bytes) {
-    ++calls;
-    if (bytes > limit - held) return last_error = hipErrorOutOfMemory;
-    *p = std::malloc(bytes);
-    live[*p] = bytes;
-    held += bytes;
-    return hipSuccess;
-  }
-  hipError_t put(void* p) {
-    if (!live.count(p)) return hipErrorInvalidValue;
-    held -= live[p];
-    live.erase(p);
-    std::free(p);
-    return hipSuccess;
-  }
-} pinned, device;
 
 int failures = 0;
 void expect(bool ok, const char* what) {
@@ -114,36 +93,48 @@ void short_of_device_memory() {
   expect(b.p != nullptr, "no workspace after a refused one");
 }
 
-}  // namespace
+// Uploads beyond the pinned bound, or where nothing can be pinned, take ordinary memory.
+void large_uploads() {
+  char* dst = (char*)std::malloc(200u << 20);
+  auto send = [&](Uploader& up, size_t bytes) {
+    uint8_t* h = up.begin(bytes);
+    std::memset(h, 7, bytes);
+    dst[bytes - 1] = 0;
+    up.send(dst, bytes, nullptr);
+    expect(dst[bytes - 1] == 7, "the upload's data");
+  };
+  {
+    Uploader up;
+    for (size_t bytes : {100u, 200u << 20, 200u << 20, 3u << 20, 200u << 20}) send(up, bytes);
+    expect(pinned.largest <= kPinnedBytes, "more than the bound is pinned");
+  }
+  pinned.limit = pinned.held;
+  {
+    Uploader up;
+    send(up, 50u << 20);
+    send(up, 10);
+  }
+  PinnedLease kernel;
+  bool refused = false;
+  try {
+    kernel.reserve(50u << 20);
+  } catch (const Error&) {
+    refused = true;
+  }
+  expect(refused && last_error == hipSuccess, "what kernels write must be pinned");
+  pinned.limit = ~size_t(0);
+  std::free(dst);
+}
 
-extern "C" {
-hipError_t hipHostMalloc(void** p, size_t bytes, unsigned int) { return pinned.get(p, bytes); }
-hipError_t hipHostFree(void* p) { return pinned.put(p); }
-hipError_t hipMalloc(void** p, size_t bytes) { return device.get(p, bytes); }
-hipError_t hipFree(void* p) { return device.put(p); }
-hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
-hipError_t hipGetLastError() {
-  const hipError_t e = last_error;
-  last_error = hipSuccess;
-  return e;
-}
-const char* hipGetErrorString(hipError_t) { return "stub"; }
-hipError_t hipEventCreateWithFlags(hipEvent_t*, unsigned) { return hipSuccess; }
-hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind, hipStream_t) {
-  std::memcpy(d, s, bytes);
-  return hipSuccess;
-}
-}
+}  // namespace
 
 int main(int argc, char** argv) {
   struct {
     const char* name;
     void (*run)();
   } const checks[] = {{"state_per_circuit", state_per_circuit}, {"call_without_a_state", call_without_a_state},
-                {"short_of_device_memory", short_of_device_memory}};
+                {"short_of_device_memory", short_of_device_memory},
+                {"large_uploads", large_uploads}};
   for (const auto& c : checks)
     if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
       c.run();
