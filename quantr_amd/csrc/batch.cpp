@@ -104,15 +104,6 @@ PlanParams fwd_params(uint32_t n, int prec, int k = 0) {
   return pp;
 }
 
-PlanParams dual_params(uint32_t n, int prec, int k = 0) {
-  PlanParams pp;
-  pp.tile_bits = std::min<int>(k ? k : (prec == 0 ? 10 : 11), (int)n);
-  pp.reg_bits = dual_reg_bits(pp.tile_bits);  // 32 instances of 10..18 qubits: 2.65 -> 2.50 ms per run
-  pp.low_bits = prec == 0 ? 3 : 4;
-  if (pp.tile_bits == (int)n) pp.max_ops = kWholeStateStageOps;
-  return pp;
-}
-
 // Lowers one instance's program (forward ops and the reverse-sweep ops).
 void lower_instance(Inst& I, const qr_program* prog) {
   validate_program(I.n, prog);
@@ -253,7 +244,7 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
     I.key = structure_key(I.fwd);
     I.terms = parse_observable(I.n, &observables[i]);
     I.ppf = fwd_params(I.n, b->prec, widths[i].fwd);
-    I.ppb = dual_params(I.n, b->prec, widths[i].dual);
+    I.ppb = dual_plan_params(I.n, b->prec, widths[i].dual, 0);
     I.pf = get_plan_for(I.n, b->prec, I.fwd, I.ppf, true, false, false);
     I.pb = get_plan_for(I.n, b->prec, I.rev, I.ppb, true, true, false);
     for (const auto& op : I.fwd)
@@ -513,7 +504,7 @@ void autotune_widths(uint64_t m, const uint32_t* nq, const qr_program* programs,
         }
       }
       for (int k : cands(def_d, n, tune_dual ? 0 : widths[i].dual)) {
-        const PlanParams pp = dual_params(n, prec, k);
+        const PlanParams pp = dual_plan_params(n, prec, k, 0);
         auto cp = get_plan_for(n, prec, I.rev, pp, true, true, false);
         if (cp->fns.empty()) {
           auto src = jit_stage_sources(cp->stages, prec, pp.reg_bits, false, true);

@@ -284,6 +284,11 @@ std::vector<Stage> plan_fused_balanced(uint32_t n, const std::vector<FastOp>& op
 std::vector<std::vector<Stage>> plan_fused_candidates(uint32_t n, const std::vector<FastOp>& ops,
                                                      const PlanParams& pp, int bytes_per_amp, bool dual,
                                                      int count, std::vector<PlanParams>* chosen = nullptr);
+// Planning parameters of a reverse sweep (psi and lam per tile) of n qubits, precision prec
+// (0 = complex128), with tiles of tile_bits (0 = the default). simds: the SIMDs of a device that has
+// this gradient to itself; 0 for an instance of a batch, which shares it.
+PlanParams dual_plan_params(uint32_t n, int prec, int tile_bits, uint64_t simds);
+
 // Appends what the planner's output depends on for one op (kind, bits, controls and the
 // value-derived forms), so that programs with equal keys share one plan; coefficients are
 // then taken from each program's own ops (TileOpHost::src).

@@ -354,6 +354,34 @@ int choose_split_pos(int k, int nts, const std::vector<int>& om, const std::vect
 
 }  // namespace
 
+// Psi and lam share a workgroup, so tiles are half the width of the forward sweep's: 2^10 complex128 /
+// 2^11 complex64 amplitudes. A complex64 gradient of up to 18 qubits alone takes 2^10, which gives
+// twice the workgroups; in a batch the instances fill the chip together and the wider tile is the
+// faster one (32 instances, 12..14 / 17..18 / 10..18 qubits: 2.52 / 4.05 / 3.07 ms with 2^10, 2.49 /
+// 3.81 / 2.95 with 2^11).
+// Register bits: as many as leave a whole wavefront of threads (taps are then summed through LDS), 3
+// at most below the widest tiles. Reverse sweeps of 7 / 8 / 9 qubits, complex128, 115 / 125 / 190 us
+// with 4 bits, 89 / 86 / 97 with 1 / 2 / 3; 32 instances of 10..18 qubits 2.65 -> 2.50 ms. With 3, a
+// wavefront's straight-line code (fetched once, from a cold instruction cache) is half as long and
+// twice as many of them hide each other's waits, which pays for the exchanges of the fourth register
+// bit; us per reverse sweep with 4 / with 3: complex128 at 10, 16, 19, 21, 22 qubits 121/108,
+// 190/179, 339/309, 664/632, 1130/1039; complex64 at 13, 17, 20, 22 qubits 178/146, 226/189, 376/334,
+// 883/797. The exception is a complex128 gradient alone that gives every SIMD of the device exactly
+// one wavefront with 4 bits (20 qubits on 1024 SIMDs: 578 with 4, 630 with 3), in tiles of at least
+// a wavefront then.
+PlanParams dual_plan_params(uint32_t n, int prec, int tile_bits, uint64_t simds) {
+  PlanParams pp;
+  const int k = tile_bits ? tile_bits : prec == 0 || (simds && n <= 18) ? 10 : 11;
+  pp.tile_bits = std::min(k, (int)n);
+  if (pp.tile_bits >= 12) pp.reg_bits = 4;
+  else pp.reg_bits = pp.tile_bits >= 7 ? std::min(3, pp.tile_bits - 6) : std::min(2, pp.tile_bits);
+  constexpr uint64_t kWave = 64, kRegs = 16;
+  if (prec == 0 && (1ull << n) == simds * kWave * kRegs && (1ull << pp.tile_bits) >= kWave * kRegs) pp.reg_bits = 4;
+  pp.low_bits = prec == 0 ? 3 : 4;
+  if (pp.tile_bits == (int)n) pp.max_ops = kWholeStateStageOps;
+  return pp;
+}
+
 void plan_key_append(const FastOp& op, std::vector<uint64_t>& key) {
   uint64_t cls = 0;
   if (op.kind == FK_DENSE1) {

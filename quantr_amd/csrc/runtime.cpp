@@ -703,32 +703,12 @@ void apply_observable(int prec, void* lam, const void* psi, uint64_t dim, const 
             "pauli sum");
 }
 
-// As many register bits as leave a whole wavefront of threads (taps are then summed through LDS), 3
-// at most below the widest tiles: reverse sweeps of 7 / 8 / 9 qubits, complex128, 115 / 125 / 190 us
-// with 4 bits, 89 / 86 / 97 with 1 / 2 / 3.
-int dual_reg_bits(int tile_bits) {
-  if (tile_bits >= 12) return 4;
-  return tile_bits >= 7 ? std::min(3, tile_bits - 6) : std::min(2, tile_bits);
-}
-
-// Tile shape of the adjoint sweep: psi and lam share a workgroup, so tiles are half the
-// width of the forward sweep's (2^10 complex128 / 2^11 complex64 amplitudes by default; complex64
-// states of up to 18 qubits take 2^10, which gives twice the workgroups), 8 amplitudes of each
-// state per thread. A wavefront's straight-line code (fetched once, from a cold instruction cache)
-// is then half as long and twice as many of them hide each other's waits, which pays for the
-// exchanges of the fourth register bit; us per reverse sweep with 16 / with 8 per thread:
-// complex128 at 10, 16, 19, 21, 22 qubits 121/108, 190/179, 339/309, 664/632, 1130/1039; complex64
-// at 13, 17, 20, 22 qubits 178/146, 226/189, 376/334, 883/797. The exception is complex128 at 2^20
-// amplitudes, where 16 per thread give every one of the 1024 SIMDs exactly one wavefront:
-// 578 with 16, 630 with 8.
-PlanParams dual_plan_params(const qr_state* st) {
-  PlanParams pp;
-  int k = st->prec == 0 || st->n <= 18 ? 10 : 11;
-  if (st->opt.tile_bits) k = std::min<int>(tile_max_bits(st->prec), (int)st->opt.tile_bits);
-  pp.tile_bits = std::min<int>(k, (int)st->n);
-  pp.reg_bits = dual_reg_bits(pp.tile_bits);
-  if (st->prec == 0 && st->dim == 1024ull * 64 * 16) pp.reg_bits = std::min(4, pp.tile_bits);
-  pp.low_bits = st->opt.low_bits ? (int)st->opt.low_bits : (st->prec == 0 ? 3 : 4);
+PlanParams dual_plan_params(qr_state* st) {
+  if (st->cus == 0)
+    hip_check(hipDeviceGetAttribute(&st->cus, hipDeviceAttributeMultiprocessorCount, st->device), "compute units");
+  const int width = std::min<int>(tile_max_bits(st->prec), (int)st->opt.tile_bits);
+  PlanParams pp = dual_plan_params(st->n, st->prec, width, 4 * (uint64_t)st->cus);
+  if (st->opt.low_bits) pp.low_bits = (int)st->opt.low_bits;
   pp.max_ops = stage_op_limit(st, pp.tile_bits);
   return pp;
 }

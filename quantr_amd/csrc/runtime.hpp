@@ -36,6 +36,7 @@ struct qr_state {
   void* amp = nullptr;
   hipStream_t stream = nullptr;
   int device = 0;
+  int cus = 0;  // the device's compute units, once a reverse sweep has asked for them
   qr_options opt{1, 0, 0, 2, 0, 0, 2, 0, 0};
   qr::DevBuf aux;   // plan / coefficients / small uploads
   qr::DevBuf aux2;  // partial sums, sampler scratch
@@ -104,8 +105,7 @@ T* upload(qr_state* st, DevBuf& buf, const std::vector<T>& v) {
 PlanParams plan_params(const qr_state* st);       // forward sweeps
 // The same for a state of n qubits, precision prec (0 = complex128) and options opt.
 PlanParams plan_params(uint32_t n, int prec, const qr_options& opt);
-PlanParams dual_plan_params(const qr_state* st);  // adjoint sweeps (psi and lam per tile)
-int dual_reg_bits(int tile_bits);                 // register bits of adjoint tiles
+PlanParams dual_plan_params(qr_state* st);        // adjoint sweeps (psi and lam per tile)
 
 // Offsets of one stage's data in a packed plan blob.
 struct Loc {

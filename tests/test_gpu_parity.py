@@ -847,3 +847,21 @@ def test_adjoint_tap_rows(tile_bits, precision, tol):
         got.append(g.backward())
         g.close()
     assert np.max(np.abs(got[0] - got[1])) < tol * n
+
+
+def test_adjoint_one_wavefront_per_simd_widths():
+    """The size at which a complex128 gradient takes 16 amplitudes per thread (20 qubits on 1024
+    SIMDs), in tiles of half a wavefront of such threads up to two, against 8 per thread in complex128
+    at the default width: the same products in binary64, in other orders."""
+    n = 20
+    gates, _ = W.hea(n, 1, seed=33)
+    p, obs = W.to_program(gates), _capi.Observable(W.hea_observable(n))
+    got = {}
+    for tile_bits in (0, 7, 9, 10, 11):
+        g = _capi.Grad(n)
+        g.set_options(tile_bits=tile_bits)
+        g.forward(p, obs)
+        got[tile_bits] = g.backward()
+        g.close()
+    for tile_bits, grads in got.items():
+        assert np.max(np.abs(grads - got[0])) < 1e-11, tile_bits
