@@ -100,6 +100,29 @@ void many_draws_of_programs() {
   expect(stub::pinned.largest <= 24 * kDrawSlice, "pinned memory grows with the draws");
 }
 
+// Blocks that the host folds arrive together, however many have a halfway case.
+void halfway_blocks() {
+  const std::vector<double> u = draws(1000, 9);
+  std::vector<double> us;
+  std::vector<uint64_t> perm, res;
+  sort_draws(u.data(), u.size(), us, perm);
+  for (int prec : {0, 1})
+    for (uint32_t n : {16u, 20u, 22u}) {
+      qr_state st;
+      random_state(st, n, prec, n);
+      if (prec == 0 && n == 22)  // short mantissas: hundreds of blocks
+        for (uint64_t i = 0; i < 2 * st.dim; ++i) {
+          double& x = ((double*)st.amp)[i];
+          x = std::ldexp(std::rint(std::ldexp(x, 34)), -34);
+        }
+      gathers = 0;
+      sample_exact_parallel(&st, us, res);
+      expect(res == left_fold(prec, st.amp, st.dim, us), "bins of a state with halfway cases");
+      if (gathers > 2) std::printf("%zu launches, %u qubits, precision %d\n", gathers, n, prec);
+      expect(gathers <= 2, "blocks fetched one by one");
+    }
+}
+
 }  // namespace
 
 namespace qr {
@@ -211,7 +234,8 @@ int main(int argc, char** argv) {
   struct {
     const char* name;
     void (*run)();
-  } const checks[] = {{"many_draws", many_draws}, {"many_draws_of_programs", many_draws_of_programs}};
+  } const checks[] = {{"many_draws", many_draws}, {"many_draws_of_programs", many_draws_of_programs},
+                {"halfway_blocks", halfway_blocks}};
   for (const auto& c : checks)
     if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
       c.run();

@@ -851,8 +851,8 @@ def test_adjoint_tap_rows(tile_bits, precision, tol):
 
 def test_adjoint_one_wavefront_per_simd_widths():
     """The size at which a complex128 gradient takes 16 amplitudes per thread (20 qubits on 1024
-    SIMDs), in tiles of half a wavefront of such threads up to two, against 8 per thread in complex128
-    at the default width: the same products in binary64, in other orders."""
+    SIMDs), in tiles too narrow for a wavefront of such threads up to two of them, against the
+    default width: the same products in binary64, in other orders."""
     n = 20
     gates, _ = W.hea(n, 1, seed=33)
     p, obs = W.to_program(gates), _capi.Observable(W.hea_observable(n))

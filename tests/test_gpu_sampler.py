@@ -145,3 +145,26 @@ def test_draw_sorting_and_small_states(precision, n):
         st.set_options(exact_sample=1)
         assert np.array_equal(got, st.sample(draws))
     st.close()
+
+
+@pytest.mark.parametrize("precision,n,bits", [(_capi.QR_C64, 16, 0), (_capi.QR_C64, 22, 0), (_capi.QR_C128, 22, 34)])
+def test_many_halfway_blocks(precision, n, bits):
+    """States with more blocks that hold a halfway case than the exact sums leave places for: random
+    complex64 amplitudes, and complex128 ones rounded to multiples of 2^-bits."""
+    rng = np.random.default_rng(880 + n)
+    dim = 1 << n
+    psi = (rng.standard_normal(dim) + 1j * rng.standard_normal(dim)) * 2.0 ** (-0.5 * (n + 1))
+    if bits:
+        psi = (np.rint(psi.real * 2.0 ** bits) + 1j * np.rint(psi.imag * 2.0 ** bits)) * 2.0 ** -bits
+    if precision == _capi.QR_C64:
+        psi = psi.astype(np.complex64).astype(np.complex128)
+    st = _capi.State(n, precision)
+    st.set_amplitudes(psi)
+    S = left_fold(psi)
+    u = boundary_draws(S, rng, 3000)
+    say("halfway", precision, n)
+    got = st.sample(u)
+    st.close()
+    want = np.searchsorted(S, u, side="right").astype(np.uint64)
+    want[u >= S[-1]] = NONE
+    assert np.array_equal(got, want)

@@ -43,6 +43,6 @@ def test_kept_blocks(workspace, check):
     run(workspace, check)
 
 
-@pytest.mark.parametrize("check", ["many_draws", "many_draws_of_programs"])
+@pytest.mark.parametrize("check", ["many_draws", "many_draws_of_programs", "halfway_blocks"])
 def test_sampler(sampler, check):
     run(sampler, check)
