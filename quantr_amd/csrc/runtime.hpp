@@ -11,6 +11,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -201,8 +202,8 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
                      const double* u, uint64_t* out);
 double norm_sqr(qr_state* st);
 double expectation(qr_state* st, const std::vector<PauliMasks>& terms);
-// fn(i) for i in [0, count) on up to 16 of the host's cores; the error of the lowest failing i is
-// rethrown.
+// fn(i) for i in [0, count) on up to 16 of the host's cores, fewer where the system refuses threads;
+// the error of the lowest failing i is rethrown.
 template <class F>
 void parallel_for(uint64_t count, F fn) {
   const unsigned nt = (unsigned)std::min<uint64_t>(count, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
@@ -218,7 +219,11 @@ void parallel_for(uint64_t count, F fn) {
     }
   };
   std::vector<std::thread> th;
-  for (unsigned t = 1; t < nt; ++t) th.emplace_back(work);
+  th.reserve(nt);
+  try {
+    for (unsigned t = 1; t < nt; ++t) th.emplace_back(work);
+  } catch (const std::system_error&) {  // no more threads: those there are, and this one, do the work
+  }
   work();
   for (auto& t : th) t.join();
   for (auto& e : err)

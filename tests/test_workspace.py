@@ -46,3 +46,13 @@ def test_kept_blocks(workspace, check):
 @pytest.mark.parametrize("check", ["many_draws", "many_draws_of_programs", "halfway_blocks"])
 def test_sampler(sampler, check):
     run(sampler, check)
+
+
+def test_refused_threads(tmp_path):
+    """parallel_for with fewer threads than it asks for (tests/cpp/threads_check.cpp)."""
+    exe = str(tmp_path / "threads_check")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-include", "algorithm",
+                    "-I" + os.path.join(H.ROOT, "include"), "-I" + CSRC, "-I/opt/rocm/include",
+                    os.path.join(H.ROOT, "tests", "cpp", "threads_check.cpp"), "-o", exe, "-ldl", "-lpthread"], check=True)
+    r = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout
