@@ -128,7 +128,7 @@ class OpCoefs {
 struct FastOp {
   int kind = FK_DENSE1;
   int k = 1;
-  int bits[8] = {0};    // target bits, local MSB first
+  int8_t bits[16] = {0};  // target bits, local MSB first (custom gates have up to 16)
   uint64_t cmask = 0;   // control bits that must be 1
   OpCoefs m;            // DENSE1: 4 row-major; DIAG1: 2; DENSEK: dim*dim; DIAGK: dim
   int form = U1_GENERAL;

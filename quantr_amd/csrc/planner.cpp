@@ -397,12 +397,13 @@ void plan_key_append(const FastOp& op, std::vector<uint64_t>& key) {
   } else if (op.kind == FK_DENSEK) {
     cls = is_swap_perm(op) ? 1 : 0;
   }
-  uint64_t bits = 0;
-  for (int q = 0; q < op.k && q < 8; ++q) bits |= (uint64_t)(op.bits[q] & 0xFF) << (8 * q);
+  uint64_t bits[2] = {0, 0};
+  for (int q = 0; q < op.k; ++q) bits[q / 8] |= (uint64_t)(op.bits[q] & 0xFF) << (8 * (q % 8));
   key.push_back((uint64_t)op.kind | ((uint64_t)op.k << 8) | ((uint64_t)op.gen << 16) | (cls << 24) |
                 ((uint64_t)op.sub << 40));
   key.push_back(op.cmask);
-  key.push_back(bits);
+  key.push_back(bits[0]);
+  if (op.k > 8) key.push_back(bits[1]);
 }
 
 std::vector<Stage> plan_fused(uint32_t n, const std::vector<FastOp>& ops, const PlanParams& pp,

@@ -865,3 +865,29 @@ def test_adjoint_one_wavefront_per_simd_widths():
         g.close()
     for tile_bits, grads in got.items():
         assert np.max(np.abs(grads - got[0])) < 1e-11, tile_bits
+
+
+@pytest.mark.parametrize("k,diagonal", [(8, False), (9, False), (9, True), (10, True)])
+def test_wide_custom_gates_fused(k, diagonal):
+    """Custom gates on eight to ten wires in fused programs, on two sets of wires that differ in the
+    last one only (one structure must not take the other's plan), against the oracle. Each amplitude
+    is a sum of at most 2^k products of modulus at most 1."""
+    n = 12
+    rng = np.random.default_rng(940 + k)
+    st = _capi.State(n)
+    for last in (10, 11):
+        wires = [(5 * q) % 10 for q in range(k - 1)] if k <= 9 else [9, 1, 3, 5, 7, 0, 2, 4, 6]
+        wires = list(dict.fromkeys(wires))
+        while len(wires) < k - 1:
+            wires.append(next(w for w in range(10) if w not in wires))
+        images = np.diag(np.exp(1j * rng.uniform(-3, 3, 1 << k))) if diagonal else W.random_unitary(k, 50 + last).T
+        gates = W.brickwork(n, depth=3, seed=last)
+        p = H.to_program(gates + [("Custom", last, tuple(wires), 0.0, 0)] + gates[:20],
+                         {len(gates): (np.ascontiguousarray(images), np.ones(1 << k, dtype=np.uint8))})
+        say("wide custom", k, diagonal, last)
+        want = H.oracle_simulate(n, p)
+        for _ in range(2):  # interpreted, then compiled stages
+            st.reset()
+            st.apply(p)
+            assert np.max(np.abs(st.amplitudes() - want)) < TOL_FUSED
+    st.close()
