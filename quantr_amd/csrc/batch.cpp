@@ -321,8 +321,8 @@ qr_batch* batch_create_widths(uint64_t m, const uint32_t* nq, const qr_program* 
   b->host_blob.reserve_for_copies(std::max<size_t>(blob_size, 1));
   b->host_blob_size = blob_size;
   for (Inst& I : b->inst) {  // standalone and observable tables (fixed for the batch's lifetime)
-    std::memcpy(b->host_blob.data() + I.blob_f, I.pf->image.bytes.data(), I.pf->image.live);
-    std::memcpy(b->host_blob.data() + I.blob_b, I.pb->image.bytes.data(), I.pb->image.live);
+    I.pf->image.write_fixed(b->host_blob.data() + I.blob_f, I.pf->image.live);
+    I.pb->image.write_fixed(b->host_blob.data() + I.blob_b, I.pb->image.live);
     std::vector<PauliGroup> groups;
     std::vector<PauliZTerm> flat;
     pauli_tables(I.terms, groups, flat);

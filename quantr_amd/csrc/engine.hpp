@@ -298,4 +298,30 @@ void plan_key_append(const FastOp& op, std::vector<uint64_t>& key);
 void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, std::vector<cd>& c);
 void stage_coefficients(const Stage& s, const std::vector<FastOp>& ops, cd* c);  // 4 * s.ops.size() entries
 
+// ---- plan blobs (plan_image.cpp): what a plan's kernels read -------------------------------
+
+// Offsets of one stage's data in a plan's blob.
+struct Loc {
+  size_t ops = 0, maps = 0, coefs = 0, off = 0;
+};
+
+// The layout of a plan's blob and the part of it that is the same for all programs of its structure,
+// made once per plan. First what a program's values fill, [0, values): coefficients and standalone
+// tables, of which the plan keeps no copy (a dense gate on 8 wires has 1 MB). Then the standalone
+// offset tables, up to `live`, and behind them what only interpreted stages read (ops, maps, LDS
+// patterns).
+struct PlanImage {
+  std::vector<uint8_t> fixed;  // [values, size())
+  std::vector<Loc> loc;
+  size_t values = 0, live = 0;
+  size_t size() const { return values + fixed.size(); }
+  // Writes the fixed part of the blob's first `bytes` bytes (live or size()).
+  void write_fixed(uint8_t* blob, size_t bytes) const { std::copy_n(fixed.begin(), bytes - values, blob + values); }
+};
+
+PlanImage plan_image(const std::vector<FastOp>& ops, const std::vector<Stage>& stages);
+// Fills [0, values) of a blob with the values of `ops`, a program of the plan's structure.
+void write_values(const std::vector<FastOp>& ops, const std::vector<Stage>& stages, const std::vector<Loc>& loc,
+                  uint8_t* blob);
+
 }  // namespace qr

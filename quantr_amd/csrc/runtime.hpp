@@ -108,20 +108,6 @@ PlanParams plan_params(const qr_state* st);       // forward sweeps
 PlanParams plan_params(uint32_t n, int prec, const qr_options& opt);
 PlanParams dual_plan_params(qr_state* st);        // adjoint sweeps (psi and lam per tile)
 
-// Offsets of one stage's data in a packed plan blob.
-struct Loc {
-  size_t ops = 0, maps = 0, coefs = 0, off = 0;
-};
-
-// Host image of a plan's blob, made once per plan: what a program's values fill (coefficients) and
-// the standalone tables first, [0, live), then what only interpreted stages read (ops, maps, LDS
-// patterns).
-struct PlanImage {
-  std::vector<uint8_t> bytes;
-  std::vector<Loc> loc;
-  size_t live = 0;
-};
-
 // A plan's stages plus the device copy of its blob.
 struct PackedPlan {
   const std::vector<Stage>* stages = nullptr;
@@ -164,11 +150,6 @@ std::shared_ptr<CachedPlan> get_plan(const qr_state* st, const std::vector<FastO
 std::shared_ptr<CachedPlan> get_plan_for(uint32_t n, int prec, const std::vector<FastOp>& ops, const PlanParams& pp,
                                          bool fused, bool dual, bool persistent);
 void prepare_compiled(CachedPlan& cp, int prec, int RB, bool persistent, bool dual);
-// The image of a plan (its values those of `ops`, a program of the plan's structure).
-PlanImage plan_image(const std::vector<FastOp>& ops, const std::vector<Stage>& stages);
-// Writes the values of `ops` into a copy of the image's first `live` bytes.
-void write_values(const std::vector<FastOp>& ops, const std::vector<Stage>& stages, const std::vector<Loc>& loc,
-                  uint8_t* blob);
 // Uploads the plan's blob with the values of `ops` (all of it, or only its live part) to st->aux.
 void upload_plan(qr_state* st, const std::vector<FastOp>& ops, const CachedPlan& cp, bool live_only, PackedPlan& P);
 TileArgs tile_args_at(uint32_t n, const Stage& s, const uint8_t* dblob, const Loc& loc);

@@ -106,7 +106,7 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
       // coefficient blobs of the chunk's programs, back to back (same layout: same plan)
       host.reserve_for_copies(std::max<size_t>(cnt * blob_stride, 1));
       parallel_for(cnt, [&](uint64_t y) {
-        if (blob_size) std::memcpy(host.data() + y * blob_stride, cp->image.bytes.data(), blob_size);
+        cp->image.write_fixed(host.data() + y * blob_stride, blob_size);
         write_values(pr[members[c0 + y]].ops, stages, loc, host.data() + y * blob_stride);
       });
       blobs.reserve(std::max<size_t>(cnt * blob_stride, 1));

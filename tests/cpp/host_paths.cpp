@@ -1,5 +1,6 @@
 // host_paths.cpp — the host code between a caller's program and the kernels (lower.cpp,
 // planner.cpp, plan_image.cpp), built with sanitizers; no GPU is used. The argument names the check.
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <random>
@@ -83,13 +84,109 @@ void wide_customs() {
     }
 }
 
+// Random gates of every kind but Custom on n >= 3 wires, the same gates for the same seed, angles apart.
+Prog random_program(uint32_t n, int count, uint64_t seed, uint64_t angles) {
+  std::mt19937_64 rng(seed), ang(angles);
+  Prog p;
+  for (int g = 0; g < count; ++g) {
+    qr_op op{};
+    op.kind = (uint32_t)(rng() % QR_GATE_CUSTOM);
+    std::vector<uint32_t> w(n);
+    for (uint32_t i = 0; i < n; ++i) w[i] = i;
+    std::shuffle(w.begin(), w.end(), rng);
+    op.position = w[0];
+    op.arg = 0.1 + (double)(ang() % 1000) / 400.0;
+    op.arg_int = 1 + (int)(rng() % 5);
+    switch (op.kind) {
+      case QR_GATE_CR: case QR_GATE_CRK: case QR_GATE_CZ: case QR_GATE_CY: case QR_GATE_CNOT: case QR_GATE_SWAP:
+        op.ncontrols = 1; break;
+      case QR_GATE_TOFFOLI: op.ncontrols = 2; break;
+      default: break;
+    }
+    op.controls_offset = p.ctl.size();
+    for (uint32_t i = 0; i < op.ncontrols; ++i) p.ctl.push_back(w[1 + i]);
+    p.ops.push_back(op);
+  }
+  return p;
+}
+
+// A plan's blob: its values are those of the program at hand, its standalone offsets those of the
+// wires, nothing of it is left unwritten, and the plan keeps no table of its own.
+void plan_images() {
+  std::mt19937_64 rng(11);
+  for (int trial = 0; trial < 24; ++trial) {
+    const uint32_t n = 4 + (uint32_t)(trial % 9);
+    Prog a = random_program(n, 80, 100 + trial, 1), b = random_program(n, 80, 100 + trial, 2);
+    std::vector<std::vector<uint32_t>> wires = {{2, 0}, {1, 3, 0}, {3, 2, 1, 0}};
+    if (n >= 10) wires.push_back({9, 8, 7, 6, 5, 4, 3, 2, 1});
+    for (const auto& w : wires)
+      for (bool dense : {true, false}) {
+        std::mt19937_64 ra(rng()), rb(rng());
+        a.custom(w, dense, ra);
+        b.custom(w, dense, rb);
+      }
+    const qr_program va = a.view(), vb = b.view();
+    const bool dual = trial % 2 == 1;
+    std::vector<FastOp> opa = lower_program(n, &va, dual), opb = lower_program(n, &vb, dual);
+    if (dual) {
+      opa = adjoint_sweep_ops(opa);
+      opb = adjoint_sweep_ops(opb);
+    }
+    expect(key_of(opa) == key_of(opb), "programs that differ in values have one structure");
+    PlanParams pp;
+    pp.tile_bits = std::min<int>(trial % 3 ? 10 : 5, (int)n);
+    pp.reg_bits = std::min(4, pp.tile_bits);
+    pp.low_bits = 3;
+    const std::vector<Stage> stages = plan_fused(n, opa, pp, 16, dual);
+    const PlanImage im = plan_image(opa, stages);
+    std::vector<uint8_t> x(im.size() + 16, 0x11), y(im.size() + 16, 0x77);
+    for (std::vector<uint8_t>* blob : {&x, &y}) {
+      im.write_fixed(blob->data(), im.size());
+      write_values(opb, stages, im.loc, blob->data());
+    }
+    expect(std::equal(x.begin(), x.begin() + im.size(), y.begin()), "part of the blob is left unwritten");
+    expect(x[im.size()] == 0x11, "written behind the blob");
+    std::vector<uint8_t> live(im.live + 16, 0x33);
+    im.write_fixed(live.data(), im.live);
+    write_values(opb, stages, im.loc, live.data());
+    expect(std::equal(x.begin(), x.begin() + im.live, live.begin()) && live[im.live] == 0x33, "the live part");
+    size_t tables = 0, offsets = 0;
+    for (size_t si = 0; si < stages.size(); ++si) {
+      const Stage& s = stages[si];
+      const cd* c = (const cd*)(x.data() + im.loc[si].coefs);
+      if (s.tile) {
+        std::vector<cd> want;
+        stage_coefficients(s, opb, want);
+        expect(want.empty() || std::memcmp(c, want.data(), want.size() * sizeof(cd)) == 0, "a stage's coefficients");
+        expect(im.loc[si].ops >= im.live && im.loc[si].ops % 64 == 0, "a stage's ops");
+        const TileOpDev* d = (const TileOpDev*)(x.data() + im.loc[si].ops);
+        for (size_t i = 0; i < s.ops.size(); ++i) expect((d[i].w0 & 0xFF) == (uint32_t)s.ops[i].code, "an op's code");
+        continue;
+      }
+      const FastOp& op = opb[s.standalone];
+      if (op.kind != FK_DENSEK && op.kind != FK_DIAGK) continue;
+      tables += op.m.size() * sizeof(cd);
+      offsets += sizeof(uint64_t) << op.k;
+      expect(std::equal(op.m.begin(), op.m.end(), c), "a table");
+      const uint64_t* off = (const uint64_t*)(x.data() + im.loc[si].off);
+      for (uint64_t j = 0; j < 1ull << op.k; ++j) {
+        uint64_t want = 0;
+        for (int q = 0; q < op.k; ++q)
+          if ((j >> (op.k - 1 - q)) & 1) want |= 1ull << op.bits[q];
+        expect(off[j] == want, "an offset");
+      }
+    }
+    expect(im.values >= tables && im.live - im.values == offsets, "the plan keeps values");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   struct {
     const char* name;
     void (*run)();
-  } const checks[] = {{"wide_customs", wide_customs}};
+  } const checks[] = {{"wide_customs", wide_customs}, {"plan_images", plan_images}};
   for (const auto& c : checks)
     if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
       c.run();

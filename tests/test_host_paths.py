@@ -8,7 +8,7 @@ import pytest
 import helpers as H
 
 CSRC = os.path.join(H.ROOT, "quantr_amd", "csrc")
-SOURCES = ["lower.cpp", "planner.cpp"]
+SOURCES = ["lower.cpp", "planner.cpp", "plan_image.cpp"]
 
 
 @pytest.fixture(scope="module")
@@ -21,7 +21,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["wide_customs"])
+@pytest.mark.parametrize("check", ["wide_customs", "plan_images"])
 def test_host_paths(exe, check):
     r = subprocess.run([exe, check], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
