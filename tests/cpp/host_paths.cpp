@@ -180,13 +180,152 @@ void plan_images() {
   }
 }
 
+// ---- expectation records, read as k_pauli_expect_tiles reads them -----------------------------
+
+uint64_t deposit(uint64_t x, uint64_t mask) {
+  uint64_t out = 0;
+  for (int b = 0; mask; ++b) {
+    const uint64_t low = mask & (0ull - mask);
+    mask ^= low;
+    if ((x >> b) & 1u) out |= low;
+  }
+  return out;
+}
+double sign(uint64_t x) { return __builtin_popcountll(x) & 1 ? -1.0 : 1.0; }
+
+double replay(int prec, uint32_t n, const std::vector<cd>& psi, const uint8_t* group_records, const uint8_t* term_records,
+              const std::vector<PauliTilePass>& passes, const uint32_t* diag_count) {
+  const int K = pauli_tile_bits(prec);
+  const PauliTileGroup* groups = (const PauliTileGroup*)group_records;
+  const PauliTileTerm* terms = (const PauliTileTerm*)term_records;
+  double total = 0.0;
+  for (const PauliTilePass& ps : passes) {
+    if (ps.tmask == 0) {
+      for (uint32_t i = 0; i < ps.cnt[0]; ++i) {
+        const PauliGroup& g = ((const PauliGroup*)group_records)[ps.first + i];
+        for (uint32_t t = 0; t < g.count; ++t) {
+          const PauliZTerm& z = ((const PauliZTerm*)term_records)[g.first + t];
+          for (uint64_t o = 0; o < psi.size(); ++o)
+            total += (std::conj(psi[o]) * cd(z.cr, z.ci) * sign((o ^ g.xm) & z.zm) * psi[o ^ g.xm]).real();
+        }
+      }
+      continue;
+    }
+    expect(__builtin_popcountll(ps.tmask) == K, "a pass's tile");
+    const uint64_t nontile = (psi.size() - 1) & ~ps.tmask;
+    std::vector<uint64_t> at(1u << K);
+    for (uint64_t p = 0; p < at.size(); ++p) at[p] = deposit(p, ps.tmask);
+    for (uint64_t tile = 0; tile < psi.size() >> K; ++tile) {
+      const uint64_t base = deposit(tile, nontile);
+      for (uint32_t lane = 0; lane < 1u << (K - 4); ++lane) {
+        const PauliTileGroup* gp = groups + ps.first;
+        const PauliTileTerm* tp = terms + ps.term0;
+        for (int arr = 0; arr < kPauliArrangements; ++arr) {
+          if (!((ps.arrs >> arr) & 1u)) continue;
+          const int nb = pauli_arrangement_bit(K, arr);
+          const uint32_t pt = (lane & ((1u << nb) - 1u)) | ((lane >> nb) << (nb + 4));
+          auto amp = [&](uint32_t r, uint32_t lx = 0) { return psi[base | at[(pt | (r << nb)) ^ lx]]; };
+          auto coef = [&](const PauliTileTerm& t) { return t.c * sign(pt & t.lz) * sign(base & t.zout); };
+          if (arr == 0 && ps.diag)
+            for (uint32_t p = 0; p < 16; ++p)
+              for (uint32_t c = diag_count[p]; c; --c, ++tp) {
+                expect(tp->pat == p, "the order of Z strings");
+                for (uint32_t r = 0; r < 16; ++r) total += coef(*tp) * sign(r & p) * std::norm(amp(r));
+              }
+          for (uint32_t m = 1; m < 16; ++m)
+            if ((ps.plain[arr] >> m) & 1u) {
+              const uint32_t top = 31 - __builtin_clz(m);
+              for (uint32_t r = 0; r < 16; ++r)
+                if (!((r >> top) & 1u)) total += coef(*tp) * (std::conj(amp(r)) * amp(r ^ m)).real();
+              ++tp;
+            }
+          for (uint32_t g = 0; g < ps.cnt[arr]; ++g, ++gp) {
+            const uint32_t top = gp->op >= PAULI_LDS ? gp->op - PAULI_LDS : 31 - (uint32_t)__builtin_clz(gp->op);
+            expect(gp->op >= PAULI_LDS ? ((gp->lx >> nb) & 15u) >> top == 1u : gp->lx == gp->op << nb, "a group's pairs");
+            for (uint32_t q = 0; q < gp->nre + gp->nim; ++q, ++tp)
+              for (uint32_t r = 0; r < 16; ++r) {
+                if ((r >> top) & 1u) continue;
+                const uint32_t i = (r & ((1u << top) - 1u)) | ((r >> (top + 1)) << top);
+                const cd v = std::conj(amp(r)) * amp(r, gp->lx);
+                total += coef(*tp) * sign(i & tp->pat) * (q < gp->nre ? v.real() : v.imag());
+              }
+          }
+        }
+      }
+    }
+  }
+  return total;
+}
+
+// The records of observables that use every arrangement, masks that cross them, both parities of Y,
+// more passes than one launch takes and masks too wide for a tile, against the plain sum. Both are
+// sums of products of modulus at most 1 in binary64.
+void expectation_records() {
+  struct Shape {
+    int prec;
+    uint32_t n;
+    int kind;
+  };
+  for (const Shape sh : {Shape{0, 15, 0}, Shape{0, 15, 1}, Shape{0, 16, 2}, Shape{0, 10, 0}, Shape{1, 16, 0},
+                         Shape{1, 16, 1}, Shape{1, 17, 2}}) {
+    std::mt19937_64 rng(500 + sh.n + (uint64_t)sh.kind);
+    std::normal_distribution<double> g;
+    const uint32_t n = sh.n;
+    std::vector<cd> psi(1ull << n);
+    for (cd& a : psi) a = cd(g(rng), g(rng)) * std::ldexp(1.0, -(int)n / 2);
+    std::vector<PauliMasks> obs;
+    auto term = [&](uint64_t xm, uint64_t zm) { obs.push_back(PauliMasks{g(rng), xm, zm, __builtin_popcountll(xm & zm)}); };
+    const uint64_t all = (1ull << n) - 1;
+    const int tile = pauli_tile_bits(sh.prec), low = pauli_low_bits(sh.prec);
+    if (sh.kind < 2)
+      for (uint32_t b = 0; b < n; ++b) {
+        term(1ull << b, 0);
+        term(0, (1ull << b) | (1ull << ((b + 5) % n)));
+        if (sh.kind == 1) continue;
+        term(1ull << b, 1ull << b);
+        term(3ull << (b % (n - 1)), rng() & all);
+        term(15ull << (b % (n - 3)), rng() & all);
+        term((1ull << b) | (1ull << (rng() % n)), rng() & all);
+      }
+    if (sh.kind == 2)
+      for (int t = 0; t < 60; ++t) {  // as many high bits as a tile holds beside the low ones, and all
+        uint64_t xm = rng() & ((1ull << low) - 1);
+        while (__builtin_popcountll(xm >> low) < tile - low) xm |= 1ull << (low + (int)(rng() % (n - (uint32_t)low)));
+        term(t % 20 == 19 ? all : xm, rng() & all);
+      }
+    std::vector<PauliGroup> groups;
+    std::vector<PauliZTerm> flat;
+    pauli_tables(obs, groups, flat);
+    const int G = (int)groups.size();
+    std::vector<PauliPass> passes(G + 1);
+    std::vector<uint32_t> lxm(G);
+    const int np = pauli_passes(n, sh.prec, groups.data(), G, passes.data(), lxm.data());
+    if (sh.kind == 2) expect(np > (int)kPauliPassesPerLaunch, "more passes than one launch takes");
+    std::vector<PauliTilePass> tp(np);
+    uint32_t diag_count[16];
+    std::vector<uint8_t> gr((G + 1) * sizeof(PauliGroup)), tr((flat.size() + 1) * sizeof(PauliZTerm));
+    pauli_tile_tables(sh.prec, groups.data(), lxm.data(), passes.data(), np, flat.data(), gr.data(), tr.data(), tp.data(),
+                      diag_count);
+    const double got = replay(sh.prec, n, psi, gr.data(), tr.data(), tp, diag_count);
+    double want = 0.0, weight = 0.0;
+    for (const PauliMasks& t : obs) {
+      cd f = t.coeff;
+      for (int q = 0; q < t.ny; ++q) f *= cd(0, 1);
+      weight += std::fabs(t.coeff);
+      for (uint64_t j = 0; j < psi.size(); ++j) want += (std::conj(psi[j ^ t.xm]) * f * sign(j & t.zm) * psi[j]).real();
+    }
+    expect(std::fabs(got - want) < 64 * n * 2.3e-16 * weight * 2.0, "the value of an observable");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   struct {
     const char* name;
     void (*run)();
-  } const checks[] = {{"wide_customs", wide_customs}, {"plan_images", plan_images}};
+  } const checks[] = {{"wide_customs", wide_customs}, {"plan_images", plan_images},
+                {"expectation_records", expectation_records}};
   for (const auto& c : checks)
     if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
       c.run();

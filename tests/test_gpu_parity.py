@@ -891,3 +891,36 @@ def test_wide_custom_gates_fused(k, diagonal):
             st.apply(p)
             assert np.max(np.abs(st.amplitudes() - want)) < TOL_FUSED
     st.close()
+
+
+@pytest.mark.parametrize("n,precision", [(15, _capi.QR_C128), (16, _capi.QR_C64)])
+def test_expectation_plain_groups_smallest_tiled(n, precision):
+    """The same at the smallest states whose expectations are tiled (three qubits more than a tile;
+    narrower ones are read directly)."""
+    test_expectation_plain_groups(n, precision)
+
+
+@pytest.mark.parametrize("n,precision", [(16, _capi.QR_C128), (17, _capi.QR_C64), (20, _capi.QR_C128)])
+def test_expectation_many_passes(n, precision):
+    """Observables of more tiled passes than one launch takes (16), so that launches add to each
+    other's partial sums, with X mask 0 in one of them and with masks too wide for any tile read
+    directly behind them. Tolerance as for every arrangement above."""
+    rng = np.random.default_rng(4500 + n)
+    tile, low = (12, 3) if precision == _capi.QR_C128 else (13, 4)
+    st = _capi.State(n, precision)
+    st.apply(W.to_program(W.brickwork(n, depth=7, seed=n + 3)))
+    psi = st.amplitudes()
+
+    def string(bits, paulis):
+        return (float(rng.uniform(-1, 1)), [(n - 1 - int(b), paulis[int(rng.integers(len(paulis)))]) for b in bits])
+
+    high = [low + rng.permutation(n - low)[:tile - low] for _ in range(40)]
+    plain = [string(b, "X") for b in high]
+    general = [string(list(b) + [0], "XY") for b in high] + [string(rng.permutation(n)[:3], "Z") for _ in range(20)]
+    wide = [string(range(n), "XY") for _ in range(3)]
+    for terms in (plain, general, plain + general + wide):
+        obs = _capi.Observable(terms)
+        want = H.oracle_expectation(n, psi, obs)
+        for got in (st.expectation(obs), st.expectation(obs)):
+            assert abs(got - want) < 16 * n * 2.0 ** -52 * sum(abs(c) for c, _ in terms)
+    st.close()

@@ -21,7 +21,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["wide_customs", "plan_images"])
+@pytest.mark.parametrize("check", ["wide_customs", "plan_images", "expectation_records"])
 def test_host_paths(exe, check):
     r = subprocess.run([exe, check], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
