@@ -50,7 +50,7 @@ struct JitKernel {
   hipFunction_t fn = nullptr;
 };
 
-constexpr size_t kTapRows = 14;  // qr::dev::kTapRows of tile_ops.hpp
+constexpr size_t kTapRows = 14, kTapStride = 72;  // those of tile_ops.hpp, which stage sources check
 
 std::mutex g_mu;
 std::map<std::string, JitKernel> g_cache;
@@ -158,12 +158,14 @@ std::string stage_source(const Stage& s, int prec, int RB, bool persistent, bool
   bool rows = false;
   if (dual && TPB >= 64) {
     const size_t exchange = (size_t)(lds2 ? 2 : 1) * (1ull << K) * amp_bytes, cu = 160 * 1024;
-    const size_t with_rows = exchange + (size_t)(TPB / 64) * kTapRows * 72 * sizeof(double);
+    const size_t with_rows = exchange + (size_t)(TPB / 64) * kTapRows * kTapStride * sizeof(double);
     if (cu / with_rows >= std::min<size_t>(2, cu / exchange))
       for (const TileOpHost& op : s.ops) rows = rows || op.code == TC_GRAD;
   }
   if (rows)
-    o << "  __shared__ __align__(16) double taprows[" << TPB / 64 << " * qr::dev::kTapRows * qr::dev::kTapStride];\n"
+    o << "  static_assert(qr::dev::kTapRows == " << kTapRows << " && qr::dev::kTapStride == " << kTapStride
+      << ", \"LDS rows\");\n"
+      << "  __shared__ __align__(16) double taprows[" << TPB / 64 << " * qr::dev::kTapRows * qr::dev::kTapStride];\n"
       << "  double* const myrows = taprows + (threadIdx.x >> 6) * (qr::dev::kTapRows * qr::dev::kTapStride);\n";
   auto flush_taps = [&]() {
     if (taps.empty()) return;

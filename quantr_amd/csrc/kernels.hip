@@ -389,10 +389,11 @@ __device__ __forceinline__ double units_of(double p, double scale, bool& tie) {
 // the exact sum of rint(p_i * 2^(52-e)) (sums[3b + c]; exact while below 2^53, and at least
 // 2^53 exactly when the true sum is) and flags[b] bit c when some p_i * 2^(52-e) is a halfway
 // case or e is outside [-960, 52] (then the scaling could overflow or the binade is unusable).
-// A state whose probabilities have full mantissas holds about one halfway case per binade: blocks
-// with one in the middle candidate (the binade the block most likely starts in) leave their
-// probabilities for the host's fold in the next of tie.most places, so that it need not ask for
-// them one by one (17 qubits, 1000 draws on a state of full mantissas: 228 -> 150 us).
+// A complex128 state of full mantissas holds about one halfway case per binade, a complex64 state,
+// whose probabilities have 48 bits, about 32: blocks with one in the middle candidate (the binade the
+// block most likely starts in) leave their probabilities for the host's fold in the next of tie.most
+// places, so that it need not ask for them one by one (complex128, 17 qubits, 1000 draws on a state of
+// full mantissas: 228 -> 150 us).
 template <typename R>
 __global__ __launch_bounds__(256) void k_block_exact_sums(const typename CT<R>::T* __restrict__ psi, uint64_t dim,
                                                           int bb, const int32_t* __restrict__ ebase,
@@ -1071,7 +1072,7 @@ __device__ __forceinline__ void plain_arrangements(T (&a)[16], R* lds, uint32_t 
 // of 2^(K-4) threads walk the tiles; a thread holds 16 amplitudes, which differ in 4 tile bits.
 // What bounds it: HBM when a pass holds few groups, else vector issue, then LDS (a 16-byte read
 // per amplitude costs a quarter of the CU's 128 B/clk for 8 clocks). So:
-//  * the tile is held in up to three arrangements, each with another 4 of the tile bits in
+//  * the tile is held in up to three arrangements (four for 2^13 tiles), each with another 4 of its bits in
 //    registers: a group whose X mask lies in one of them pairs registers, with no LDS access;
 //    only masks that cross them read partners from LDS;
 //  * a hermitian term gives the same for (o, o ^ xm) and (o ^ xm, o): one product for each pair;
@@ -1089,7 +1090,7 @@ __device__ __forceinline__ void plain_arrangements(T (&a)[16], R* lds, uint32_t 
 // 5.0. Complex64, 28 qubits, 6.5 -> 1.6 ms (2.1 with vector loads); 120 strings of up to 4 factors on 22 qubits
 // 520 -> 335 us (355). Fetching the next tile ahead took longer (5.9 ms: its registers spill).
 // Element p of the tile sits at LDS slot p ^ (bits above the lowest arrangement's nibble, at its
-// place): consecutive lanes hit distinct slots in all three arrangements.
+// place): consecutive lanes hit distinct slots in every arrangement.
 template <typename R, int K, bool NT, bool GENERAL>
 __global__ __launch_bounds__(1 << (K - 4), K == 12 && GENERAL ? 2 : 4) void k_pauli_expect_tiles(
     const typename CT<R>::T* __restrict__ psi, uint64_t dim, PauliTilePasses P,

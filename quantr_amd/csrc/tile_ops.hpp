@@ -344,8 +344,10 @@ __device__ __forceinline__ void tap_store(double acc, double* row, unsigned long
 // 16 values from LDS in a fixed order, then across the four. One by one, a tap's six exchanges
 // between lanes take longer than its products where a wavefront has its SIMD to itself (20 qubits,
 // complex128, 400 parameters: 32 -> 21 us per sweep together with the folded rotations).
-// A row is 4 x 18 doubles: the lanes of an access then hit distinct banks. 14 rows: with the 32 KB
-// of both states' exchange, four workgroups still share a CU's LDS.
+// A row is 4 x 18 doubles: the lanes of an access then hit distinct banks. 14 rows beside the 32 KB of
+// both states' exchange let three workgroups of two wavefronts (8 amplitudes of each state per thread)
+// or four of one (16) share a CU's LDS. With 7 rows four of two fit: the same within 2% up to 21 qubits
+// in complex128 and 20 in complex64; forward and backward of 22 qubits 2.05 -> 2.02 and 1.49 -> 1.39 ms.
 constexpr int kTapRows = 14, kTapStride = 72;
 __device__ __forceinline__ void tap_put(double* rows, int row, unsigned int lane, double acc) {
   rows[row * kTapStride + lane + 2 * (lane >> 4)] = acc;
