@@ -293,8 +293,11 @@ qr_status qr_grad_forward(qr_grad* g, const qr_program* program, const qr_observ
     qr_state* st = g->psi.get();
     validate_program(st->n, program);
     check_unitary_customs(st->n, program);  // the reverse sweep needs U^dagger = U^-1
-    g->ops = lower_program(st->n, program, true);
+    auto ops = lower_program(st->n, program, true);
     g->terms = parse_observable(st->n, observable);
+    // a program or observable refused above leaves the last forward in force; from here on it is gone
+    g->have_forward = false;
+    g->ops = std::move(ops);
     g->nparams = 0;
     for (const auto& op : g->ops)
       if (op.param >= 0) g->nparams++;

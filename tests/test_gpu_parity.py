@@ -924,3 +924,22 @@ def test_expectation_many_passes(n, precision):
         for got in (st.expectation(obs), st.expectation(obs)):
             assert abs(got - want) < 16 * n * 2.0 ** -52 * sum(abs(c) for c, _ in terms)
     st.close()
+
+
+def test_backward_after_a_refused_forward():
+    """A forward whose observable is refused leaves the one before in force, its gradient included,
+    even where the refused program has as many parameters."""
+    n = 6
+    first, second = (W.to_program(W.hea(n, 2, seed=s)[0]) for s in (1, 2))
+    obs = _capi.Observable(W.hea_observable(n))
+    bad = _capi.Observable([(1.0, [(n, "Z")])])
+    g = _capi.Grad(n)
+    g.forward(first, obs)
+    want = g.backward()
+    g.forward(first, obs)
+    with pytest.raises(_capi.QrError):
+        g.forward(second, bad)
+    assert np.array_equal(g.backward(), want)
+    with pytest.raises(_capi.QrError):  # a gradient is taken once per forward
+        g.backward()
+    g.close()
