@@ -211,8 +211,9 @@ void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vec
   };
   // the blocks with a halfway case that found no place, in one more launch (as many as 16 MB hold)
   std::vector<uint64_t> rest;
-  for (uint64_t b = 0; b < nblk && rest.size() < (2ull << 20) / len; ++b)
-    if ((flags[b] & 2u) && mass[b] != 0.0 && !fetched(b)) rest.push_back(b);
+  if (tie_block[most_ties - 1] != ~0ull)
+    for (uint64_t b = 0; b < nblk && rest.size() < (2ull << 20) / len; ++b)
+      if ((flags[b] & 2u) && mass[b] != 0.0 && !fetched(b)) rest.push_back(b);
   PinnedLease pin_rest;
   if (!rest.empty()) {
     pin_rest.reserve(rest.size() * (len + 1) * 8);
@@ -278,12 +279,15 @@ void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vec
   // whose end exceeds u); draws at or above the total are None. A job takes at most kJobDraws.
   constexpr uint64_t kJobDraws = 2048;
   std::vector<ExactJob> jobs;
+  jobs.reserve(std::min(shots, nblk) + shots / kJobDraws);
+  const double* const u = us.data();
   uint64_t d = 0;
   while (d < shots) {
-    const uint64_t b = (uint64_t)(std::upper_bound(ends.begin(), ends.end(), us[d]) - ends.begin());
+    const uint64_t b = (uint64_t)(std::upper_bound(ends.begin(), ends.end(), u[d]) - ends.begin());
     if (b >= nblk) break;
+    const double end = ends[b];
     uint64_t last = d;
-    while (last < shots && us[last] < ends[b]) ++last;
+    while (last < shots && u[last] < end) ++last;
     const BlockFold& f = bf[b];
     if (f.exact) {
       const double un = std::ldexp(1.0, f.e - 52);
@@ -291,7 +295,7 @@ void sample_exact_parallel(qr_state* st, const std::vector<double>& us, std::vec
         jobs.push_back(ExactJob{b, f.start / un, un, std::ldexp(1.0, 52 - f.e), j, std::min(last, j + kJobDraws)});
     } else {
       uint64_t at = d;
-      fold(probs_of(b), len, f.start, us.data(), at, last, res.data(), b << bb, true);
+      fold(probs_of(b), len, f.start, u, at, last, res.data(), b << bb, true);
     }
     d = last;
   }
