@@ -226,7 +226,8 @@ qr_status qr_sample(qr_state* state, const double* uniforms, uint64_t shots, uin
  * re-simulates the circuit for every shot because custom functions may answer differently
  * (examples/post_select.rs:39-49), done for all shots at once: programs of one structure share
  * a plan and their sweeps run as one launch over all of their states. Fused mode; states use
- * the current device and are freed before returning. */
+ * the current device. Their memory is freed before returning, or kept for later calls: at most
+ * 256 MB while a qr_state, qr_grad or qr_batch lives, 4 MB while none does. */
 qr_status qr_sample_programs(uint32_t num_qubits, qr_precision precision, const qr_program* programs,
                              uint64_t count, const uint64_t* draws_per_program, const double* uniforms,
                              uint64_t* idx_out);

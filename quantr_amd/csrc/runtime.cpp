@@ -24,15 +24,17 @@
 namespace qr {
 
 // Default tile shape: 2^12 complex128 / 2^13 complex64 amplitudes (64 KB of LDS, two
-// workgroups per CU), 16 amplitudes per thread. Complex128 states of up to 19 qubits leave most CUs
+// workgroups per CU), 16 amplitudes per thread. Complex128 states of 13 to 19 qubits leave most CUs
 // without such a tile: 2^11 amplitudes give twice the workgroups, which pays for a sweep more or
-// less (brickwork of 20 layers, 12 / 13 / 16 / 19 qubits: 95 / 98 / 121 / 165 us with 2^12,
-// 83 / 87 / 106 / 148 with 2^11; an ansatz of 20 qubits 268 -> 301). Complex64 states keep 2^13: more
+// less (brickwork of 20 layers, 13 / 14 / 16 / 19 qubits: 107 / 112 / 132 / 169 us with 2^12,
+// 95 / 106 / 120 / 160 with 2^11; an ansatz of 20 qubits 268 -> 301). A state that one tile holds keeps
+// it: alone it takes 103 us (95 with 2^11), but 500 of them re-simulated together 2.2 ms (3.0 with
+// 2^11), and both must run the same stages to return the same bins. Complex64 states keep 2^13: more
 // sweeps mean more factored scalars applied, and the energies of an 18-qubit ansatz were 1.4
 // times further from 64 bits with 2^11.
 int pick_tile_bits(const qr_state* st) {
   int k = st->prec == 0 ? 12 : 13;
-  if (st->prec == 0 && st->n <= 19) k = 11;
+  if (st->prec == 0 && st->n > 12 && st->n <= 19) k = 11;
   if (st->opt.tile_bits) k = std::min<int>(tile_max_bits(st->prec), (int)st->opt.tile_bits);
   return std::min<int>(k, (int)st->n);
 }

@@ -76,9 +76,9 @@ void sample_programs(uint32_t n, int prec, const qr_program* programs, uint64_t 
   }
   int count_dev = 0;
   if (hipGetDeviceCount(&count_dev) != hipSuccess || count_dev == 0) throw Error{QR_ERR_NO_DEVICE, "no GPU visible"};
-  // planning parameters of a state of this size and precision with default options, but the wide
-  // tile also for small states: the programs' states fill the chip together
-  const qr_options defaults{1, prec == 0 ? 12u : 13u, 0, 2, 0, 0, 2, 0, 0};
+  // planning parameters of a state of this size and precision with default options: the programs run
+  // the stages such a state runs, so that their bins are those of qr_sample on it, to the last bit
+  const qr_options defaults{1, 0, 0, 2, 0, 0, 2, 0, 0};
   const PlanParams pp = plan_params(n, prec, defaults);
   const uint64_t dim = 1ull << n;
   const size_t B = prec == 0 ? 16 : 8;

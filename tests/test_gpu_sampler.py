@@ -168,3 +168,25 @@ def test_many_halfway_blocks(precision, n, bits):
     want = np.searchsorted(S, u, side="right").astype(np.uint64)
     want[u >= S[-1]] = NONE
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("precision,n", [(_capi.QR_C128, 11), (_capi.QR_C128, 12), (_capi.QR_C128, 13),
+                                         (_capi.QR_C128, 17), (_capi.QR_C128, 20), (_capi.QR_C64, 13),
+                                         (_capi.QR_C64, 16)])
+def test_programs_on_fold_values(precision, n):
+    """Re-simulated programs return what qr_sample returns on the program's own state, also for draws
+    on and next to that state's fold values, which a difference in the last bit of an amplitude
+    would send to another bin: both run the same stages."""
+    rng = np.random.default_rng(890 + n)
+    table = (np.ascontiguousarray(W.random_unitary(2, n).T), np.ones(4, dtype=np.uint8))
+    gates = W.brickwork(n, depth=8, seed=n)
+    cut = len(gates) // 2
+    program = H.to_program(gates[:cut] + [("Custom", 3, (1,), 0.0, 0)] + gates[cut:], {cut: table})
+    st = _capi.State(n, precision)
+    st.set_options(fused=1, jit=1)
+    st.apply(program)
+    u = boundary_draws(left_fold(st.amplitudes()), rng, 500)
+    want = st.sample(u)
+    st.close()
+    got = _capi.sample_programs(n, [program, program], [len(u), len(u)], np.concatenate([u, u]), precision)
+    assert np.array_equal(got, np.concatenate([want, want]))
